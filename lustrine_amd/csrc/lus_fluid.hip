@@ -11,13 +11,12 @@
 //   * the pressure sweep (:90-113) is sequential in the reference: particle i
 //     reads x* of the particles before it as already corrected (in place) and
 //     of those after it as predicted, and uses lambdas[t] for the t-th entry
-//     of its list.  Here it runs as a dependency-level schedule: particle i
-//     waits for every neighbour j < i; the moving particles whose waits are
-//     all met form one level and run in one launch, and a launch boundary
-//     separates the levels.  Two particles of one level are never neighbours
-//     (the later one would wait for the earlier), so a particle reads every
-//     earlier neighbour already corrected and every later one not yet
-//     touched: exactly the reference's sequential sweep, in parallel.
+//     of its list.  Here it runs as a data flow: the corrected positions go to
+//     an array of their own, cleared to a "not yet" pattern before the sweep,
+//     and particle i waits for the entries of its neighbours j < i there and
+//     reads the predicted positions of those after it.  So a particle reads
+//     every earlier neighbour corrected and every later one predicted: exactly
+//     the reference's sequential sweep, in parallel (k_fl_sweep).
 //
 // Arithmetic follows the reference's operation order with no contraction and
 // IEEE divide and square root (the library's build flags).  One call differs
@@ -67,18 +66,18 @@ struct FluidState {
     int *cnt = nullptr, *off = nullptr, *ltiles = nullptr, *idx = nullptr;
     long cap = 0;
     void* idx_mem = nullptr;
-    int *indeg = nullptr, *q0 = nullptr, *q1 = nullptr, *ctl = nullptr;  // ctl: see kCtl*
+    float4* xs2 = nullptr;    // the sweep's output; swapped with xs after it
+    int* ctl = nullptr;       // see kCtl*
     int* host_ctl = nullptr;  // pinned mirror of ctl
 };
 
-// ctl layout: three frontier counters, processed count, deepest level, error bits
-constexpr int kCtlQ = 0;         // ctl[0..2]: frontier counters of levels L % 3
-constexpr int kCtlDone = 3;
-constexpr int kCtlLevels = 4;
-constexpr int kCtlErr = 5;
-constexpr int kCtlInts = 8;
+constexpr int kCtlTicket = 0;    // next block of the sweep
+constexpr int kCtlLevels = 1;    // longest chain of waits of the sweep
+constexpr int kCtlErr = 2;       // error bits
+constexpr int kCtlInts = 4;
 constexpr int kErrKey = 1;       // a predicted position lies outside the grid
 constexpr int kErrLambda = 2;    // a list is longer than the lambdas array
+constexpr int kErrStall = 4;     // the sweep gave up waiting
 
 void fluid_free(FluidState* F) {
     if (!F) return;
@@ -158,9 +157,11 @@ __device__ __forceinline__ float fl_resolve(float value, float lo, float hi) {
 }
 
 // integration (:48-51) and the cell key of each moving particle
+// and its "not yet" mark in the sweep's output
 __global__ __launch_bounds__(kBlock) void k_fl_predict(float4* __restrict__ x, float4* __restrict__ v,
-                                                        float4* __restrict__ xs, FluidK k, float dt,
-                                                        int* __restrict__ key, int C, int* __restrict__ ctl) {
+                                                        float4* __restrict__ xs, float4* __restrict__ xs2, FluidK k,
+                                                        float dt, int* __restrict__ key, int C,
+                                                        int* __restrict__ ctl) {
     const int t = xcd_index();
     if (t >= k.n) return;
     const int i = k.s0 + t;
@@ -176,6 +177,8 @@ __global__ __launch_bounds__(kBlock) void k_fl_predict(float4* __restrict__ x, f
     q.w = 0.0f;
     v[i] = vi;
     xs[i] = q;
+    const float open = __uint_as_float(~0u);
+    xs2[i] = make_float4(open, open, open, open);
     // get_cell_id (Utils.hpp:24-33) has no clamp: a cell index outside
     // [0, C) indexes outside the reference's cell vector; here it is reported
     // (an index inside [0, C) is used as the reference uses it, even when a
@@ -261,26 +264,22 @@ __global__ __launch_bounds__(kBlock) void k_fl_lists(const float4* __restrict__ 
     if (!fill) cnt[t] = count;
 }
 
-// lambda of each moving particle (:58-88); the number of its neighbours that
-// come before it in the sweep; the particles that wait for none start level 0
+// lambda of each moving particle (:58-88)
 __global__ __launch_bounds__(kBlock) void k_fl_lambda(const float4* __restrict__ xs, const int* __restrict__ off,
                                                        const int* __restrict__ idx, FluidK k,
-                                                       float* __restrict__ lam, int* __restrict__ indeg,
-                                                       int* __restrict__ q0, int* __restrict__ ctl) {
+                                                       float* __restrict__ lam, int* __restrict__ ctl) {
     const int t = xcd_index();
     if (t >= k.n) return;
     const int i = k.s0 + t;
     const int a = off[t], b = off[t + 1];
     const float4 pi = xs[i];
     float density = 0.0f;
-    int before = 0;
     for (int e = a; e < b; ++e) {
         const int j = idx[e];
         const float4 pj = xs[j];
         const float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const float len = sqrtf(dot3(dx, dy, dz, dx, dy, dz));
         density = density + k.mass * fl_cubic(k, len);
-        before += (j >= k.s0 && j < i) ? 1 : 0;
     }
     density = density + k.mass * k.W0;
     const float constraint = (float)((double)(density / k.rho0) - 1.0);
@@ -302,96 +301,303 @@ __global__ __launch_bounds__(kBlock) void k_fl_lambda(const float4* __restrict__
     if ((double)gsum > 0.0) l = -constraint / (gsum + k.eps);
     lam[i] = l;
     if (b - a > k.nl) atomicOr(&ctl[kCtlErr], kErrLambda);
-    indeg[t] = before;
-    if (before == 0) q0[atomicAdd(&ctl[kCtlQ + 0], 1)] = t;
 }
 
-// One dependency level of the pressure sweep (:90-113).  in / in_cnt: the
-// level's particles; out / out_cnt: the next level's, appended here as their
-// last wait is met; the counter two levels ahead is cleared for reuse.
-__global__ __launch_bounds__(kBlock) void k_fl_sweep(float4* __restrict__ x, float4* __restrict__ xs,
+// The pressure sweep (:90-113) as a data flow.  A term whose neighbour is a solid or comes later in the
+// sweep (predicted position) is computed at once; an earlier neighbour's is
+// computed when its corrected position shows up in xs2.  The terms meet in LDS
+// and are added in list order, one lane per component, so the sums are the
+// sequential sweep's bit for bit.
+//
+// A corrected position is its own signal: x, y, z and the chain length are
+// agent-scope 4-byte stores over the all-ones words k_fl_predict left, and a
+// reader takes the position when none of them is all ones (no flag, no fence,
+// which would write back and invalidate an XCD's whole L2).
+//
+// Blocks take their particles in slot order by ticket, so every particle waited for
+// belongs to the same wave (whose loop serves all its particles) or to a wave
+// that already runs: every wait ends.  (kSweepSpins passes without progress
+// end it with an error all the same.)
+//
+// What bounds it is the longest chain of waits, 2.7 to 3.2 us a link at 32 K
+// particles (a bare store and load between two XCDs takes 0.6; the rest is the
+// last term, its sum and the divides).  One launch per level took 36 us a
+// link: 32 K particles, 218 to 870 links, step 8 to 29 ms -> 0.85 to 2.8 ms;
+// 1 M, 762 links, step 67 -> 18 ms.  A particle that waits for many neighbours
+// asks for the latest of them only, one that waits for at most kSweepFew asks
+// for each, with a pause between (1, 4, 10, 30 x 64 cycles at the 870 links:
+// 3.4, 2.9, 2.8, 2.8 ms), so that the waves far from the front leave the ones
+// at it alone.
+//
+// kLanes lanes hold one particle and take its list kLanes * kPer entries at a
+// time, entry e in lane e % kLanes.  Few particles per wave shorten a link
+// (they take turns), many widen the window of particles in flight, which bounds
+// large scenes (launch_sweep).
+// kPow4: s_corr_n = 4 (the Simulation default), else any exponent.
+constexpr unsigned int kOpen = ~0u;                      // "not yet"
+constexpr int kSweepSpins = 1 << 22;
+constexpr int kSweepPause = 10;                          // x 64 cycles between two askings
+constexpr int kSweepFew = 4;
+
+// max over the kLanes lanes of a particle, in every one of them
+template <int kCtrl>
+__device__ __forceinline__ int dpp_max(int v) {
+    const int o = __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xF, 0xF, false);
+    return o > v ? o : v;
+}
+template <int kLanes>
+__device__ __forceinline__ int sweep_max(int v) {
+    v = dpp_max<0xB1>(v);                        // lane ^ 1
+    v = dpp_max<0x4E>(v);                        // lane ^ 2
+    v = dpp_max<0x141>(v);                       // half row mirrored
+    v = dpp_max<0x140>(v);                       // row mirrored
+#pragma unroll
+    for (int d = 16; d < kLanes; d <<= 1) {
+        const int o = __shfl_xor(v, d, 64);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
+struct SweepPos {
+    unsigned long long xy, zc;  // (x, y), (z, chain length)
+    __device__ __forceinline__ bool here() const {
+        return (unsigned int)xy != kOpen && (unsigned int)(xy >> 32) != kOpen && (unsigned int)zc != kOpen &&
+               (unsigned int)(zc >> 32) != kOpen;
+    }
+};
+__device__ __forceinline__ SweepPos sweep_load(const unsigned long long* out, int j) {
+    SweepPos q;
+    q.xy = __hip_atomic_load(out + 2 * (size_t)j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    q.zc = __hip_atomic_load(out + 2 * (size_t)j + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return q;
+}
+__device__ __forceinline__ unsigned long long pack2(float a, float b) {
+    return (unsigned long long)__float_as_uint(b) << 32 | __float_as_uint(a);
+}
+
+// one term of the sweep's sum: (lambda_i + lambdas[t] + s_corr) grad W
+template <bool kPow4, int kRow>
+__device__ __forceinline__ void fl_term(const FluidK& k, const float4 pi, float px, float py, float pz, float ll,
+                                        float* __restrict__ out) {
+    const float dx = pi.x - px, dy = pi.y - py, dz = pi.z - pz;
+    const float len = sqrtf(dot3(dx, dy, dz, dx, dy, dz));
+    const float ratio = fl_cubic(k, len) / k.Wdq;
+    float pw;
+    if constexpr (kPow4) {
+        const double b = (double)ratio, b2 = b * b;
+        pw = (float)(b2 * b2);
+    } else {
+        pw = fl_pow(k, ratio);
+    }
+    const float coef = ll + -k.scorr_k * pw;
+    float gx, gy, gz;
+    fl_cubic_grad(k, dx, dy, dz, &gx, &gy, &gz);
+    out[0] = coef * gx;
+    out[kRow] = coef * gy;
+    out[2 * kRow] = coef * gz;
+}
+
+template <bool kPow4, int kLanes, int kPer>
+__global__ __launch_bounds__(kBlock) void k_fl_sweep(float4* __restrict__ x, const float4* __restrict__ xs, float4* xs2,
                                                       float4* __restrict__ v, const float* __restrict__ lam,
                                                       const int* __restrict__ off, const int* __restrict__ idx,
-                                                      FluidK k, float dt, int level, const int* __restrict__ in,
-                                                      int* __restrict__ out, int* __restrict__ indeg,
-                                                      int* __restrict__ ctl) {
-    const int qi = level % 3;
-    const int cnt = ctl[kCtlQ + qi];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl[kCtlQ + (level + 2) % 3] = 0;
-        if (cnt > 0) atomicMax(&ctl[kCtlLevels], level + 1);
-    }
-    int* out_cnt = &ctl[kCtlQ + (level + 1) % 3];
-    int processed = 0;
-    // A level holds about n / depth particles, one per thread: the time of a
-    // level is the latency of one particle's walk, so each walk requests its
-    // list entries, their positions and lambdas[t] eight at a time before
-    // using them (the terms are still added in list order).  The later
-    // neighbours waiting for this particle are released in the same walk:
-    // they run in a later launch, which sees this launch's writes.
-    constexpr int kW = 8;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < cnt; q += gridDim.x * blockDim.x) {
-        const int t = in[q];
-        const int i = k.s0 + t;
-        const int a = off[t], b = off[t + 1];
-        const float4 pi = xs[i];
-        const float li = lam[i];
-        float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-        for (int e0 = a; e0 < b; e0 += kW) {
-            int j[kW];
+                                                      FluidK k, float dt, int* __restrict__ ctl) {
+    static_assert(kLanes == 16 || kLanes == 32 || kLanes == 64, "DPP rows");
+    constexpr int kChunk = kLanes * kPer, kBlockP = kBlock / kLanes;
+    constexpr int kRow = kChunk + 8;  // LDS floats per component (read eight at a time)
+    __shared__ float terms[kBlockP][3 * kRow];
+    __shared__ int ticket;
+    if (threadIdx.x == 0) ticket = atomicAdd(&ctl[kCtlTicket], 1);
+    __syncthreads();
+    const int lane = (int)(threadIdx.x & 63);
+    const int sub = lane & (kLanes - 1);
+    const int first = lane - sub;  // the particle's first lane
+    const unsigned long long group = (~0ull >> (64 - kLanes)) << first;
+    const int t = ticket * kBlockP + (int)threadIdx.x / kLanes;
+    float* const T = terms[threadIdx.x / kLanes];
+    bool live = t < k.n;
+    const int i = k.s0 + (live ? t : 0);
+    const int a = live ? off[t] : 0, b = live ? off[t + 1] : 0;
+    const float4 pi = xs[i];
+    const float p0 = reinterpret_cast<const float*>(x + i)[sub & 3];
+    const float li = lam[i];
+    unsigned long long* const out = reinterpret_cast<unsigned long long*>(xs2);
+    int j[kPer];
+    float ll[kPer];
+    SweepPos w[kPer];   // entry u's neighbour
+    unsigned int pend = 0u;  // bit u: it is missing
+    bool fresh = live;       // the chunk at c0 is to be taken
+    bool ask = live;         // ask for everything missing
+    int c0 = a, summed = 0;  // entries of the chunk in the sum
+    float f = 0.0f;          // component sub (< 3) of the sum
+    int chain = 0;
+    unsigned int have = 0u;  // bit u: entry u's position is here, its term is not
+    while (__any(live)) {
+        if (fresh) {
+            fresh = false;
+            summed = 0;
 #pragma unroll
-            for (int u = 0; u < kW; ++u) j[u] = (e0 + u < b) ? idx[e0 + u] : i;
-            float4 pj[kW];
-            float lt[kW];
-            int old[kW];
-#pragma unroll
-            for (int u = 0; u < kW; ++u) {
-                pj[u] = xs[j[u]];
-                // lambdas[j] with j the list position (:97); a list longer
+            for (int u = 0; u < kPer; ++u) {
+                const int e = c0 + sub + u * kLanes;
+                j[u] = e < b ? idx[e] : -1;
+                // lambdas[t] with t the list position (:97); a list longer
                 // than the lambdas array is reported after the step
-                const int tp = e0 + u - a;
-                lt[u] = (tp < k.nl) ? lam[tp] : 0.0f;
+                ll[u] = li + (e < b && e - a < k.nl ? lam[e - a] : 0.0f);
             }
 #pragma unroll
-            for (int u = 0; u < kW; ++u)
-                old[u] = (j[u] > i && j[u] < k.s0 + k.n) ? atomicSub(&indeg[j[u] - k.s0], 1) : 0;
-#pragma unroll
-            for (int u = 0; u < kW; ++u) {
-                if (e0 + u >= b) break;
-                const float dx = pi.x - pj[u].x, dy = pi.y - pj[u].y, dz = pi.z - pj[u].z;
-                const float len = sqrtf(dot3(dx, dy, dz, dx, dy, dz));
-                const float sc = -k.scorr_k * fl_pow(k, fl_cubic(k, len) / k.Wdq);
-                const float coef = (li + lt[u]) + sc;
-                float gx, gy, gz;
-                fl_cubic_grad(k, dx, dy, dz, &gx, &gy, &gz);
-                fx = fx + coef * gx;
-                fy = fy + coef * gy;
-                fz = fz + coef * gz;
+            for (int u = 0; u < kPer; ++u) {
+                const float4 p = xs[j[u] < 0 ? i : j[u]];
+                w[u].xy = pack2(p.x, p.y);
+                w[u].zc = pack2(p.z, 0.0f);
+                if (j[u] >= k.s0 && j[u] < i)
+                    pend |= 1u << u;
+                else if (j[u] >= 0)
+                    have |= 1u << u;
             }
-#pragma unroll
-            for (int u = 0; u < kW; ++u)
-                if (j[u] > i && j[u] < k.s0 + k.n && old[u] == 1) out[atomicAdd(out_cnt, 1)] = j[u] - k.s0;
         }
-        fx = fx / k.rho0;
-        fy = fy / k.rho0;
-        fz = fz / k.rho0;
-        float4 o;
-        o.x = fl_resolve(pi.x + fx, k.r, k.hi[0]);
-        o.y = fl_resolve(pi.y + fy, k.r, k.hi[1]);
-        o.z = fl_resolve(pi.z + fz, k.r, k.hi[2]);
-        o.w = 0.0f;
-        xs[i] = o;
-        const float4 p0 = x[i];
-        float4 vi;
-        vi.x = (o.x - p0.x) / dt;
-        vi.y = (o.y - p0.y) / dt;
-        vi.z = (o.z - p0.z) / dt;
-        vi.w = 0.0f;
-        v[i] = vi;
-        x[i] = o;
-        ++processed;
+        if (ask) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (pend >> u & 1u) w[u] = sweep_load(out, j[u]);
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if ((pend >> u & 1u) && w[u].here()) {
+                    pend &= ~(1u << u);
+                    have |= 1u << u;
+                }
+        }
+        // a term per lane and turn, whichever entry it is
+        while (__any((int)have)) {
+            if (have) {
+                // (a predicted position's chain length is 0)
+                SweepPos q = w[0];
+                float ql = ll[0];
+                int e = sub;
+#pragma unroll
+                for (int u = 1; u < kPer; ++u)
+                    if (!(have & ((1u << u) - 1u))) {
+                        q = w[u];
+                        ql = ll[u];
+                        e = sub + u * kLanes;
+                    }
+                fl_term<kPow4, kRow>(k, pi, __uint_as_float((unsigned int)q.xy), __uint_as_float((unsigned int)(q.xy >> 32)),
+                               __uint_as_float((unsigned int)q.zc), ql, T + e);
+                const int c = (int)(q.zc >> 32);
+                chain = c > chain ? c : chain;
+                have &= have - 1u;
+            }
+        }
+        wave_lds_sync();  // the terms are seen by the particle's other lanes
+        // the sum goes on, in list order, up to the first missing term
+        const int m = b - c0 < kChunk ? b - c0 : kChunk;
+        int upto = m;
+#pragma unroll
+        for (int u = kPer - 1; u >= 0; --u) {
+            const unsigned long long miss = __ballot(pend >> u & 1u) & group;
+            if (miss) upto = __ffsll(miss) - 1 - first + u * kLanes;
+        }
+        if (live && sub < 3) {
+            const float* const q = T + sub * kRow;
+            for (int e = summed; e < upto; e += 8) {
+                float w8[8];
+#pragma unroll
+                for (int d = 0; d < 8; ++d) w8[d] = q[e + d];
+#pragma unroll
+                for (int d = 0; d < 8; ++d)
+                    if (e + d < upto) f = f + w8[d];
+            }
+        }
+        summed = upto;
+        if (live && upto == m) {
+            c0 += kChunk;
+            if (c0 < b) {
+                fresh = true;
+            } else {
+                live = false;
+                chain = sweep_max<kLanes>(chain) + 1;
+                if (sub < 4) {
+                    // lanes 0..2: the components; lane 3: the chain length
+                    const float pc = sub == 0 ? pi.x : (sub == 1 ? pi.y : pi.z);
+                    const float hc = sub == 0 ? k.hi[0] : (sub == 1 ? k.hi[1] : k.hi[2]);
+                    const float o = fl_resolve(pc + f / k.rho0, k.r, hc);
+                    // an all-ones NaN is published as another NaN
+                    unsigned int word = __float_as_uint(o);
+                    word = word == kOpen ? kOpen >> 1 : word;
+                    __hip_atomic_store(reinterpret_cast<unsigned int*>(xs2 + i) + sub, sub < 3 ? word : (unsigned int)chain,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    reinterpret_cast<float*>(x + i)[sub] = sub < 3 ? o : 0.0f;
+                    reinterpret_cast<float*>(v + i)[sub] = sub < 3 ? (o - p0) / dt : 0.0f;
+                }
+            }
+        }
+        ask = fresh;
+        if (__any(fresh) || !__any(live)) continue;
+        // wait for a missing neighbour of any of the wave's particles
+        int top = -1, u0 = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            if ((pend >> u & 1u) && j[u] > top) {
+                top = j[u];
+                u0 = u;
+            }
+        const bool few = __popcll(__ballot(pend != 0u) & group) <= kSweepFew;
+        const bool asks = top >= 0 && (few || sweep_max<kLanes>(top) == top);
+        SweepPos q = {};
+        bool here = false;
+        int spins = 0;
+        do {
+            if (asks) {
+                q = sweep_load(out, top);
+                here = q.here();
+            }
+            if (__any(here)) break;
+            __builtin_amdgcn_s_sleep(kSweepPause);
+        } while (++spins < kSweepSpins);
+        if (spins >= kSweepSpins) {
+            if (lane == 0) atomicOr(&ctl[kCtlErr], kErrStall);
+            break;
+        }
+        if (here) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (u == u0) w[u] = q;
+            pend &= ~(1u << u0);
+            have |= 1u << u0;
+        }
+        ask = !few && (__ballot(here) & group) != 0ull;
     }
-    if (processed) atomicAdd(&ctl[kCtlDone], processed);
+    // the longest chain, one atomic per wave
+    for (int d = 32; d >= 1; d >>= 1) {
+        const int o = __shfl_xor(chain, d, 64);
+        chain = o > chain ? o : chain;
+    }
+    if (lane == 0) atomicMax(&ctl[kCtlLevels], chain);
+}
+
+template <int kLanes, int kPer>
+static void launch_sweep_lanes(float4* x, const float4* xs, float4* xs2, float4* v, const float* lam, const int* off,
+                               const int* idx, const FluidK& k, float dt, int* ctl, hipStream_t s) {
+    const dim3 g((k.n + kBlock / kLanes - 1) / (kBlock / kLanes)), b(kBlock);
+    if (k.ipow == 4)
+        launch_kernel((k_fl_sweep<true, kLanes, kPer>), g, b, 0, s, x, xs, xs2, v, lam, off, idx, k, dt, ctl);
+    else
+        launch_kernel((k_fl_sweep<false, kLanes, kPer>), g, b, 0, s, x, xs, xs2, v, lam, off, idx, k, dt, ctl);
+}
+
+// A wave per particle while the particles in flight (8,192 at 8 waves per
+// SIMD) cover most of the sweep's front, else four particles per wave
+// (measured, one / two / four per wave: 32 K at 870 links 2.8 / 3.6 / 4.4 ms,
+// 262 K 6.4 / 4.6 / 4.2 ms, 1 M 27 / 20 / 18 ms).
+constexpr int kSweepWideN = 65536;
+
+static hipError_t launch_sweep(float4* x, const float4* xs, float4* xs2, float4* v, const float* lam, const int* off,
+                               const int* idx, const FluidK& k, float dt, int* ctl, hipStream_t s) {
+    if (k.n <= kSweepWideN)
+        launch_sweep_lanes<64, 1>(x, xs, xs2, v, lam, off, idx, k, dt, ctl, s);
+    else
+        launch_sweep_lanes<16, 4>(x, xs, xs2, v, lam, off, idx, k, dt, ctl, s);
+    return hipGetLastError();
 }
 
 }  // namespace lus
@@ -550,9 +756,7 @@ int lus_fluid_init(LusGpu* c, const LusFluidParams* p, int total, int sand_start
     FL_HIP(fl_alloc(F, &F->cnt, n + 1));
     FL_HIP(fl_alloc(F, &F->off, n + 1));
     FL_HIP(fl_alloc(F, &F->ltiles, lus::scan_tile_count(n + 1) + 1));
-    FL_HIP(fl_alloc(F, &F->indeg, n));
-    FL_HIP(fl_alloc(F, &F->q0, n));
-    FL_HIP(fl_alloc(F, &F->q1, n));
+    FL_HIP(fl_alloc(F, &F->xs2, total));
     FL_HIP(fl_alloc(F, &F->ctl, lus::kCtlInts));
     FL_HIP(hipHostMalloc((void**)&F->host_ctl, sizeof(int) * lus::kCtlInts, hipHostMallocDefault));
     FL_HIP(hipMemsetAsync(F->counts, 0, sizeof(int) * (C + 1), s));
@@ -562,6 +766,7 @@ int lus_fluid_init(LusGpu* c, const LusFluidParams* p, int total, int sand_start
     FL_HIP(hipStreamSynchronize(s));
     h = aos_to_f4(positions_star, 0, total);
     FL_HIP(hipMemcpyAsync(F->xs, h.data(), sizeof(float4) * total, hipMemcpyHostToDevice, s));
+    FL_HIP(hipMemcpyAsync(F->xs2, F->xs, sizeof(float4) * total, hipMemcpyDeviceToDevice, s));
     FL_HIP(hipStreamSynchronize(s));
     std::vector<float4> hv((size_t)total, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     for (int i = sand_start; i < sand_end; ++i) {
@@ -627,8 +832,8 @@ int lus_fluid_step(LusGpu* c, float dt) {
         return LUS_OK;
     }
     const int gb = lus::grid_for(n);
-    lus::launch_kernel(lus::k_fl_predict, dim3(gb), dim3(lus::kBlock), 0, s, F->x, F->v, F->xs, k, dt, F->key,
-                       F->C, F->ctl);
+    lus::launch_kernel(lus::k_fl_predict, dim3(gb), dim3(lus::kBlock), 0, s, F->x, F->v, F->xs, F->xs2, k, dt,
+                       F->key, F->C, F->ctl);
     FL_HIP(hipGetLastError());
     // stable counting sort of the moving particles by cell
     FL_HIP(lus::launch_count_keys(F->key, n, F->counts, F->slot, s));
@@ -668,30 +873,14 @@ int lus_fluid_step(LusGpu* c, float dt) {
                        os, F->ocs, F->oref, k, (const int*)F->off, F->cnt, F->idx, 1);
     FL_HIP(hipGetLastError());
     lus::launch_kernel(lus::k_fl_lambda, dim3(gb), dim3(lus::kBlock), 0, s, (const float4*)F->xs,
-                       (const int*)F->off, (const int*)F->idx, k, F->lam, F->indeg, F->q0, F->ctl);
+                       (const int*)F->off, (const int*)F->idx, k, F->lam, F->ctl);
     FL_HIP(hipGetLastError());
-    // the sweep: one launch per dependency level, checked every kBatch levels
-    constexpr int kBatch = 32;
-    const int sweep_grid = std::min(lus::grid_for(n), 64);
-    int level = 0, done_prev = -1;
-    for (;;) {
-        for (int b = 0; b < kBatch; ++b, ++level) {
-            int* in = (level % 2 == 0) ? F->q0 : F->q1;
-            int* out = (level % 2 == 0) ? F->q1 : F->q0;
-            lus::launch_kernel(lus::k_fl_sweep, dim3(sweep_grid), dim3(lus::kBlock), 0, s, F->x, F->xs, F->v,
-                               (const float*)F->lam, (const int*)F->off, (const int*)F->idx, k, dt, level,
-                               (const int*)in, out, F->indeg, F->ctl);
-        }
-        FL_HIP(hipGetLastError());
-        FL_HIP(hipMemcpyAsync(F->host_ctl, F->ctl, sizeof(int) * lus::kCtlInts, hipMemcpyDeviceToHost, s));
-        FL_HIP(hipStreamSynchronize(s));
-        const int done = F->host_ctl[lus::kCtlDone];
-        if (done >= n) break;
-        if (done == done_prev)
-            return lus::report_error(LUS_EHIP, "lus_fluid_step: the sweep stopped after %d of %d particles", done,
-                                     n);
-        done_prev = done;
-    }
+    FL_HIP(lus::launch_sweep(F->x, F->xs, F->xs2, F->v, F->lam, F->off, F->idx, k, dt, F->ctl, s));
+    std::swap(F->xs, F->xs2);
+    FL_HIP(hipMemcpyAsync(F->host_ctl, F->ctl, sizeof(int) * lus::kCtlInts, hipMemcpyDeviceToHost, s));
+    FL_HIP(hipStreamSynchronize(s));
+    if (F->host_ctl[lus::kCtlErr] & lus::kErrStall)
+        return lus::report_error(LUS_EHIP, "lus_fluid_step: the sweep stopped waiting for a particle");
     F->last_levels = F->host_ctl[lus::kCtlLevels];
     if (F->host_ctl[lus::kCtlErr] & lus::kErrLambda)
         return lus::report_error(LUS_EINVAL,
