@@ -1455,72 +1455,34 @@ int lus_pbf_time_kernels(LusGpu* c, int reps, float* us) {
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int kChunk = 256;  // split-K chunk of the weight-gradient products
-
-// device buffers of one forward/backward pass over up to B rows
+// device buffers of one forward/backward pass over up to `rows` rows
 struct MlpBufs {
     Arena mem;
-    int B = 0, chunks = 0;
-    unsigned short *Xb = nullptr, *H1 = nullptr, *H2 = nullptr, *d3 = nullptr, *dZ2 = nullptr,
-                   *dZ1 = nullptr, *pbf = nullptr;  // bf16 storage
-    float *Yb = nullptr, *Z1 = nullptr, *Z2 = nullptr, *Z3 = nullptr, *dH2 = nullptr, *dH1 = nullptr,
-          *err = nullptr, *part = nullptr, *grad = nullptr, *acc = nullptr;
+    long ld = 0;  // row stride of the transposed activations
+    lus::MlpTrainAct act;
+    void *w = nullptr, *wt = nullptr;  // bf16 weights, as stored and transposed
+    float *err = nullptr, *part = nullptr, *grad = nullptr, *acc = nullptr;
     hipError_t alloc(int rows) {
-        B = rows;
-        chunks = (rows + kChunk - 1) / kChunk;
-        const size_t b = (size_t)rows;
+        const int chunks = (rows + lus::kMlpChunk - 1) / lus::kMlpChunk;
+        ld = (long)chunks * lus::kMlpChunk;
+        unsigned short* u = nullptr;  // bf16 storage
         hipError_t e;
-        if ((e = mem.alloc(&Xb, b * lus::kMlpIn)) || (e = mem.alloc(&H1, b * lus::kMlpHid)) ||
-            (e = mem.alloc(&H2, b * lus::kMlpHid)) || (e = mem.alloc(&d3, b * lus::kMlpOut)) ||
-            (e = mem.alloc(&dZ2, b * lus::kMlpHid)) || (e = mem.alloc(&dZ1, b * lus::kMlpHid)) ||
-            (e = mem.alloc(&pbf, lus::kMlpParams)) || (e = mem.alloc(&Yb, b * lus::kMlpOut)) ||
-            (e = mem.alloc(&Z1, b * lus::kMlpHid)) || (e = mem.alloc(&Z2, b * lus::kMlpHid)) ||
-            (e = mem.alloc(&Z3, b * lus::kMlpOut)) || (e = mem.alloc(&dH2, b * lus::kMlpHid)) ||
-            (e = mem.alloc(&dH1, b * lus::kMlpHid)) || (e = mem.alloc(&err, b)) ||
-            (e = mem.alloc(&part, (size_t)chunks * (lus::kMlpHid + 1) * lus::kMlpHid)) ||
-            (e = mem.alloc(&grad, lus::kMlpParams)) || (e = mem.alloc(&acc, 1)))
+        auto units = [&](int n, void** out) {
+            hipError_t r = mem.alloc(&u, (size_t)n * ld);
+            *out = u;
+            return r;
+        };
+        if ((e = units(lus::kMlpIn, &act.x)) || (e = units(lus::kMlpHid, &act.h1)) ||
+            (e = units(lus::kMlpHid, &act.h2)) || (e = units(lus::kMlpOut, &act.d3)) ||
+            (e = units(lus::kMlpHid, &act.dz2)) || (e = units(lus::kMlpHid, &act.dz1)))
             return e;
-        return hipSuccess;
+        if ((e = mem.alloc(&u, 2 * (lus::kMlpParams + 8)))) return e;
+        w = u;
+        wt = u + (lus::kMlpParams + 7) / 8 * 8;
+        if ((e = mem.alloc(&err, rows)) || (e = mem.alloc(&grad, lus::kMlpParams)) || (e = mem.alloc(&acc, 1))) return e;
+        return chunks > lus::kMlpFuseChunks ? mem.alloc(&part, (size_t)chunks * lus::kMlpParams) : hipSuccess;
     }
 };
-
-// Forward pass of the training kernels over `rows` rows of b.Xb / b.Yb with
-// fp32 parameters p; err[r] = squared error of row r.  grad: also the
-// backward pass, gradient of the mean loss into b.grad.
-//   Z1 = X W1, H1 = bf16(silu(Z1 + b1)), Z2 = H1 W2, H2 = bf16(silu(Z2 + b2)),
-//   o = H2 W3 + b3;  dW|db = [A^T; 1] dZ per layer (bf16 operands)
-int mlp_pass(hipStream_t s, MlpBufs& b, const float* p, int rows, float inv_scale, bool grad) {
-    using namespace lus;
-    const unsigned short* W1 = b.pbf + kMlpW1;
-    const unsigned short* W2 = b.pbf + kMlpW2;
-    const unsigned short* W3 = b.pbf + kMlpW3;
-    LUS_HIP(launch_to_bf16(p, kMlpParams, b.pbf, s));
-    LUS_HIP(launch_gemm_bf16(b.Xb, kMlpIn, 1, W1, kMlpHid, 1, b.Z1, kMlpHid, rows, kMlpHid, kMlpIn, 32, 0, s));
-    LUS_HIP(launch_bias_silu(b.Z1, p + kMlpB1, rows, kMlpHid, b.H1, s));
-    LUS_HIP(launch_gemm_bf16(b.H1, kMlpHid, 1, W2, kMlpHid, 1, b.Z2, kMlpHid, rows, kMlpHid, kMlpHid, 64, 0, s));
-    LUS_HIP(launch_bias_silu(b.Z2, p + kMlpB2, rows, kMlpHid, b.H2, s));
-    LUS_HIP(launch_gemm_bf16(b.H2, kMlpHid, 1, W3, kMlpOut, 1, b.Z3, kMlpOut, rows, kMlpOut, kMlpHid, 64, 0, s));
-    LUS_HIP(launch_out_loss(b.Z3, p + kMlpB3, b.Yb, rows, inv_scale, b.d3, b.err, s));
-    if (!grad) return LUS_OK;
-    const int ch = (rows + kChunk - 1) / kChunk;
-    // layer 3: [H2^T; 1] d3 -> dW3|db3; dH2 = d3 W3^T
-    LUS_HIP(launch_gemm_bf16(b.H2, 1, kMlpHid, b.d3, kMlpOut, 1, b.part, kMlpOut, kMlpHid + 1, kMlpOut, rows,
-                             kChunk, 1, s));
-    LUS_HIP(launch_sum_partials(b.part, ch, (kMlpHid + 1) * kMlpOut, b.grad + kMlpW3, s));
-    LUS_HIP(launch_gemm_bf16(b.d3, kMlpOut, 1, W3, 1, kMlpOut, b.dH2, kMlpHid, rows, kMlpHid, kMlpOut, 32, 0, s));
-    LUS_HIP(launch_silu_back(b.dH2, b.Z2, (long)rows * kMlpHid, b.dZ2, s));
-    // layer 2
-    LUS_HIP(launch_gemm_bf16(b.H1, 1, kMlpHid, b.dZ2, kMlpHid, 1, b.part, kMlpHid, kMlpHid + 1, kMlpHid, rows,
-                             kChunk, 1, s));
-    LUS_HIP(launch_sum_partials(b.part, ch, (kMlpHid + 1) * kMlpHid, b.grad + kMlpW2, s));
-    LUS_HIP(launch_gemm_bf16(b.dZ2, kMlpHid, 1, W2, 1, kMlpHid, b.dH1, kMlpHid, rows, kMlpHid, kMlpHid, 64, 0, s));
-    LUS_HIP(launch_silu_back(b.dH1, b.Z1, (long)rows * kMlpHid, b.dZ1, s));
-    // layer 1
-    LUS_HIP(launch_gemm_bf16(b.Xb, 1, kMlpIn, b.dZ1, kMlpHid, 1, b.part, kMlpHid, kMlpIn + 1, kMlpHid, rows,
-                             kChunk, 1, s));
-    LUS_HIP(launch_sum_partials(b.part, ch, (kMlpIn + 1) * kMlpHid, b.grad + kMlpW1, s));
-    return LUS_OK;
-}
 
 bool net_layout_ok(int nfloats) { return nfloats == LUS_NET_FLOATS; }
 
@@ -1785,27 +1747,37 @@ int lus_mlp_fit(LusMlpTrainer* t, const LusMlpFitParams* fp, float* train_loss, 
     const long nb = ntr / B;
     const double total = (double)fp->epochs * (double)nb;
     long step = 0;
+    MlpAdam ad;
+    ad.p = dp;
+    ad.m = dm;
+    ad.v = dv;
+    ad.w = b.w;
+    ad.wt = b.wt;
+    ad.b1 = 0.9f;
+    ad.b2 = 0.999f;
+    ad.eps = 1e-8f;
+    LUS_HIP(launch_mlp_train_pack(dp, b.w, b.wt, s));
     for (int e = 0; e < fp->epochs; ++e) {
         std::shuffle(tr.begin(), tr.end(), rng);
         LUS_HIP(hipStreamSynchronize(s));
         LUS_HIP(hipMemcpy(dtr, tr.data(), sizeof(int) * ntr, hipMemcpyHostToDevice));
         for (long q = 0; q < nb; ++q) {
-            LUS_HIP(launch_normalize_rows(t->feat, dtr + q * B, B, dmu, dinv, b.Xb, s));
-            LUS_HIP(launch_gather_rows(t->tgt, dtr + q * B, B, 3, b.Yb, s));
-            if (int r = mlp_pass(s, b, dp, B, inv_scale, true)) return r;
             ++step;
             const double cosw = 0.5 * (1.0 + std::cos(M_PI * (double)(step - 1) / total));
             const float lr = (float)(fp->lr_final + (fp->lr - fp->lr_final) * cosw);
             const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)step)));
             const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)step)));
-            LUS_HIP(launch_adam(dp, b.grad, dm, dv, kMlpParams, lr, 0.9f, 0.999f, 1e-8f, c1, c2, s));
-            LUS_HIP(launch_sum_into(b.err, B, tl + e, s));
+            ad.lr = lr;
+            ad.c1 = c1;
+            ad.c2 = c2;
+            LUS_HIP(launch_mlp_train_rows(t->feat, t->tgt, dtr + q * B, B, dmu, dinv, inv_scale, dp, b.w, b.wt, b.err,
+                                          &b.act, b.ld, s));
+            LUS_HIP(launch_mlp_train_weights(b.act, b.ld, B, ad, b.part ? b.grad : nullptr, b.part, b.err, tl + e, s));
         }
         for (long q = 0; q < nval; q += B) {
             const int rr = (int)std::min<long>(B, nval - q);
-            LUS_HIP(launch_normalize_rows(t->feat, dval + q, rr, dmu, dinv, b.Xb, s));
-            LUS_HIP(launch_gather_rows(t->tgt, dval + q, rr, 3, b.Yb, s));
-            if (int r = mlp_pass(s, b, dp, rr, inv_scale, false)) return r;
+            LUS_HIP(launch_mlp_train_rows(t->feat, t->tgt, dval + q, rr, dmu, dinv, inv_scale, dp, b.w, b.wt, b.err,
+                                          nullptr, b.ld, s));
             LUS_HIP(launch_sum_into(b.err, rr, vl + e, s));
         }
     }
@@ -1843,19 +1815,21 @@ int lus_mlp_loss_grad(LusGpu* c, const float* params, int rows, const float* X, 
     LUS_HIP(hipSetDevice(c->device));
     LUS_HIP(hipStreamSynchronize(s));
     Arena m;
-    float *dp, *dx;
+    float *dp, *dx, *dy;
     LUS_HIP(m.alloc(&dp, kMlpParams));
     LUS_HIP(m.alloc(&dx, (size_t)rows * kMlpIn));
+    LUS_HIP(m.alloc(&dy, (size_t)rows * kMlpOut));
     MlpBufs b;
     LUS_HIP(b.alloc(rows));
     LUS_HIP(hipMemcpy(dp, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice));
     LUS_HIP(hipMemcpy(dx, X, sizeof(float) * kMlpIn * rows, hipMemcpyHostToDevice));
-    LUS_HIP(hipMemcpy(b.Yb, Y, sizeof(float) * kMlpOut * rows, hipMemcpyHostToDevice));
+    LUS_HIP(hipMemcpy(dy, Y, sizeof(float) * kMlpOut * rows, hipMemcpyHostToDevice));
     LUS_HIP(hipMemset(b.acc, 0, sizeof(float)));
     LUS_HIP(hipDeviceSynchronize());
-    LUS_HIP(launch_to_bf16(dx, (long)rows * kMlpIn, b.Xb, s));
-    if (int r = mlp_pass(s, b, dp, rows, inv_scale, true)) return r;
-    LUS_HIP(launch_sum_into(b.err, rows, b.acc, s));
+    LUS_HIP(launch_mlp_train_pack(dp, b.w, b.wt, s));
+    LUS_HIP(launch_mlp_train_rows(dx, dy, nullptr, rows, nullptr, nullptr, inv_scale, dp, b.w, b.wt, b.err, &b.act,
+                                  b.ld, s));
+    LUS_HIP(launch_mlp_train_weights(b.act, b.ld, rows, MlpAdam(), b.grad, b.part, b.err, b.acc, s));
     LUS_HIP(hipStreamSynchronize(s));
     float acc = 0.0f;
     LUS_HIP(hipMemcpy(&acc, b.acc, sizeof(float), hipMemcpyDeviceToHost));

@@ -322,8 +322,8 @@ __global__ __launch_bounds__(kBlock) void k_fl_lambda(const float4* __restrict__
 // What bounds it is the longest chain of waits, 2.7 to 3.2 us a link at 32 K
 // particles (a bare store and load between two XCDs takes 0.6; the rest is the
 // last term, its sum and the divides).  One launch per level took 36 us a
-// link: 32 K particles, 218 to 870 links, step 8 to 29 ms -> 0.85 to 2.8 ms;
-// 1 M, 762 links, step 67 -> 18 ms.  A particle that waits for many neighbours
+// link and more: 32 K particles, 218 to 870 links, step 8.7 to 66 -> 0.85 to 2.8 ms;
+// 1 M, 762 links, step 37 -> 18 ms.  A particle that waits for many neighbours
 // asks for the latest of them only, one that waits for at most kSweepFew asks
 // for each, with a pause between (1, 4, 10, 30 x 64 cycles at the 870 links:
 // 3.4, 2.9, 2.8, 2.8 ms), so that the waves far from the front leave the ones

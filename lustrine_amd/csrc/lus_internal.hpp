@@ -273,23 +273,30 @@ hipError_t launch_mlp_forward(const void* X, int n, const float* params, const v
                               float out_scale, float* out, const float4* xp, float4* xa,
                               const PbfK& k, hipStream_t s);
 // training kernels (row-major fp32 / bf16 matrices)
-hipError_t launch_gemm_bf16(const void* A, long sam, long sak, const void* B, long sbk, long sbn,
-                            float* C, int ldc, int M, int N, int K, int kchunk, int ones_row,
-                            hipStream_t s);
+hipError_t launch_mlp_train_pack(const float* params, void* w, void* wt, hipStream_t s);
+// transposed bf16 activations and activation gradients of a batch, [units][ld]
+struct MlpTrainAct {
+    void *x = nullptr, *h1 = nullptr, *h2 = nullptr, *d3 = nullptr, *dz2 = nullptr, *dz1 = nullptr;
+};
+// Adam state and step constants: c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
+struct MlpAdam {
+    float *p = nullptr, *m = nullptr, *v = nullptr;
+    void *w = nullptr, *wt = nullptr;  // bf16 copies kept with p
+    float lr = 0.0f, b1 = 0.0f, b2 = 0.0f, eps = 0.0f, c1 = 0.0f, c2 = 0.0f;
+};
+constexpr int kMlpChunk = 256;      // rows per partial sum of a weight gradient
+constexpr int kMlpFuseChunks = 64;  // chunks up to which the weight gradients need no partials in memory
+hipError_t launch_mlp_train_rows(const float* feat, const float* tgt, const int* sel, int rows, const float* mu,
+                                 const float* inv_sigma, float inv_scale, const float* params, const void* w,
+                                 const void* wt, float* err, const MlpTrainAct* act, long ld, hipStream_t s);
+// grad and part: needed past kMlpFuseChunks chunks (part: chunks * kMlpParams floats)
+hipError_t launch_mlp_train_weights(const MlpTrainAct& act, long ld, int rows, const MlpAdam& adam, float* grad,
+                                    float* part, const float* err, float* loss_acc, hipStream_t s);
 hipError_t launch_sum_partials(const float* part, int chunks, int MN, float* out, hipStream_t s);
-hipError_t launch_bias_silu(float* z, const float* bias, int rows, int N, void* h, hipStream_t s);
-hipError_t launch_out_loss(const float* z3, const float* b3, const float* y, int rows,
-                           float inv_scale, void* dbf, float* err, hipStream_t s);
-hipError_t launch_silu_back(const float* dh, const float* z, long tot, void* dzb, hipStream_t s);
-hipError_t launch_to_bf16(const float* a, long tot, void* b, hipStream_t s);
 hipError_t launch_normalize_rows(const float* x, const int* rows, long nrows, const float* mu,
                                  const float* inv_sigma, void* xb, hipStream_t s);
-hipError_t launch_gather_rows(const float* y, const int* rows, long nrows, int w, float* out,
-                              hipStream_t s);
 hipError_t launch_sum_into(const float* v, int n, float* acc, hipStream_t s);
 hipError_t launch_col_stats(const float* x, long rows, int w, double* out, hipStream_t s);
-hipError_t launch_adam(float* p, const float* g, float* m, float* v, int np, float lr, float b1,
-                       float b2, float eps, float c1, float c2, hipStream_t s);
 
 // sand (simulate_sand)
 hipError_t launch_sand_predict_key(float4* x, float4* v, int* att, int n, SandK k, float dt, int* err,

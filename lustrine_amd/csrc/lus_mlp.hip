@@ -187,53 +187,234 @@ hipError_t launch_mlp_forward(const void* X, int n, const float* params, const v
 }
 
 // ------------------------------------------------------------------ training
-// C[M][N] (fp32, row stride ldc) = sum_k A(m,k) B(k,n) over bf16 operands
-// addressed through strides: A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn].
-// ones_row: row M-1 of A is all ones (not read), which appends the column
-// sums of B -- the bias gradient under the weight gradient.  One wave per
-// 16x16 C tile; blockIdx.y takes K in chunks of kchunk (a multiple of 32) and
-// writes C + blockIdx.y * M * ldc, summed afterwards in chunk order, so the
-// result does not depend on scheduling.
-__global__ __launch_bounds__(64) void k_gemm_bf16(const __bf16* __restrict__ A, long sam, long sak,
-                                                  const __bf16* __restrict__ B, long sbk, long sbn,
-                                                  float* __restrict__ C, int ldc, int M, int N, int K,
-                                                  int kchunk, int ones_row) {
-    const int lane = threadIdx.x;
-    const int col = lane % 16, grp = lane / 16;
-    const int tiles_n = (N + 15) / 16;
-    const int m0 = (blockIdx.x / tiles_n) * 16, n0 = (blockIdx.x % tiles_n) * 16;
-    const int kb = blockIdx.y * kchunk;
-    const int ke = min(K, kb + kchunk);
-    const int m = m0 + col, nn = n0 + col;
-    const bool ones = ones_row && m == M - 1;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = kb; k0 < ke; k0 += 32) {
-        bf16x8 a, b;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int kk = k0 + 8 * grp + e;
-            const bool kin = kk < ke;
-            a[e] = (m < M && kin) ? (ones ? (__bf16)1.0f : A[m * sam + kk * sak]) : (__bf16)0.0f;
-            b[e] = (nn < N && kin) ? B[kk * sbk + nn * sbn] : (__bf16)0.0f;
-        }
-        acc = mfma(a, b, acc);
-    }
-    float* Cc = C + (size_t)blockIdx.y * M * ldc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int mr = m0 + 4 * grp + i;
-        if (mr < M && nn < N) Cc[(size_t)mr * ldc + nn] = acc[i];
+// A training step is two launches: k_mlp_train_rows takes a batch's rows
+// forward and backward to the activations' gradients, k_mlp_train_weights
+// contracts them over the rows to the weights' gradients and applies Adam.
+// One launch per product and per elementwise pass (24 of 2 to 6 us each) took
+// 97 us per step of 4,096 rows, all of it launches and their tails (a fit of
+// 131,072 rows over 4 epochs: 11.7 -> 3.7 ms, the same bits).
+//
+// The weights are kept in bf16 twice, as stored ([fan_in][fan_out], w) and
+// transposed ([fan_out][fan_in], wt), each layer at its fp32 offset, so that
+// either product reads a lane's eight reduction elements as one 16-byte load.
+// The activations the weight gradients need go out transposed ([unit][row],
+// row stride ld) for the same reason.
+
+// w and wt from the fp32 parameters
+__global__ void k_mlp_train_pack(const float* __restrict__ p, __bf16* __restrict__ w, __bf16* __restrict__ wt) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= kMlpParams) return;
+    const __bf16 v = (__bf16)p[t];
+    w[t] = v;
+    if (t < kMlpB1) {
+        wt[(t % kMlpHid) * kMlpIn + t / kMlpHid] = v;
+    } else if (t >= kMlpW2 && t < kMlpB2) {
+        const int q = t - kMlpW2;
+        wt[kMlpW2 + (q % kMlpHid) * kMlpHid + q / kMlpHid] = v;
+    } else if (t >= kMlpW3 && t < kMlpB3) {
+        const int q = t - kMlpW3;
+        wt[kMlpW3 + (q % kMlpOut) * kMlpHid + q / kMlpOut] = v;
     }
 }
 
-hipError_t launch_gemm_bf16(const void* A, long sam, long sak, const void* B, long sbk, long sbn,
-                            float* C, int ldc, int M, int N, int K, int kchunk, int ones_row,
-                            hipStream_t s) {
-    if (kchunk <= 0 || kchunk % 32) return hipErrorInvalidValue;
-    const int tiles = ((M + 15) / 16) * ((N + 15) / 16);
-    const int chunks = (K + kchunk - 1) / kchunk;
-    launch_kernel(k_gemm_bf16, dim3(tiles, chunks), dim3(64), 0, s, (const __bf16*)A, sam, sak,
-                       (const __bf16*)B, sbk, sbn, C, ldc, M, N, K, kchunk, ones_row);
+hipError_t launch_mlp_train_pack(const float* params, void* w, void* wt, hipStream_t s) {
+    launch_kernel(k_mlp_train_pack, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, params, (__bf16*)w, (__bf16*)wt);
+    return hipGetLastError();
+}
+
+// Sixteen rows per block, wave j computing units 16j..16j+15 of a layer (its
+// z values stay in registers for the backward pass; the layers meet in LDS).
+// Row r is row sel[r] (sel null: r) of feat and tgt; inputs are
+// bf16((x - mu) inv_sigma), or bf16(x) without mu.
+//   err[r] = sum_c (o_rc - y_rc inv_scale)^2, the loss is their mean
+// kGrad: also the transposed activations and gradients t (rows past `rows` as
+// zeros, up to the grid's end).  Latency of the four layers' chain bounds it:
+// one block per CU at 4,096 rows.
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+template <bool kGrad>
+__global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict__ feat, const float* __restrict__ tgt,
+                                                        const int* __restrict__ sel, int rows,
+                                                        const float* __restrict__ mu,
+                                                        const float* __restrict__ inv_sigma, float inv_scale,
+                                                        const float* __restrict__ p, const __bf16* __restrict__ w,
+                                                        const __bf16* __restrict__ wt, float* __restrict__ err,
+                                                        MlpTrainAct t, long ld) {
+    constexpr int kStride = kMlpHid + 8;  // LDS row stride (16-byte aligned rows, spread over the banks)
+    __shared__ __attribute__((aligned(16))) __bf16 H1[16][kStride], H2[16][kStride], D[16][kStride];
+    __shared__ __bf16 d3[16][4];
+    __shared__ float sq[16][4];
+    const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;
+    const int col = lane % 16, grp = lane / 16;
+    const int m0 = blockIdx.x * 16;
+    const int n = 16 * j + col;       // this lane's unit (C columns, B columns)
+    const int c0 = m0 + 4 * grp;      // and first row (C rows)
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    bool in[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) in[i] = c0 + i < rows;
+    // layer 1
+    bf16x8 a = {};
+    {
+        const int r = m0 + col;
+        if (r < rows) {
+            const float4* x = reinterpret_cast<const float4*>(feat + (size_t)(sel ? sel[r] : r) * kMlpIn + 8 * grp);
+            const float4 q0 = x[0], q1 = x[1];
+            const float v[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                a[e] = mu ? (__bf16)((v[e] - mu[8 * grp + e]) * inv_sigma[8 * grp + e]) : (__bf16)v[e];
+        }
+        if (kGrad && j == 0) {
+            __bf16* xt = (__bf16*)t.x;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xt[(8 * grp + e) * ld + r] = a[e];
+        }
+    }
+    const f32x4 y1 = mfma(a, *reinterpret_cast<const bf16x8*>(wt + kMlpW1 + n * kMlpIn + 8 * grp), zero);
+    float z1[4], z2[4];
+    bf16x4 h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z1[i] = y1[i] + p[kMlpB1 + n];
+        h[i] = in[i] ? (__bf16)silu(z1[i]) : (__bf16)0.0f;
+        H1[4 * grp + i][n] = h[i];
+    }
+    if (kGrad) *reinterpret_cast<bf16x4*>((__bf16*)t.h1 + n * ld + c0) = h;
+    __syncthreads();
+    // layer 2
+    f32x4 y2 = zero;
+#pragma unroll
+    for (int k = 0; k < kMlpHid; k += 32)
+        y2 = mfma(*reinterpret_cast<const bf16x8*>(&H1[col][k + 8 * grp]),
+                  *reinterpret_cast<const bf16x8*>(wt + kMlpW2 + n * kMlpHid + k + 8 * grp), y2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z2[i] = y2[i] + p[kMlpB2 + n];
+        h[i] = in[i] ? (__bf16)silu(z2[i]) : (__bf16)0.0f;
+        H2[4 * grp + i][n] = h[i];
+    }
+    if (kGrad) *reinterpret_cast<bf16x4*>((__bf16*)t.h2 + n * ld + c0) = h;
+    __syncthreads();
+    // output and loss (wave 0)
+    if (j == 0) {
+        f32x4 o = zero;
+#pragma unroll
+        for (int k = 0; k < kMlpHid; k += 32) {
+            bf16x8 b = {};
+            if (col < kMlpOut) b = *reinterpret_cast<const bf16x8*>(wt + kMlpW3 + col * kMlpHid + k + 8 * grp);
+            o = mfma(*reinterpret_cast<const bf16x8*>(&H2[col][k + 8 * grp]), b, o);
+        }
+        if (col < kMlpOut) {
+            bf16x4 d;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float diff = 0.0f;
+                if (in[i])
+                    diff = (o[i] + p[kMlpB3 + col]) - tgt[(size_t)(sel ? sel[c0 + i] : c0 + i) * kMlpOut + col] * inv_scale;
+                d[i] = (__bf16)(2.0f * diff / (float)rows);
+                d3[4 * grp + i][col] = d[i];
+                sq[4 * grp + i][col] = diff * diff;
+            }
+            if (kGrad) *reinterpret_cast<bf16x4*>((__bf16*)t.d3 + col * ld + c0) = d;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 16 && m0 + (int)threadIdx.x < rows) {
+        float e = 0.0f;
+#pragma unroll
+        for (int c = 0; c < kMlpOut; ++c) e += sq[threadIdx.x][c];
+        err[m0 + threadIdx.x] = e;
+    }
+    if (!kGrad) return;
+    // back through layer 3: dH2 = d3 W3^T
+    bf16x8 b = {};
+    a = b;
+    if (grp == 0) {
+#pragma unroll
+        for (int c = 0; c < kMlpOut; ++c) {
+            a[c] = d3[col][c];
+            b[c] = w[kMlpW3 + n * kMlpOut + c];
+        }
+    }
+    const f32x4 g2 = mfma(a, b, zero);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = in[i] ? (__bf16)(g2[i] * silu_grad(z2[i])) : (__bf16)0.0f;
+        D[4 * grp + i][n] = h[i];
+    }
+    *reinterpret_cast<bf16x4*>((__bf16*)t.dz2 + n * ld + c0) = h;
+    __syncthreads();
+    // layer 2: dH1 = dZ2 W2^T
+    f32x4 g1 = zero;
+#pragma unroll
+    for (int k = 0; k < kMlpHid; k += 32)
+        g1 = mfma(*reinterpret_cast<const bf16x8*>(&D[col][k + 8 * grp]),
+                  *reinterpret_cast<const bf16x8*>(w + kMlpW2 + n * kMlpHid + k + 8 * grp), g1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = in[i] ? (__bf16)(g1[i] * silu_grad(z1[i])) : (__bf16)0.0f;
+    *reinterpret_cast<bf16x4*>((__bf16*)t.dz1 + n * ld + c0) = h;
+}
+
+hipError_t launch_mlp_train_rows(const float* feat, const float* tgt, const int* sel, int rows, const float* mu,
+                                 const float* inv_sigma, float inv_scale, const float* params, const void* w,
+                                 const void* wt, float* err, const MlpTrainAct* act, long ld, hipStream_t s) {
+    if (act) {
+        // rows up to the next multiple of 32 (a matrix step of the weight gradients) written, as zeros
+        const int tiles = 2 * ((rows + 31) / 32);
+        if ((long)tiles * 16 > ld || ld % 32) return hipErrorInvalidValue;
+        launch_kernel((k_mlp_train_rows<true>), dim3(tiles), dim3(256), 0, s, feat, tgt, sel, rows, mu, inv_sigma,
+                      inv_scale, params, (const __bf16*)w, (const __bf16*)wt, err, *act, ld);
+    } else {
+        launch_kernel((k_mlp_train_rows<false>), dim3((rows + 15) / 16), dim3(256), 0, s, feat, tgt, sel, rows, mu,
+                      inv_sigma, inv_scale, params, (const __bf16*)w, (const __bf16*)wt, err, MlpTrainAct(), ld);
+    }
+    return hipGetLastError();
+}
+
+// Adam (Kingma & Ba, ICLR 2015) on the fp32 master parameters; returns the
+// updated parameter
+__device__ __forceinline__ float adam_step(const MlpAdam& a, int t, float g) {
+    const float mt = a.b1 * a.m[t] + (1.0f - a.b1) * g;
+    const float vt = a.b2 * a.v[t] + (1.0f - a.b2) * g * g;
+    a.m[t] = mt;
+    a.v[t] = vt;
+    const float p = a.p[t] - a.lr * (mt * a.c1) / (sqrtf(vt * a.c2) + a.eps);
+    a.p[t] = p;
+    return p;
+}
+
+__global__ void k_adam(MlpAdam a, const float* __restrict__ g) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < kMlpParams) adam_step(a, t, g[t]);
+}
+
+// *acc += the sum of v[0..n): 256 strided sums, then a tree (every thread of
+// the block calls it)
+__device__ __forceinline__ void block_sum_into(const float* __restrict__ v, int n, float* __restrict__ acc,
+                                               float* part) {
+    const int t = (int)threadIdx.x;
+    if (t < 256) {
+        float s = 0.0f;
+        for (int i = t; i < n; i += 256) s += v[i];
+        part[t] = s;
+    }
+    __syncthreads();
+    for (int d = 128; d >= 1; d >>= 1) {
+        if (t < d) part[t] += part[t + d];
+        __syncthreads();
+    }
+    if (t == 0) acc[0] += part[0];
+}
+
+// *acc += sum of v[0..n), one block
+__global__ __launch_bounds__(256) void k_sum_into(const float* __restrict__ v, int n, float* __restrict__ acc) {
+    __shared__ float part[256];
+    block_sum_into(v, n, acc, part);
+}
+
+hipError_t launch_sum_into(const float* v, int n, float* acc, hipStream_t s) {
+    launch_kernel(k_sum_into, dim3(1), dim3(256), 0, s, v, n, acc);
     return hipGetLastError();
 }
 
@@ -251,69 +432,124 @@ hipError_t launch_sum_partials(const float* part, int chunks, int MN, float* out
     return hipGetLastError();
 }
 
-// z[r][c] += bias[c]; h = bf16(silu(z)); z (fp32, with bias) kept for the backward pass
-__global__ void k_bias_silu(float* __restrict__ z, const float* __restrict__ bias, int rows, int N,
-                            __bf16* __restrict__ h) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)rows * N) return;
-    const float v = z[t] + bias[t % N];
-    z[t] = v;
-    h[t] = (__bf16)silu(v);
-}
+// Weight gradients: per layer [A^T; 1] dZ over the rows, the row of ones giving
+// the bias gradient under the weight gradient.  One block per 16 x 16 tile of a layer's
+// [fan_in + 1][fan_out] gradient; its waves take the row chunks of kMlpChunk
+// in turn (sixteen at a time) and the chunks' sums are added in chunk order, so the
+// result does not depend on scheduling.
+//   adam      the tile's parameters are updated from their gradient (and w, wt)
+//   otherwise the gradient goes to grad
+//   part      (blockIdx.y > 0 too) every chunk's sum goes to part for
+//             k_sum_partials: many chunks keep more than these blocks busy
+// The block after the last tile adds the rows' err to *loss_acc.
+constexpr int kTrainTiles1 = 3 * 4, kTrainTiles2 = 5 * 4, kTrainTiles3 = 5;
+constexpr int kTrainTiles = kTrainTiles1 + kTrainTiles2 + kTrainTiles3;
+constexpr int kTrainWaves = 16;
 
-hipError_t launch_bias_silu(float* z, const float* bias, int rows, int N, void* h, hipStream_t s) {
-    const long tot = (long)rows * N;
-    launch_kernel(k_bias_silu, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, z, bias, rows, N,
-                       (__bf16*)h);
-    return hipGetLastError();
-}
-
-// Loss L = (1/rows) sum_r sum_c (o_rc - y_rc * inv_scale)^2 with o = z3 + b3.
-// dbf = bf16(dL/do); err[r] = sum_c (o_rc - y_rc * inv_scale)^2.
-__global__ void k_out_loss(const float* __restrict__ z3, const float* __restrict__ b3,
-                           const float* __restrict__ y, int rows, float inv_scale,
-                           __bf16* __restrict__ dbf, float* __restrict__ err) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    float e = 0.0f;
-    for (int c = 0; c < 3; ++c) {
-        const float o = z3[(size_t)r * 3 + c] + b3[c];
-        const float diff = o - y[(size_t)r * 3 + c] * inv_scale;
-        dbf[(size_t)r * 3 + c] = (__bf16)(2.0f * diff / (float)rows);
-        e += diff * diff;
+__global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train_weights(MlpTrainAct act, long ld, int rows, MlpAdam ad,
+                                                                        float* __restrict__ grad,
+                                                                        float* __restrict__ part,
+                                                                        const float* __restrict__ err,
+                                                                        float* __restrict__ loss_acc) {
+    __shared__ float sum[kTrainWaves][256];
+    int tile = blockIdx.x;
+    if (tile == kTrainTiles) {
+        block_sum_into(err, rows, loss_acc, sum[0]);
+        return;
     }
-    err[r] = e;
+    const __bf16 *A, *B;
+    int M, N, off;
+    if (tile < kTrainTiles1) {
+        A = (const __bf16*)act.x, B = (const __bf16*)act.dz1, M = kMlpIn + 1, N = kMlpHid, off = kMlpW1;
+    } else if (tile < kTrainTiles1 + kTrainTiles2) {
+        tile -= kTrainTiles1;
+        A = (const __bf16*)act.h1, B = (const __bf16*)act.dz2, M = kMlpHid + 1, N = kMlpHid, off = kMlpW2;
+    } else {
+        tile -= kTrainTiles1 + kTrainTiles2;
+        A = (const __bf16*)act.h2, B = (const __bf16*)act.d3, M = kMlpHid + 1, N = kMlpOut, off = kMlpW3;
+    }
+    const int tiles_n = (N + 15) / 16;
+    const int m0 = (tile / tiles_n) * 16, n0 = (tile % tiles_n) * 16;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int col = lane % 16, grp = lane / 16;
+    const int m = m0 + col, nn = n0 + col;
+    const int chunks = (rows + kMlpChunk - 1) / kMlpChunk;
+    const int t = (int)threadIdx.x;
+    const int mr = m0 + t / 16, nc = n0 + t % 16;  // thread t < 256: its element of the tile
+    const bool mine = t < 256 && mr < M && nc < N;
+    float total = 0.0f;
+    const int g1 = (chunks + kTrainWaves - 1) / kTrainWaves;
+    for (int g = blockIdx.y; g < g1; g += gridDim.y) {
+        const int c = g * kTrainWaves + wv;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < chunks) {
+            const int ke = rows < (c + 1) * kMlpChunk ? rows : (c + 1) * kMlpChunk;
+#pragma unroll 4
+            for (int k = c * kMlpChunk; k < ke; k += 32) {
+                bf16x8 a = {}, b = {};
+                if (m < M - 1) {
+                    a = *reinterpret_cast<const bf16x8*>(A + m * ld + k + 8 * grp);
+                } else if (m == M - 1) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) a[e] = (__bf16)1.0f;
+                }
+                if (nn < N) b = *reinterpret_cast<const bf16x8*>(B + nn * ld + k + 8 * grp);
+                acc = mfma(a, b, acc);
+            }
+            if (part) {
+                // partials of layer 1, then 2, then 3, each [chunk][M][N]
+                const size_t base = (size_t)chunks * (off == kMlpW1 ? 0 : (off == kMlpW2 ? kMlpW2 : kMlpW3));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = m0 + 4 * grp + i;
+                    if (r < M && nn < N) part[base + ((size_t)c * M + r) * N + nn] = acc[i];
+                }
+            }
+        }
+        if (part) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[wv][(4 * grp + i) * 16 + col] = acc[i];
+        __syncthreads();
+        if (mine) {
+            const int left = chunks - g * kTrainWaves;
+            for (int q = 0; q < kTrainWaves && q < left; ++q) total += sum[q][t];
+        }
+        __syncthreads();
+    }
+    if (part || !mine) return;
+    const int e = off + mr * N + nc;
+    if (grad) grad[e] = total;
+    if (ad.p) {
+        const float v = adam_step(ad, e, total);
+        const __bf16 h = (__bf16)v;
+        ((__bf16*)ad.w)[e] = h;
+        if (mr < M - 1) ((__bf16*)ad.wt)[off + nc * (M - 1) + mr] = h;
+    }
 }
 
-hipError_t launch_out_loss(const float* z3, const float* b3, const float* y, int rows, float inv_scale,
-                           void* dbf, float* err, hipStream_t s) {
-    launch_kernel(k_out_loss, dim3((rows + 255) / 256), dim3(256), 0, s, z3, b3, y, rows, inv_scale,
-                       (__bf16*)dbf, err);
-    return hipGetLastError();
-}
-
-// dz = bf16(dh * silu'(z))
-__global__ void k_silu_back(const float* __restrict__ dh, const float* __restrict__ z, long tot,
-                            __bf16* __restrict__ dzb) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= tot) return;
-    dzb[t] = (__bf16)(dh[t] * silu_grad(z[t]));
-}
-
-hipError_t launch_silu_back(const float* dh, const float* z, long tot, void* dzb, hipStream_t s) {
-    launch_kernel(k_silu_back, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, dh, z, tot,
-                       (__bf16*)dzb);
-    return hipGetLastError();
-}
-
-__global__ void k_to_bf16(const float* __restrict__ a, long tot, __bf16* __restrict__ b) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < tot) b[t] = (__bf16)a[t];
-}
-
-hipError_t launch_to_bf16(const float* a, long tot, void* b, hipStream_t s) {
-    launch_kernel(k_to_bf16, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, a, tot, (__bf16*)b);
-    return hipGetLastError();
+hipError_t launch_mlp_train_weights(const MlpTrainAct& act, long ld, int rows, const MlpAdam& adam, float* grad,
+                                    float* part, const float* err, float* loss_acc, hipStream_t s) {
+    const int chunks = (rows + kMlpChunk - 1) / kMlpChunk;
+    if (rows < 1 || ld < (long)((rows + 31) / 32) * 32) return hipErrorInvalidValue;
+    // up to kMlpFuseChunks chunks a block sums its tile alone
+    const int gy = chunks <= kMlpFuseChunks ? 1 : (chunks + kTrainWaves - 1) / kTrainWaves;
+    if (gy == 1) {
+        launch_kernel(k_mlp_train_weights, dim3(kTrainTiles + 1), dim3(64 * kTrainWaves), 0, s, act, ld, rows, adam,
+                      grad, (float*)nullptr, err, loss_acc);
+        return hipGetLastError();
+    }
+    if (!part || !grad) return hipErrorInvalidValue;
+    launch_kernel(k_mlp_train_weights, dim3(kTrainTiles, gy), dim3(64 * kTrainWaves), 0, s, act, ld, rows, MlpAdam(),
+                  (float*)nullptr, part, err, loss_acc);
+    const int off[4] = {kMlpW1, kMlpW2, kMlpW3, kMlpParams};
+    for (int l = 0; l < 3; ++l)
+        if (hipError_t e = launch_sum_partials(part + (size_t)chunks * off[l], chunks, off[l + 1] - off[l], grad + off[l], s))
+            return e;
+    if (hipError_t e = launch_sum_into(err, rows, loss_acc, s)) return e;
+    if (!adam.p) return hipSuccess;
+    launch_kernel(k_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, adam, (const float*)grad);
+    if (hipError_t e = hipGetLastError()) return e;
+    return launch_mlp_train_pack(adam.p, adam.w, adam.wt, s);
 }
 
 // xb[r][c] = bf16((x[src][c] - mu[c]) * inv_sigma[c]), src = rows ? rows[r] : r
@@ -333,41 +569,6 @@ hipError_t launch_normalize_rows(const float* x, const int* rows, long nrows, co
     const long tot = nrows * kFeat;
     launch_kernel(k_normalize_rows, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, x, rows, nrows,
                        mu, inv_sigma, (__bf16*)xb);
-    return hipGetLastError();
-}
-
-__global__ void k_gather_rows(const float* __restrict__ y, const int* __restrict__ rows, long nrows, int w,
-                              float* __restrict__ out) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nrows * w) return;
-    const long r = t / w;
-    const int c = (int)(t % w);
-    out[t] = y[(long)rows[r] * w + c];
-}
-
-hipError_t launch_gather_rows(const float* y, const int* rows, long nrows, int w, float* out, hipStream_t s) {
-    const long tot = nrows * w;
-    launch_kernel(k_gather_rows, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, y, rows, nrows, w,
-                       out);
-    return hipGetLastError();
-}
-
-// *acc += sum of v[0..n) (one block; fixed order per thread, then a tree)
-__global__ __launch_bounds__(256) void k_sum_into(const float* __restrict__ v, int n, float* __restrict__ acc) {
-    __shared__ float part[256];
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) s += v[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int d = 128; d >= 1; d >>= 1) {
-        if (threadIdx.x < d) part[threadIdx.x] += part[threadIdx.x + d];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) acc[0] += part[0];
-}
-
-hipError_t launch_sum_into(const float* v, int n, float* acc, hipStream_t s) {
-    launch_kernel(k_sum_into, dim3(1), dim3(256), 0, s, v, n, acc);
     return hipGetLastError();
 }
 
@@ -400,27 +601,6 @@ __global__ __launch_bounds__(256) void k_col_stats(const float* __restrict__ x, 
 
 hipError_t launch_col_stats(const float* x, long rows, int w, double* out, hipStream_t s) {
     launch_kernel(k_col_stats, dim3(w), dim3(256), 0, s, x, rows, w, out);
-    return hipGetLastError();
-}
-
-// Adam (Kingma & Ba, ICLR 2015) on the fp32 master parameters;
-// c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, int np, float lr, float b1, float b2, float eps, float c1,
-                       float c2) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= np) return;
-    const float gt = g[t];
-    const float mt = b1 * m[t] + (1.0f - b1) * gt;
-    const float vt = b2 * v[t] + (1.0f - b2) * gt * gt;
-    m[t] = mt;
-    v[t] = vt;
-    p[t] -= lr * (mt * c1) / (sqrtf(vt * c2) + eps);
-}
-
-hipError_t launch_adam(float* p, const float* g, float* m, float* v, int np, float lr, float b1, float b2,
-                       float eps, float c1, float c2, hipStream_t s) {
-    launch_kernel(k_adam, dim3((np + 255) / 256), dim3(256), 0, s, p, g, m, v, np, lr, b1, b2, eps, c1, c2);
     return hipGetLastError();
 }
 
