@@ -1688,9 +1688,10 @@ int lus_mlp_fit(LusMlpTrainer* t, const LusMlpFitParams* fp, float* train_loss, 
     Arena m;
     // normalisation of the inputs and scale of the targets, from the whole set
     double* st = nullptr;
-    LUS_HIP(m.alloc(&st, 2 * kFeat + 6));
-    LUS_HIP(launch_col_stats(t->feat, rows, kFeat, st, s));
-    LUS_HIP(launch_col_stats(t->tgt, rows, 3, st + 2 * kFeat, s));
+    LUS_HIP(m.alloc(&st, 2 * kFeat + 6 + col_stats_part(kFeat)));
+    double* sums = st + 2 * kFeat + 6;
+    LUS_HIP(launch_col_stats(t->feat, rows, kFeat, sums, st, s));
+    LUS_HIP(launch_col_stats(t->tgt, rows, 3, sums, st + 2 * kFeat, s));
     std::vector<double> hs(2 * kFeat + 6);
     LUS_HIP(hipStreamSynchronize(s));
     LUS_HIP(hipMemcpy(hs.data(), st, sizeof(double) * hs.size(), hipMemcpyDeviceToHost));

@@ -296,7 +296,9 @@ hipError_t launch_sum_partials(const float* part, int chunks, int MN, float* out
 hipError_t launch_normalize_rows(const float* x, const int* rows, long nrows, const float* mu,
                                  const float* inv_sigma, void* xb, hipStream_t s);
 hipError_t launch_sum_into(const float* v, int n, float* acc, hipStream_t s);
-hipError_t launch_col_stats(const float* x, long rows, int w, double* out, hipStream_t s);
+// part: col_stats_part(w) doubles of scratch
+int col_stats_part(int w);
+hipError_t launch_col_stats(const float* x, long rows, int w, double* part, double* out, hipStream_t s);
 
 // sand (simulate_sand)
 hipError_t launch_sand_predict_key(float4* x, float4* v, int* att, int n, SandK k, float dt, int* err,

@@ -192,7 +192,7 @@ hipError_t launch_mlp_forward(const void* X, int n, const float* params, const v
 // contracts them over the rows to the weights' gradients and applies Adam.
 // One launch per product and per elementwise pass (24 of 2 to 6 us each) took
 // 97 us per step of 4,096 rows, all of it launches and their tails (a fit of
-// 131,072 rows over 4 epochs: 11.7 -> 3.7 ms, the same bits).
+// 131,072 rows over 4 epochs: 11.7 -> 3.2 ms, the same bits).
 //
 // The weights are kept in bf16 twice, as stored ([fan_in][fan_out], w) and
 // transposed ([fan_out][fan_in], wt), each layer at its fp32 offset, so that
@@ -228,8 +228,9 @@ hipError_t launch_mlp_train_pack(const float* params, void* w, void* wt, hipStre
 // bf16((x - mu) inv_sigma), or bf16(x) without mu.
 //   err[r] = sum_c (o_rc - y_rc inv_scale)^2, the loss is their mean
 // kGrad: also the transposed activations and gradients t (rows past `rows` as
-// zeros, up to the grid's end).  Latency of the four layers' chain bounds it:
-// one block per CU at 4,096 rows.
+// zeros, up to the grid's end).  The latency of the chain from the row index to
+// the last layer's gradient bounds it (one block per CU at 4,096 rows): every
+// weight, bias and target is requested at the start, beside the inputs.
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 template <bool kGrad>
@@ -244,7 +245,9 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     __shared__ __attribute__((aligned(16))) __bf16 H1[16][kStride], H2[16][kStride], D[16][kStride];
     __shared__ __bf16 d3[16][4];
     __shared__ float sq[16][4];
-    const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;
+    // the wave's number is made uniform for the compiler: matrix instructions
+    // ignore the lane mask, so the conditions around them have to be branches
+    const int lane = threadIdx.x & 63, j = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int col = lane % 16, grp = lane / 16;
     const int m0 = blockIdx.x * 16;
     const int n = 16 * j + col;       // this lane's unit (C columns, B columns)
@@ -253,6 +256,28 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     bool in[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) in[i] = c0 + i < rows;
+    const bf16x8 W1 = *reinterpret_cast<const bf16x8*>(wt + kMlpW1 + n * kMlpIn + 8 * grp);
+    const float bias1 = p[kMlpB1 + n], bias2 = p[kMlpB2 + n];
+    bf16x8 W2[2], W3[2] = {}, V2[2] = {}, V3 = {};
+    float bias3 = 0.0f, y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        W2[k] = *reinterpret_cast<const bf16x8*>(wt + kMlpW2 + n * kMlpHid + 32 * k + 8 * grp);
+        if (kGrad) V2[k] = *reinterpret_cast<const bf16x8*>(w + kMlpW2 + n * kMlpHid + 32 * k + 8 * grp);
+    }
+    if (j == 0 && col < kMlpOut) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            W3[k] = *reinterpret_cast<const bf16x8*>(wt + kMlpW3 + col * kMlpHid + 32 * k + 8 * grp);
+        bias3 = p[kMlpB3 + col];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (in[i]) y[i] = tgt[(size_t)(sel ? sel[c0 + i] : c0 + i) * kMlpOut + col];
+    }
+    if (kGrad && grp == 0) {
+#pragma unroll
+        for (int c = 0; c < kMlpOut; ++c) V3[c] = w[kMlpW3 + n * kMlpOut + c];
+    }
     // layer 1
     bf16x8 a = {};
     {
@@ -271,12 +296,12 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
             for (int e = 0; e < 8; ++e) xt[(8 * grp + e) * ld + r] = a[e];
         }
     }
-    const f32x4 y1 = mfma(a, *reinterpret_cast<const bf16x8*>(wt + kMlpW1 + n * kMlpIn + 8 * grp), zero);
+    const f32x4 y1 = mfma(a, W1, zero);
     float z1[4], z2[4];
     bf16x4 h;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        z1[i] = y1[i] + p[kMlpB1 + n];
+        z1[i] = y1[i] + bias1;
         h[i] = in[i] ? (__bf16)silu(z1[i]) : (__bf16)0.0f;
         H1[4 * grp + i][n] = h[i];
     }
@@ -285,12 +310,10 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     // layer 2
     f32x4 y2 = zero;
 #pragma unroll
-    for (int k = 0; k < kMlpHid; k += 32)
-        y2 = mfma(*reinterpret_cast<const bf16x8*>(&H1[col][k + 8 * grp]),
-                  *reinterpret_cast<const bf16x8*>(wt + kMlpW2 + n * kMlpHid + k + 8 * grp), y2);
+    for (int k = 0; k < 2; ++k) y2 = mfma(*reinterpret_cast<const bf16x8*>(&H1[col][32 * k + 8 * grp]), W2[k], y2);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        z2[i] = y2[i] + p[kMlpB2 + n];
+        z2[i] = y2[i] + bias2;
         h[i] = in[i] ? (__bf16)silu(z2[i]) : (__bf16)0.0f;
         H2[4 * grp + i][n] = h[i];
     }
@@ -300,18 +323,12 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     if (j == 0) {
         f32x4 o = zero;
 #pragma unroll
-        for (int k = 0; k < kMlpHid; k += 32) {
-            bf16x8 b = {};
-            if (col < kMlpOut) b = *reinterpret_cast<const bf16x8*>(wt + kMlpW3 + col * kMlpHid + k + 8 * grp);
-            o = mfma(*reinterpret_cast<const bf16x8*>(&H2[col][k + 8 * grp]), b, o);
-        }
+        for (int k = 0; k < 2; ++k) o = mfma(*reinterpret_cast<const bf16x8*>(&H2[col][32 * k + 8 * grp]), W3[k], o);
         if (col < kMlpOut) {
             bf16x4 d;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float diff = 0.0f;
-                if (in[i])
-                    diff = (o[i] + p[kMlpB3 + col]) - tgt[(size_t)(sel ? sel[c0 + i] : c0 + i) * kMlpOut + col] * inv_scale;
+                const float diff = in[i] ? (o[i] + bias3) - y[i] * inv_scale : 0.0f;
                 d[i] = (__bf16)(2.0f * diff / (float)rows);
                 d3[4 * grp + i][col] = d[i];
                 sq[4 * grp + i][col] = diff * diff;
@@ -328,16 +345,12 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     }
     if (!kGrad) return;
     // back through layer 3: dH2 = d3 W3^T
-    bf16x8 b = {};
-    a = b;
+    bf16x8 d = {};
     if (grp == 0) {
 #pragma unroll
-        for (int c = 0; c < kMlpOut; ++c) {
-            a[c] = d3[col][c];
-            b[c] = w[kMlpW3 + n * kMlpOut + c];
-        }
+        for (int c = 0; c < kMlpOut; ++c) d[c] = d3[col][c];
     }
-    const f32x4 g2 = mfma(a, b, zero);
+    const f32x4 g2 = mfma(d, V3, zero);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         h[i] = in[i] ? (__bf16)(g2[i] * silu_grad(z2[i])) : (__bf16)0.0f;
@@ -348,9 +361,7 @@ __global__ __launch_bounds__(256) void k_mlp_train_rows(const float* __restrict_
     // layer 2: dH1 = dZ2 W2^T
     f32x4 g1 = zero;
 #pragma unroll
-    for (int k = 0; k < kMlpHid; k += 32)
-        g1 = mfma(*reinterpret_cast<const bf16x8*>(&D[col][k + 8 * grp]),
-                  *reinterpret_cast<const bf16x8*>(w + kMlpW2 + n * kMlpHid + k + 8 * grp), g1);
+    for (int k = 0; k < 2; ++k) g1 = mfma(*reinterpret_cast<const bf16x8*>(&D[col][32 * k + 8 * grp]), V2[k], g1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) h[i] = in[i] ? (__bf16)(g1[i] * silu_grad(z1[i])) : (__bf16)0.0f;
     *reinterpret_cast<bf16x4*>((__bf16*)t.dz1 + n * ld + c0) = h;
@@ -372,21 +383,21 @@ hipError_t launch_mlp_train_rows(const float* feat, const float* tgt, const int*
     return hipGetLastError();
 }
 
-// Adam (Kingma & Ba, ICLR 2015) on the fp32 master parameters; returns the
-// updated parameter
-__device__ __forceinline__ float adam_step(const MlpAdam& a, int t, float g) {
-    const float mt = a.b1 * a.m[t] + (1.0f - a.b1) * g;
-    const float vt = a.b2 * a.v[t] + (1.0f - a.b2) * g * g;
+// Adam (Kingma & Ba, ICLR 2015) on the fp32 master parameters (p0, m0, v0:
+// parameter t's state); returns the updated parameter
+__device__ __forceinline__ float adam_step(const MlpAdam& a, int t, float g, float p0, float m0, float v0) {
+    const float mt = a.b1 * m0 + (1.0f - a.b1) * g;
+    const float vt = a.b2 * v0 + (1.0f - a.b2) * g * g;
     a.m[t] = mt;
     a.v[t] = vt;
-    const float p = a.p[t] - a.lr * (mt * a.c1) / (sqrtf(vt * a.c2) + a.eps);
+    const float p = p0 - a.lr * (mt * a.c1) / (sqrtf(vt * a.c2) + a.eps);
     a.p[t] = p;
     return p;
 }
 
 __global__ void k_adam(MlpAdam a, const float* __restrict__ g) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < kMlpParams) adam_step(a, t, g[t]);
+    if (t < kMlpParams) adam_step(a, t, g[t], a.p[t], a.m[t], a.v[t]);
 }
 
 // *acc += the sum of v[0..n): 256 strided sums, then a tree (every thread of
@@ -396,6 +407,7 @@ __device__ __forceinline__ void block_sum_into(const float* __restrict__ v, int 
     const int t = (int)threadIdx.x;
     if (t < 256) {
         float s = 0.0f;
+#pragma unroll 8
         for (int i = t; i < n; i += 256) s += v[i];
         part[t] = s;
     }
@@ -470,13 +482,21 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train_weights(MlpTrain
     }
     const int tiles_n = (N + 15) / 16;
     const int m0 = (tile / tiles_n) * 16, n0 = (tile % tiles_n) * 16;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int col = lane % 16, grp = lane / 16;
     const int m = m0 + col, nn = n0 + col;
     const int chunks = (rows + kMlpChunk - 1) / kMlpChunk;
     const int t = (int)threadIdx.x;
     const int mr = m0 + t / 16, nc = n0 + t % 16;  // thread t < 256: its element of the tile
     const bool mine = t < 256 && mr < M && nc < N;
+    const int e = off + mr * N + nc;
+    // the parameter's state, requested beside the activations
+    float p0 = 0.0f, m0s = 0.0f, v0 = 0.0f;
+    if (mine && ad.p) {
+        p0 = ad.p[e];
+        m0s = ad.m[e];
+        v0 = ad.v[e];
+    }
     float total = 0.0f;
     const int g1 = (chunks + kTrainWaves - 1) / kTrainWaves;
     for (int g = blockIdx.y; g < g1; g += gridDim.y) {
@@ -484,18 +504,29 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train_weights(MlpTrain
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         if (c < chunks) {
             const int ke = rows < (c + 1) * kMlpChunk ? rows : (c + 1) * kMlpChunk;
-#pragma unroll 4
-            for (int k = c * kMlpChunk; k < ke; k += 32) {
-                bf16x8 a = {}, b = {};
-                if (m < M - 1) {
-                    a = *reinterpret_cast<const bf16x8*>(A + m * ld + k + 8 * grp);
-                } else if (m == M - 1) {
+            // a chunk's operands are all requested before the first product
+            // (a step past `ke` repeats the first one's addresses, unused)
+            constexpr int kSteps = kMlpChunk / 32;
+            bf16x8 a[kSteps], b[kSteps];
+            const long k0 = (long)c * kMlpChunk + 8 * grp;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) a[e] = (__bf16)1.0f;
-                }
-                if (nn < N) b = *reinterpret_cast<const bf16x8*>(B + nn * ld + k + 8 * grp);
-                acc = mfma(a, b, acc);
+            for (int q = 0; q < kSteps; ++q) {
+                const long k = (long)c * kMlpChunk + 32 * q < ke ? k0 + 32 * q : k0;
+                const bf16x8 fill = {};
+                a[q] = fill;
+                b[q] = fill;
+                if (m < M - 1) a[q] = *reinterpret_cast<const bf16x8*>(A + m * ld + k);
+                if (nn < N) b[q] = *reinterpret_cast<const bf16x8*>(B + nn * ld + k);
             }
+            if (m == M - 1) {
+#pragma unroll
+                for (int q = 0; q < kSteps; ++q)
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) a[q][u] = (__bf16)1.0f;
+            }
+#pragma unroll
+            for (int q = 0; q < kSteps; ++q)
+                if ((long)c * kMlpChunk + 32 * q < ke) acc = mfma(a[q], b[q], acc);
             if (part) {
                 // partials of layer 1, then 2, then 3, each [chunk][M][N]
                 const size_t base = (size_t)chunks * (off == kMlpW1 ? 0 : (off == kMlpW2 ? kMlpW2 : kMlpW3));
@@ -517,10 +548,9 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train_weights(MlpTrain
         __syncthreads();
     }
     if (part || !mine) return;
-    const int e = off + mr * N + nc;
     if (grad) grad[e] = total;
     if (ad.p) {
-        const float v = adam_step(ad, e, total);
+        const float v = adam_step(ad, e, total, p0, m0s, v0);
         const __bf16 h = (__bf16)v;
         ((__bf16*)ad.w)[e] = h;
         if (mr < M - 1) ((__bf16*)ad.wt)[off + nc * (M - 1) + mr] = h;
@@ -572,35 +602,66 @@ hipError_t launch_normalize_rows(const float* x, const int* rows, long nrows, co
     return hipGetLastError();
 }
 
-// out[2c] = sum_r x[r][c], out[2c+1] = sum_r x[r][c]^2 (float64), one block per column
-__global__ __launch_bounds__(256) void k_col_stats(const float* __restrict__ x, long rows, int w,
-                                                   double* __restrict__ out) {
-    __shared__ double s1[256], s2[256];
-    const int c = blockIdx.x;
+// Column sums in float64: out[2c] = sum_r x[r][c], out[2c+1] = sum_r x[r][c]^2.
+// Thread (q, c) sums the rows r with r % 256 = q in order (k_col_sums, whole rows
+// per wave, so the loads are contiguous), then a block per column adds the 256
+// sums by a tree: the order of one 256-thread block per column (155 us at
+// 131,072 x 32, its loads 128 bytes apart), whose bits these are.
+constexpr int kColSums = 256;
+
+__global__ __launch_bounds__(256) void k_col_sums(const float* __restrict__ x, long rows, int w,
+                                                  double* __restrict__ part) {
+    const int t = blockIdx.x * 256 + (int)threadIdx.x;
+    if (t >= kColSums * w) return;
+    const int q = t / w;
     double a = 0.0, b = 0.0;
-    for (long r = threadIdx.x; r < rows; r += 256) {
-        const double v = x[r * w + c];
+    const float* __restrict__ p = x + t;  // row q, column t % w
+    long r = q;
+    for (; r + 15 * kColSums < rows; r += 16 * kColSums, p += 16L * kColSums * w) {
+        float f[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) f[u] = p[(long)u * kColSums * w];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const double v = f[u];
+            a += v;
+            b += v * v;
+        }
+    }
+    for (; r < rows; r += kColSums, p += (long)kColSums * w) {
+        const double v = *p;
         a += v;
         b += v * v;
     }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
+    part[2 * t] = a;
+    part[2 * t + 1] = b;
+}
+
+__global__ __launch_bounds__(kColSums) void k_col_stats(const double* __restrict__ part, int w,
+                                                        double* __restrict__ out) {
+    __shared__ double s1[kColSums], s2[kColSums];
+    const int c = blockIdx.x, t = (int)threadIdx.x;
+    s1[t] = part[2 * (t * w + c)];
+    s2[t] = part[2 * (t * w + c) + 1];
     __syncthreads();
-    for (int d = 128; d >= 1; d >>= 1) {
-        if (threadIdx.x < d) {
-            s1[threadIdx.x] += s1[threadIdx.x + d];
-            s2[threadIdx.x] += s2[threadIdx.x + d];
+    for (int d = kColSums / 2; d >= 1; d >>= 1) {
+        if (t < d) {
+            s1[t] += s1[t + d];
+            s2[t] += s2[t + d];
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
+    if (t == 0) {
         out[2 * c] = s1[0];
         out[2 * c + 1] = s2[0];
     }
 }
 
-hipError_t launch_col_stats(const float* x, long rows, int w, double* out, hipStream_t s) {
-    launch_kernel(k_col_stats, dim3(w), dim3(256), 0, s, x, rows, w, out);
+int col_stats_part(int w) { return 2 * kColSums * w; }
+
+hipError_t launch_col_stats(const float* x, long rows, int w, double* part, double* out, hipStream_t s) {
+    launch_kernel(k_col_sums, dim3((kColSums * w + 255) / 256), dim3(256), 0, s, x, rows, w, part);
+    launch_kernel(k_col_stats, dim3(w), dim3(kColSums), 0, s, (const double*)part, w, out);
     return hipGetLastError();
 }
 
