@@ -1090,7 +1090,8 @@ struct MixLambdaAcc {
 // kMixed: the mixed scene's first lambda pass (phase runs, nph = 3): fluid
 // lanes sum MixLambdaAcc, sand lanes only build their lists, solid lanes
 // write an empty list (no pass reads it); the staged copy keeps w (the phase).
-template <bool kFast, bool kMixed>
+// kLambda: false for the learned step's build, which writes the lists only.
+template <bool kFast, bool kMixed, bool kLambda = true>
 __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, const int* __restrict__ key2,
                                                 const int* __restrict__ cs, int n, const PbfK& k,
                                                 float4* __restrict__ xl, int* __restrict__ maxc,
@@ -1120,6 +1121,7 @@ __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, c
     MixLambdaAcc<kFast> macc;
     ListWriter lw(ii);
     auto sum = [&](const float4 pj) {
+        if constexpr (!kLambda) return;
         if constexpr (kMixed) {
             if (ph == 0) macc.add(pi, pj, k);
         } else {
@@ -1268,11 +1270,11 @@ __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, c
             else
                 nbr_hdr(nb)[i] = make_int4(i, i, i, 0);
         } else {
-            Ci = acc.finish(pi, xl + i, k);
+            if constexpr (kLambda) Ci = acc.finish(pi, xl + i, k);
             lw.finish(i, nbr_hdr(nb), lst);
         }
     }
-    if (!kMixed) block_max_store(Ci, maxc);
+    if (!kMixed && kLambda) block_max_store(Ci, maxc);
 }
 
 // the plain scene's first lambda pass (kMixed is false)
@@ -1285,6 +1287,18 @@ __global__ __launch_bounds__(kBlock) void k_pbf_lambda_build_ws(const float4* __
                                                                  unsigned long long* __restrict__ nb,
                                                                  const int* __restrict__ gate) {
     lambda_build_ws<kFast, kMixed>(xp, key2, cs, n, k, xl, maxc, nb, gate);
+}
+
+// The lists alone, before the features pass of a learned or recorded step: 67
+// VGPRs (7 waves per SIMD) and no LDS for the features' bins.  At 1 M particles this
+// build and the features' walk of its lists take 103 + 74 us, the one pass that
+// gathers every candidate per lane 240 us.
+template <bool kFast>
+__global__ __launch_bounds__(kBlock) void k_pbf_list_build_ws(const float4* __restrict__ xp,
+                                                               const int* __restrict__ key2,
+                                                               const int* __restrict__ cs, int n, PbfK k,
+                                                               unsigned long long* __restrict__ nb) {
+    lambda_build_ws<kFast, false, false>(xp, key2, cs, n, k, nullptr, nullptr, nb, nullptr);
 }
 
 // The mixed scene's: held to 72 VGPRs (7 waves per SIMD, a few registers
@@ -2440,7 +2454,9 @@ __device__ __forceinline__ void features_body(int i, const float4* __restrict__ 
     }
 }
 
-template <bool kFast, bool kRecord>
+// kBuild: the pass builds the lists from per-lane gathers; else it walks the
+// lists of k_pbf_list_build_ws
+template <bool kFast, bool kRecord, bool kBuild>
 __global__ __launch_bounds__(kBlock) void k_pbf_features(
     int* __restrict__ key2, const int* __restrict__ cs, int n, PbfK k,
     unsigned long long* __restrict__ masks, const float4* __restrict__ xp,
@@ -2451,7 +2467,7 @@ __global__ __launch_bounds__(kBlock) void k_pbf_features(
     if (i >= n) return;
     features_body<kFast, kRecord, true>(i, xp, xold, k, mu, inv_sigma, fbf, frec, rec_stride, rec_off, inv_h,
                                   [&](auto&& f) {
-        for_each_neighbor<true>(i, n, key2, cs, masks, xp, xp, nullptr, k, f);
+        for_each_neighbor<kBuild, kWalkWide>(i, n, key2, cs, masks, xp, xp, nullptr, k, f);
     }, (lds_float4*)bins + threadIdx.x);
 }
 
@@ -2492,17 +2508,34 @@ hipError_t launch_pbf_features(int* key2, const int* cs, int n, PbfK k, unsigned
                                xp, xold, mu, inv_sigma, (bf16x8_t*)fbf, inv_h, ta.tiles, ta.ntiles, ta.lcap);
         return hipGetLastError();
     }
-    if (frec) {
-        if (rec_stride < 1) return hipErrorInvalidValue;
-        launch_kernel((k_pbf_features<false, true>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu,
-                           inv_sigma, (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);
-    } else if (k.exact) {
-        launch_kernel((k_pbf_features<false, false>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu,
-                           inv_sigma, (bf16x8_t*)fbf, frec, 1, 0, inv_h);
-    } else {
-        launch_kernel((k_pbf_features<true, false>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu,
-                           inv_sigma, (bf16x8_t*)fbf, frec, 1, 0, inv_h);
+    if (frec && rec_stride < 1) return hipErrorInvalidValue;
+    if (!frec) {
+        rec_stride = 1;
+        rec_off = 0;
     }
+    // the staged build and a walk of its lists, or (lus_pbf_set_build(0)) both
+    // in one pass of gathers
+    const bool staged = ta.stage && n > 0;
+    if (staged && k.exact)
+        launch_kernel((k_pbf_list_build_ws<false>), g, b, 0, s, xp, (const int*)key2, cs, n, k, masks);
+    else if (staged)
+        launch_kernel((k_pbf_list_build_ws<true>), g, b, 0, s, xp, (const int*)key2, cs, n, k, masks);
+#define LUS_FEAT(F, R)                                                                                              \
+    do {                                                                                                            \
+        if (staged)                                                                                                 \
+            launch_kernel((k_pbf_features<F, R, false>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu, inv_sigma, \
+                          (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                                        \
+        else                                                                                                        \
+            launch_kernel((k_pbf_features<F, R, true>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu, inv_sigma, \
+                          (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                                        \
+    } while (0)
+    if (frec)
+        LUS_FEAT(false, true);
+    else if (k.exact)
+        LUS_FEAT(false, false);
+    else
+        LUS_FEAT(true, false);
+#undef LUS_FEAT
     return hipGetLastError();
 }
 
