@@ -178,7 +178,9 @@ int lus_pbf_set_tiling(LusGpu* ctx, int tiled, int zt);
 /* List build of the flat passes (the first lambda pass of a step): staged = 1
  * (default) loads each wave's candidate ranges of a stencil row once into LDS
  * and tests them there; 0 gathers every candidate per lane from global memory.
- * Same results bit for bit.  No reference counterpart (launch configuration;
+ * With 1 large scenes (from 262,144 particles) also keep block-staged lists:
+ * the passes that walk them copy a block's neighbourhood into LDS and read the
+ * neighbours there; 2 does so at any size.  Same results bit for bit.  No reference counterpart (launch configuration;
  * the scan replaced is src/neighbors/Neighbors.cpp:306-361). */
 int lus_pbf_set_build(LusGpu* ctx, int staged);
 /* Lanes per particle in the list walks (lambda, delta-p, XSPH) of fused plain

@@ -205,7 +205,9 @@ struct PbfState {
     int lcap = 0, lcap_x = 0;  // staged float4 per array (XSPH stages two arrays)
     int nred = 0;          // block-reduction entries the last step wrote
     int fblock = lus::kBlock;  // threads per block of the flat neighbour passes
-    bool wsbuild = true;       // flat list build with wave-staged candidates
+    int build = 1;             // list build: 0 gathers, 1 staged, 2 block-staged at any size
+    int* blk = nullptr;        // block table of block-staged lists
+    bool lists_blk = false;    // the last step's lists are block-staged
     int lanes = 0;             // lanes per particle of the list walks (0: automatic)
     int sort_tile = 0;  // cells per block of the sort's prefix scan (0: by the cell count, pbf_sort_tile)
     int* scan_status = nullptr;  // two rows of the one-pass scan's tile sums (launch_scan_lookback)
@@ -454,11 +456,15 @@ int pbf_enqueue(LusGpu* c, float dt, std::vector<hipEvent_t>* ev, std::vector<in
         tx.lcap = P.lcap_x;
     }
     ta.block = tx.block = P.fblock;
-    ta.stage = P.wsbuild ? 1 : 0;
+    ta.stage = P.build ? 1 : 0;
     // small fused plain scenes: several lanes per particle in the list walks
     if (!ta.tiles && !P.mixed && !P.learned && !rec && !k.exact &&
         (P.lanes == lus::kSubLanes || (P.lanes == 0 && P.n <= lus::kSubMaxN)))
         ta.sub = tx.sub = lus::kSubLanes;
+    // block-staged lists (a walk gathers its neighbours from LDS)
+    P.lists_blk = ta.stage && !ta.tiles && !P.mixed && ta.sub == 1 && P.fblock == lus::kBlock &&
+                  (P.n >= lus::kBlkMinN || P.build == 2);
+    if (P.lists_blk) ta.blk = tx.blk = P.blk;
     // block-reduction entries the passes write
     const int nred = ta.tiles ? P.tgrid : lus::grid_for(P.n, P.fblock);
     const int K = P.p.iterations;
@@ -481,7 +487,7 @@ int pbf_enqueue(LusGpu* c, float dt, std::vector<hipEvent_t>* ev, std::vector<in
                                      P.check ? P.maxd : nullptr, s));
         LUS_HIP(mark(6));
         if (P.check) {
-            LUS_HIP(lus::launch_pbf_decide(P.maxd, lus::grid_for(P.n), std::max(P.n_fluid, 1), P.bound, 0, P.flag, P.counters,
+            LUS_HIP(lus::launch_pbf_decide(P.maxd, lus::grid_for(P.n), std::max(P.n_fluid, 1), 0, P.bound, 0, P.flag, P.counters,
                                            P.hist, LUS_DENSITY_HISTORY, s));
             LUS_HIP(mark(10));
         }
@@ -531,7 +537,7 @@ int pbf_enqueue(LusGpu* c, float dt, std::vector<hipEvent_t>* ev, std::vector<in
         LUS_HIP(lus::launch_pbf_xsph(P.xa, P.v2, P.key2, P.cs, P.n, k, P.v, P.x2, P.masks, P.xp, P.maxd,
                                      nullptr, tx, s));
         LUS_HIP(mark(6));
-        LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, P.bound, 1, P.flag, P.counters, P.hist,
+        LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, tx.blk != nullptr, P.bound, 1, P.flag, P.counters, P.hist,
                                        LUS_DENSITY_HISTORY, s));
         LUS_HIP(mark(10));
         // The plain step, run only when the decision asks for it (K >= 1).
@@ -544,7 +550,7 @@ int pbf_enqueue(LusGpu* c, float dt, std::vector<hipEvent_t>* ev, std::vector<in
         LUS_HIP(lus::launch_pbf_xsph(P.xa, P.v2, P.key2, P.cs, P.n, k, P.v, P.x2, P.masks, P.xp, P.maxd,
                                      P.flag, tx, s));
         LUS_HIP(mark(6));
-        LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, P.bound, 2, P.flag, P.counters, P.hist,
+        LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, tx.blk != nullptr, P.bound, 2, P.flag, P.counters, P.hist,
                                        LUS_DENSITY_HISTORY, s));
         LUS_HIP(mark(10));
     } else {
@@ -578,14 +584,14 @@ int pbf_enqueue(LusGpu* c, float dt, std::vector<hipEvent_t>* ev, std::vector<in
         if (keys_out) P.keys_dt = dt;
         LUS_HIP(mark(6));
         if (P.check) {
-            LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, P.bound, 0, P.flag, P.counters, P.hist,
+            LUS_HIP(lus::launch_pbf_decide(P.maxd, nred, P.n, tx.blk != nullptr, P.bound, 0, P.flag, P.counters, P.hist,
                                            LUS_DENSITY_HISTORY, s));
             LUS_HIP(mark(10));
         }
     }
     // the last lambda pass's block maxima: ta.sub lanes per particle (the
     // building pass and the list walks alike)
-    P.nred = ta.sub > 1 ? lus::grid_for(P.n * ta.sub) : nred;
+    P.nred = ta.sub > 1 ? lus::grid_for(P.n * ta.sub) : (ta.blk ? lus::grid_for(P.n, lus::kBlkT) : nred);
     std::swap(P.x, P.x2);
     std::swap(P.id, P.id2);
     std::swap(P.sid, P.sid2);
@@ -1073,6 +1079,8 @@ int pbf_setup(LusGpu* c, const LusPbfParams* p, int n, const float* pos, const f
     LUS_HIP(m.alloc(&P.xl, n));
     LUS_HIP(m.alloc(&P.xp, n));
     LUS_HIP(m.alloc(&P.masks, lus::nbr_words(n)));
+    LUS_HIP(m.alloc(&P.blk, (size_t)lus::grid_for(n, lus::kBlkT) * lus::kBlkInts));
+    P.lists_blk = false;
     LUS_HIP(m.alloc(&P.id, n));
     LUS_HIP(m.alloc(&P.id2, n));
     LUS_HIP(m.alloc(&P.key, n));
@@ -1232,10 +1240,11 @@ int lus_pbf_set_launch(LusGpu* c, int block) {
 
 int lus_pbf_set_build(LusGpu* c, int staged) {
     if (!c) return set_error(LUS_EINVAL, "lus_pbf_set_build: NULL context");
+    if (staged != 0 && staged != 2) staged = 1;
     LUS_HIP(hipSetDevice(c->device));
     LUS_HIP(hipStreamSynchronize(c->stream));
     pbf_drop_graph(c->pbf);
-    c->pbf.wsbuild = staged != 0;
+    c->pbf.build = staged;
     return LUS_OK;
 }
 
@@ -1411,7 +1420,8 @@ int lus_pbf_time_kernels(LusGpu* c, int reps, float* us) {
     // the last step's tiles still describe the current cell order
     lus::TileArgs ta, tx;
     ta.block = tx.block = P.fblock;
-    ta.stage = P.wsbuild ? 1 : 0;
+    ta.stage = P.build ? 1 : 0;
+    if (P.lists_blk) ta.blk = tx.blk = P.blk;
     if (P.tiled) {
         ta.tiles = tx.tiles = P.tl;
         ta.ntiles = tx.ntiles = P.toff + lus::tile_chunks(P.k, P.zt);
@@ -1574,7 +1584,7 @@ int lus_pbf_retest_count(LusGpu* c, long long* count) {
     LUS_HIP(hipSetDevice(c->device));
     hipStream_t s = c->stream;
     LUS_HIP(hipMemsetAsync(P.retest, 0, sizeof(int), s));
-    LUS_HIP(lus::launch_pbf_count_retest(P.masks, P.n, P.retest, s));
+    LUS_HIP(lus::launch_pbf_count_retest(P.masks, P.n, P.lists_blk ? P.blk : nullptr, P.retest, s));
     int v = 0;
     LUS_HIP(hipMemcpyAsync(&v, P.retest, sizeof(int), hipMemcpyDeviceToHost, s));
     LUS_HIP(hipStreamSynchronize(s));

@@ -124,7 +124,8 @@ hipError_t launch_gather4(const float4* src, const int* perm, int n, float4* dst
 hipError_t launch_pack3(const float4* src, const int* ids, int n, float* dst, hipStream_t s);
 // *out += particles of the neighbour-list buffer nb whose header marks the
 // re-test path (*out must be cleared by the caller)
-hipError_t launch_pbf_count_retest(const unsigned long long* nb, int n, int* out, hipStream_t s);
+// (blk: the block table of block-staged lists, nullptr for flat ones)
+hipError_t launch_pbf_count_retest(const unsigned long long* nb, int n, const int* blk, int* out, hipStream_t s);
 hipError_t launch_gather1(const int* src, const int* perm, int n, int* dst, hipStream_t s);
 hipError_t launch_stream_copy(const float4* src, float4* dst, size_t n4, hipStream_t s);
 
@@ -171,7 +172,14 @@ struct TileArgs {
     int block = kBlock;           // threads per block of a flat launch (64, 128 or 256)
     int stage = 1;                // flat list build: wave-staged candidates (0: per-lane gathers)
     int sub = 1;                  // lanes per particle of the list walks (small fused scenes: kSubLanes)
+    int* blk = nullptr;           // block table of block-staged lists (lus_pbf.hip), nullptr: flat lists
 };
+// Block-staged lists (lus_pbf.hip): threads (and slots) per block, ints per
+// block-table entry, and the particles from which plain, learned and recorded steps
+// use them: two blocks per CU, which is what runs at once.
+constexpr int kBlkT = 512;
+constexpr int kBlkInts = 32;
+constexpr int kBlkMinN = 2 * 256 * kBlkT;
 // A fused plain scene of at most kSubMaxN particles walks its lists with
 // kSubLanes lanes per particle (lus_pbf.hip, "Small scenes").
 constexpr int kSubLanes = 4;
@@ -252,7 +260,8 @@ hipError_t launch_pbf_record_target(const float4* xa, const float4* xp, int n, i
 // reduce the XSPH block maxima and sums (maxd: 2 * nblk): e = max(0, max C),
 // hist[step % cap] = e, hist[cap + step % cap] = mean_i max(0, C_i);
 // flag = learned && !(e <= bound); counters[0] += 1, counters[1] += flag
-hipError_t launch_pbf_decide(const int* maxd, int nblk, int n, float bound, int learned, int* flag,
+// (waves: maxd holds one value per wave, as the block-staged XSPH pass writes them)
+hipError_t launch_pbf_decide(const int* maxd, int nblk, int n, int waves, float bound, int learned, int* flag,
                              int* counters, float* hist, int cap, hipStream_t s);
 
 // MLP 32 -> 64 (SiLU) -> 64 (SiLU) -> 3, parameters (fp32) in this order:

@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <type_traits>
 
 #include "lus_device.hpp"
 #include "lus_internal.hpp"
@@ -57,6 +58,19 @@ hipError_t launch_xsph_sub(const float4* xa, const float4* vt, int* key2, const 
                            float4* vout, float4* xout, unsigned long long* masks, const float4* xp,
                            const int* gate, hipStream_t s,
                            const NextKeys& nk);
+
+// the block-staged passes, defined below
+static hipError_t launch_build_blk(const float4* xp, const int* key2, const int* cs, int n, const PbfK& k, float4* xl,
+                                   int* maxc, unsigned long long* nb, const int* gate, int* blk, hipStream_t s);
+static hipError_t launch_lambda_blk(const float4* xa, const int* key2, const int* cs, int n, const PbfK& k, float4* xl,
+                                    int* maxc, unsigned long long* nb, const float4* xp, const int* gate, const int* blk,
+                                    hipStream_t s);
+static hipError_t launch_deltap_blk(const float4* xl, const int* key2, const int* cs, int n, const PbfK& k, float4* xa,
+                                    const float4* xold, float4* vout, float dt, unsigned long long* nb,
+                                    const float4* xp, const int* gate, const int* blk, hipStream_t s);
+static hipError_t launch_xsph_blk(const float4* xa, const float4* vt, const int* key2, const int* cs, int n,
+                                  const PbfK& k, float4* vout, float4* xout, unsigned long long* nb, const float4* xp,
+                                  int* maxd, const int* gate, const NextKeys& nk, const int* blk, hipStream_t s);
 
 // clamp box and cell y offset of a particle: the scene table entry of a batch,
 // or the single scene's bounds
@@ -282,6 +296,44 @@ struct ListWriter {
     }
 };
 
+// neighbour counts of a staged block's particles
+__device__ __forceinline__ int* blk_counts(unsigned long long* nb, int tile) {
+    return reinterpret_cast<int*>(nbr_hdr(nb) + (size_t)tile * kBlkT);
+}
+
+// Places of a block-staged list being built: entry = slot + shift, the row's
+// place - slot (ListWriter's interface; no layers)
+struct BlkWriter {
+    int c = 0, shift = 0;
+    unsigned int q0 = 0u, q1 = 0u, q2 = 0u, q3 = 0u;
+    __device__ __forceinline__ explicit BlkWriter(int) {}
+    __device__ __forceinline__ void push(unsigned int e) {
+        q0 = (q0 >> 16) | (q1 << 16);
+        q1 = (q1 >> 16) | (q2 << 16);
+        q2 = (q2 >> 16) | (q3 << 16);
+        q3 = (q3 >> 16) | (e << 16);
+    }
+    __device__ __forceinline__ void row_hits(int, int) {}
+    __device__ __forceinline__ bool append_row(int j) {
+        push((unsigned int)(j + shift));
+        ++c;
+        return (c & 7) == 0 && c <= kNbrCap;
+    }
+    __device__ __forceinline__ int4 group() const { return make_int4((int)q0, (int)q1, (int)q2, (int)q3); }
+    __device__ __forceinline__ void emit(int j, int4* __restrict__ lst) {
+        if (append_row(j)) lst[(size_t)((c >> 3) - 1) * 64] = group();
+    }
+    // the last, partial group (place 0 in the unused entries: read by a walk, not visited)
+    __device__ __forceinline__ void finish(int* __restrict__ count, int4* __restrict__ lst) {
+        const int rem = c & 7;
+        if (rem != 0 && c < kNbrCap) {
+            for (int u = rem; u < 8; ++u) push(0u);
+            lst[(size_t)(c >> 3) * 64] = group();
+        }
+        *count = c > kNbrCap ? kNbrRetest : c;
+    }
+};
+
 // Test the 27-cell candidates of slot i (positions xp) row by row, in
 // ascending slot order -- a row of at most 64 slots through a 64-bit hit mask
 // (32-bit mask arithmetic when no lane of the wave has a hit above bit 31), a
@@ -444,6 +496,32 @@ __device__ __forceinline__ void visit_list(const int4 hd, const int4* __restrict
     }
 }
 
+// N(i) of a particle without a list: its candidates tested again against the
+// stored predicted positions xp (the same set in the same order)
+template <class F>
+__device__ __forceinline__ void retest_neighbors(int i, const int* __restrict__ key2, const int* __restrict__ cs,
+                                                 const float4* __restrict__ xp, const float4* __restrict__ cur,
+                                                 const float4* __restrict__ aux, const PbfK& k, F& f) {
+    int cy, cx, cz;
+    key_cell(key2[i] & ~kOvf, k, cy, cx, cz);
+    const int z0 = cz > 0 ? cz - 1 : 0;
+    const int z1 = cz + 1 < k.gZ ? cz + 1 : k.gZ - 1;
+    const float4 pi = xp[i];
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+        const int y = cy + r / 3 - 1;
+        const int x = cx + r % 3 - 1;
+        if (y < 0 || y >= k.gY || x < 0 || x >= k.gX) continue;
+        for (int c = 0; c < k.nph; ++c) {
+            const int row = row_key(y, x, c, k);
+            const int j0 = cs[row + z0];
+            const int j1 = cs[row + z1 + 1];
+            for (int j = j0; j < j1; ++j)
+                if (within_h_k(pi, xp[j], k)) f(j, cur[j], aux_at(aux, j));
+        }
+    }
+}
+
 // Visit N(i) in ascending slot order, calling f(j, cur[j], aux[j]).  build:
 // test the candidates, visiting and listing the hits (build_list); otherwise
 // walk the stored list.  A particle whose list overflowed re-tests its candidates
@@ -467,24 +545,7 @@ __device__ __forceinline__ void for_each_neighbor(int i, int n, int* __restrict_
         visit_list<kWalk>(hd, lst, cur, aux, f);
         return;
     }
-    int cy, cx, cz;
-    key_cell(key2[i] & ~kOvf, k, cy, cx, cz);
-    const int z0 = cz > 0 ? cz - 1 : 0;
-    const int z1 = cz + 1 < k.gZ ? cz + 1 : k.gZ - 1;
-    const float4 pi = xp[i];
-#pragma unroll 1
-    for (int r = 0; r < 9; ++r) {
-        const int y = cy + r / 3 - 1;
-        const int x = cx + r % 3 - 1;
-        if (y < 0 || y >= k.gY || x < 0 || x >= k.gX) continue;
-        for (int c = 0; c < k.nph; ++c) {
-            const int row = row_key(y, x, c, k);
-            const int j0 = cs[row + z0];
-            const int j1 = cs[row + z1 + 1];
-            for (int j = j0; j < j1; ++j)
-                if (within_h_k(pi, xp[j], k)) f(j, cur[j], aux_at(aux, j));
-        }
-    }
+    retest_neighbors(i, key2, cs, xp, cur, aux, k, f);
 }
 
 // ---------------------------------------------------------------------------
@@ -825,7 +886,7 @@ __device__ __forceinline__ float poly_t(float r2, const PbfK& k) {  // hf^2 - f^
 // reduces the few thousand block values when it needs them.  Every thread of
 // the block must call it.
 __device__ __forceinline__ void block_max_store(float c, int* __restrict__ out) {
-    __shared__ int wmax[kBlock / 64];
+    __shared__ int wmax[kBlkT / 64];
     int m = ordered(c);
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -942,9 +1003,8 @@ struct LambdaAcc {
 };
 
 template <bool kFast, class Visit>
-__device__ __forceinline__ float lambda_body(int i, const float4* __restrict__ xa, float4* __restrict__ xl,
-                                             const PbfK& k, Visit&& visit) {
-    const float4 pi = xa[i];
+__device__ __forceinline__ float lambda_body(int i, const float4 pi, float4* __restrict__ xl, const PbfK& k,
+                                             Visit&& visit) {
     LambdaAcc<kFast> s(k);
     visit([&](int, const float4 pj, const float4) { s.add(pi, pj, k); });
     return s.finish(pi, xl + i, k);
@@ -963,7 +1023,7 @@ __global__ __launch_bounds__(kBlock) void k_pbf_lambda(const float4* __restrict_
     const int i = xcd_index();
     float Ci = -1e30f;
     if (i < n)
-        Ci = lambda_body<kFast>(i, xa, xl, k, [&](auto&& f) {
+        Ci = lambda_body<kFast>(i, xa[i], xl, k, [&](auto&& f) {
             for_each_neighbor<kBuild, kWalkWide>(i, n, key2, cs, masks, xp, xa, nullptr, k, f);
         });
     block_max_store(Ci, maxc);
@@ -1091,20 +1151,22 @@ struct MixLambdaAcc {
 // lanes sum MixLambdaAcc, sand lanes only build their lists, solid lanes
 // write an empty list (no pass reads it); the staged copy keeps w (the phase).
 // kLambda: false for the learned step's build, which writes the lists only.
-template <bool kFast, bool kMixed, bool kLambda = true>
-__device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, const int* __restrict__ key2,
-                                                const int* __restrict__ cs, int n, const PbfK& k,
-                                                float4* __restrict__ xl, int* __restrict__ maxc,
-                                                unsigned long long* __restrict__ nb, const int* __restrict__ gate) {
+// kBlk: the lists of a staged block (entries are places, tb its table entry).
+// S: the wave's staging, kStageCap slots; returns C_i.
+template <bool kMixed>
+constexpr int kStageFloats = (kMixed ? 4 : 3) * kStageCap;
+
+template <bool kFast, bool kMixed, bool kLambda = true, bool kBlk = false>
+__device__ __forceinline__ float lambda_build_ws(const float4* __restrict__ xp, const int* __restrict__ key2,
+                                                 const int* __restrict__ cs, int n, const PbfK& k,
+                                                 float4* __restrict__ xl, unsigned long long* __restrict__ nb,
+                                                 lds_float* __restrict__ S, const int* tb = nullptr) {
     constexpr int kS = kMixed ? 4 : 3;  // floats per staged slot
     // runs per wave staged (a mixed wave holds a column's fluid, sand and
     // solid runs, so more of them)
     constexpr int kSegs = kMixed ? 2 * kStageSegs : kStageSegs;
-    if (gate && *gate == 0) return;  // uniform: before any barrier
-    __shared__ float stage[kBlock / 64][kS * kStageCap];
     const int i = xcd_index();
     const int lane = (int)(threadIdx.x & 63);
-    lds_float* __restrict__ S = (lds_float*)stage[threadIdx.x >> 6];
     // every lane of the wave takes part in the staging; a lane past n
     // (i >= n, the last wave only) has empty windows and stores nothing
     const bool act = i < n;
@@ -1119,7 +1181,7 @@ __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, c
     int4* __restrict__ lst = nbr_list(nb, n, ii);
     LambdaAcc<kFast, false> acc(k);
     MixLambdaAcc<kFast> macc;
-    ListWriter lw(ii);
+    std::conditional_t<kBlk, BlkWriter, ListWriter> lw(ii);
     auto sum = [&](const float4 pj) {
         if constexpr (!kLambda) return;
         if constexpr (kMixed) {
@@ -1140,7 +1202,10 @@ __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, c
     const unsigned long long below = (1ull << lane) - 1ull;  // lanes before this one
 #pragma unroll 1
     for (int r = 0; r < 9; ++r) {
-        lw.row(r, ii);
+        if constexpr (kBlk)
+            lw.shift = __builtin_amdgcn_readfirstlane(tb[r]);
+        else
+            lw.row(r, ii);
         const int y = cy + r / 3 - 1;
         const int x = cx + r % 3 - 1;
         const bool valid = lists && y >= 0 && y < k.gY && x >= 0 && x < k.gX;
@@ -1271,10 +1336,13 @@ __device__ __forceinline__ void lambda_build_ws(const float4* __restrict__ xp, c
                 nbr_hdr(nb)[i] = make_int4(i, i, i, 0);
         } else {
             if constexpr (kLambda) Ci = acc.finish(pi, xl + i, k);
-            lw.finish(i, nbr_hdr(nb), lst);
+            if constexpr (kBlk)
+                lw.finish(blk_counts(nb, i / kBlkT) + i % kBlkT, lst);
+            else
+                lw.finish(i, nbr_hdr(nb), lst);
         }
     }
-    if (!kMixed && kLambda) block_max_store(Ci, maxc);
+    return Ci;
 }
 
 // the plain scene's first lambda pass (kMixed is false)
@@ -1286,7 +1354,10 @@ __global__ __launch_bounds__(kBlock) void k_pbf_lambda_build_ws(const float4* __
                                                                  int* __restrict__ maxc,
                                                                  unsigned long long* __restrict__ nb,
                                                                  const int* __restrict__ gate) {
-    lambda_build_ws<kFast, kMixed>(xp, key2, cs, n, k, xl, maxc, nb, gate);
+    if (gate && *gate == 0) return;  // uniform: before any barrier
+    __shared__ float stage[kBlock / 64][kStageFloats<kMixed>];
+    const float Ci = lambda_build_ws<kFast, kMixed>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
+    block_max_store(Ci, maxc);
 }
 
 // The lists alone, before the features pass of a learned or recorded step: 67
@@ -1298,7 +1369,8 @@ __global__ __launch_bounds__(kBlock) void k_pbf_list_build_ws(const float4* __re
                                                                const int* __restrict__ key2,
                                                                const int* __restrict__ cs, int n, PbfK k,
                                                                unsigned long long* __restrict__ nb) {
-    lambda_build_ws<kFast, false, false>(xp, key2, cs, n, k, nullptr, nullptr, nb, nullptr);
+    __shared__ float stage[kBlock / 64][kStageFloats<false>];
+    lambda_build_ws<kFast, false, false>(xp, key2, cs, n, k, nullptr, nb, (lds_float*)stage[threadIdx.x >> 6]);
 }
 
 // The mixed scene's: held to 72 VGPRs (7 waves per SIMD, a few registers
@@ -1309,7 +1381,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) 
     const float4* __restrict__ xp, const int* __restrict__ key2, const int* __restrict__ cs, int n, PbfK k,
     float4* __restrict__ xl, int* __restrict__ maxc, unsigned long long* __restrict__ nb,
     const int* __restrict__ gate) {
-    lambda_build_ws<kFast, true>(xp, key2, cs, n, k, xl, maxc, nb, gate);
+    __shared__ float stage[kBlock / 64][kStageFloats<true>];
+    lambda_build_ws<kFast, true>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
 }
 
 template <bool kBuild, bool kFast>
@@ -1332,7 +1405,7 @@ __global__ __launch_bounds__(kTileT) void k_pbf_lambda_t(const float4* __restric
         tile_stage(S, tiles[t], cs, k, xa, nullptr, lds, nullptr, lcap);
         const int i = S.i0 + (int)threadIdx.x;
         if (i < S.i1) {
-            const float c = lambda_body<kFast>(i, xa, xl, k, [&](auto&& f) {
+            const float c = lambda_body<kFast>(i, xa[i], xl, k, [&](auto&& f) {
                 for_each_neighbor_tiled<kBuild>(S, i, n, key2, masks, xp, xa, nullptr, lds, nullptr, k, f);
             });
             cmax = c > cmax ? c : cmax;
@@ -1366,6 +1439,8 @@ hipError_t launch_pbf_lambda(const float4* xa, int* key2, const int* cs, int n, 
     if (!build && ta.sub > 1 && !k.exact) return launch_lambda_sub(xa, key2, cs, n, k, xl, maxc, masks, xp, gate, s);
     if (build && ta.sub > 1 && !k.exact && xa == xp && k.nph == 1 && n > 0)
         return launch_lambda_build_sub(xp, key2, cs, n, k, xl, maxc, masks, gate, s);
+    if (ta.blk && build) return launch_build_blk(xp, key2, cs, n, k, xl, maxc, masks, gate, ta.blk, s);
+    if (ta.blk) return launch_lambda_blk(xa, key2, cs, n, k, xl, maxc, masks, xp, gate, ta.blk, s);
     const dim3 g(grid_for(n, ta.block)), b(ta.block);
     if (build && ta.stage && xa == xp && n > 0 && k.nph == 1) {
         if (k.exact)
@@ -1472,10 +1547,9 @@ __device__ __forceinline__ void deltap_commit(int i, const float4 pi, float ax, 
 
 // delta-p pass: the sums of DeltapAcc, Jacobi update, box clamp
 template <bool kFast, int kNS, class Visit>
-__device__ __forceinline__ void deltap_body(int i, const float4* __restrict__ xl, const PbfK& k,
-                                            float4* __restrict__ xa, const float4* __restrict__ xold,
-                                            float4* __restrict__ vout, float dt, Visit&& visit) {
-    const float4 pi = xl[i];
+__device__ __forceinline__ void deltap_body(int i, const float4 pi, const PbfK& k, float4* __restrict__ xa,
+                                            const float4* __restrict__ xold, float4* __restrict__ vout, float dt,
+                                            Visit&& visit) {
     const float li = pi.w;
     DeltapAcc<kFast, kNS> d(k);
     visit([&](int, const float4 pj, const float4) { d.add(pi, li, pj, k); });
@@ -1495,7 +1569,7 @@ __global__ __launch_bounds__(kBlock) void k_pbf_deltap(const float4* __restrict_
     if (gate && *gate == 0) return;
     const int i = xcd_index();
     if (i >= n) return;
-    deltap_body<kFast, kNS>(i, xl, k, xa, xold, vout, dt, [&](auto&& f) {
+    deltap_body<kFast, kNS>(i, xl[i], k, xa, xold, vout, dt, [&](auto&& f) {
         for_each_neighbor<false, kWalkWide>(i, n, key2, cs, masks, xp, xl, nullptr, k, f);
     });
 }
@@ -1520,7 +1594,7 @@ __global__ __launch_bounds__(kTileT) void k_pbf_deltap_t(const float4* __restric
         tile_stage(S, tiles[t], cs, k, xl, nullptr, lds, nullptr, lcap);
         const int i = S.i0 + (int)threadIdx.x;
         if (i < S.i1)
-            deltap_body<kFast, kNS>(i, xl, k, xa, xold, vout, dt, [&](auto&& f) {
+            deltap_body<kFast, kNS>(i, xl[i], k, xa, xold, vout, dt, [&](auto&& f) {
                 for_each_neighbor_tiled<false>(S, i, n, key2, masks, xp, xl, nullptr, lds, nullptr, k, f);
             });
         __syncthreads();
@@ -1549,6 +1623,7 @@ hipError_t launch_pbf_deltap(const float4* xl, int* key2, const int* cs, int n, 
         return hipGetLastError();
     }
     if (ta.sub > 1 && !k.exact) return launch_deltap_sub(xl, key2, cs, n, k, xa, xold, vout, dt, masks, xp, gate, s);
+    if (ta.blk) return launch_deltap_blk(xl, key2, cs, n, k, xa, xold, vout, dt, masks, xp, gate, ta.blk, s);
     const dim3 g(grid_for(n, ta.block)), b(ta.block);
     if (k.exact && n4)
         launch_kernel((k_pbf_deltap<false, 4>), g, b, 0, s, xl, key2, cs, n, k, xa, xold, vout, dt, masks, xp, gate);
@@ -1582,11 +1657,9 @@ hipError_t launch_pbf_velocity(const float4* xa, const float4* xold, int n, floa
 // maximum goes to maxd (the learned step's fallback test and the density
 // error statistics).
 template <bool kFast, bool kCheck, class Visit>
-__device__ __forceinline__ float xsph_body(int i, const float4* __restrict__ xa, const float4* __restrict__ vt,
-                                           const PbfK& k, float4* __restrict__ vout, float4* __restrict__ xout,
-                                           Visit&& visit, float4* xn = nullptr, float4* vn = nullptr) {
-    const float4 pi = xa[i];
-    const float4 vi = vt[i];
+__device__ __forceinline__ float xsph_body(int i, const float4 pi, const float4 vi, const PbfK& k,
+                                           float4* __restrict__ vout, float4* __restrict__ xout, Visit&& visit,
+                                           float4* xn = nullptr, float4* vn = nullptr) {
     float sx = 0.0f, sy = 0.0f, sz = 0.0f, rho = 0.0f;
     visit([&](int, const float4 pj, const float4 vj) {
         const float dx = pi.x - pj.x;
@@ -1646,7 +1719,7 @@ __global__ __launch_bounds__(kBlock) void k_pbf_xsph(const float4* __restrict__ 
     float Ci = -1e30f;
     float4 xn = make_float4(0.0f, 0.0f, 0.0f, 0.0f), vn = xn;
     if (i < n)
-        Ci = xsph_body<kFast, kCheck>(i, xa, vt, k, vout, xout, [&](auto&& f) {
+        Ci = xsph_body<kFast, kCheck>(i, xa[i], vt[i], k, vout, xout, [&](auto&& f) {
             for_each_neighbor<false, kWalkPairs>(i, n, key2, cs, masks, xp, xa, vt, k, f);
         }, &xn, &vn);
     if (nk.key) next_key(i, i < n, xn, vn, k, nk);
@@ -1675,7 +1748,7 @@ __global__ __launch_bounds__(kTileT) void k_pbf_xsph_t(const float4* __restrict_
         tile_stage(S, tiles[t], cs, k, xa, vt, lds, lds + lcap, lcap);
         const int i = S.i0 + (int)threadIdx.x;
         if (i < S.i1) {
-            const float c = xsph_body<kFast, kCheck>(i, xa, vt, k, vout, xout, [&](auto&& f) {
+            const float c = xsph_body<kFast, kCheck>(i, xa[i], vt[i], k, vout, xout, [&](auto&& f) {
                 for_each_neighbor_tiled<false>(S, i, n, key2, masks, xp, xa, vt, lds, lds + lcap, k, f);
             });
             cmax = c > cmax ? c : cmax;
@@ -1684,6 +1757,355 @@ __global__ __launch_bounds__(kTileT) void k_pbf_xsph_t(const float4* __restrict_
         __syncthreads();
     }
     if (kCheck) block_max_sum_store(cmax, csum, maxd);
+}
+
+// ---------------------------------------------------------------------------
+// Block-staged lists (large scenes).  A walk that gathers each neighbour from
+// global memory is bound by the L1's tag lookups, about 48 per 64-lane gather of
+// 16 bytes, and past the last-level cache by its misses.  So a block of kBlkT
+// consecutive slots copies the nine slot ranges that its particles' stencil
+// rows can reach into LDS, once per pass, coalesced, and its list entries are
+// places in that copy (a walk decodes nothing).  The ranges follow from the block's first and last
+// key: keys ascend with the slot, so row (dy, dx) of every particle lies within
+// cells [first + o - 1, last + o + 1], o = (dy gX + dx) gZ.  A block whose ranges
+// exceed kBlkCap slots (2 to 11 % of them on the dam breaks) keeps flat lists and
+// gathers.  The XSPH pass keeps a place's slot in w of the copy and gathers the
+// velocity from it: two copies would leave one block per CU (105 us at 1 M
+// against 68).
+//
+// Two blocks of 81 KB per CU run at once, 4 waves per SIMD.  With 256 slots per
+// block the copy is 10 instead of 9 slots per slot and a third of the blocks do not fit
+// when the fluid is compressed; 320 and 384 leave the SIMDs unequal (60 to
+// 90 us).  Measured at 1 M / 4 M / the 64-scene batch, us per launch, flat lists then
+// these: lambda 48 -> 47, 233 -> 198, 226 -> 170; delta-p 51 -> 45, 249 -> 191,
+// 244 -> 172; XSPH 99 -> 68, 523 -> 333, 479 -> 290; the build 145 -> 147, 491 -> 483,
+// 493 -> 505.  At 106 K particles (208 blocks) nothing is gained, so scenes
+// below kBlkMinN keep flat lists.
+//
+// Rows of one layer overlap when the block spans several columns; the shared
+// slots are copied once.
+//
+// Block table, kBlkInts ints per block; per stencil row r: [r] place - slot of
+// its range, [9 + r] first slot to copy, [18 + r] slots to copy; [27] 1 if the
+// block is staged.  Staged blocks keep their particles' neighbour counts (or
+// kNbrRetest) as ints at the start of the block's headers.
+//
+// Same candidates, same order, same arithmetic as the flat passes: the same bits.
+// ---------------------------------------------------------------------------
+constexpr int kBlkCap = 5110;
+constexpr int kBlkStaged = 27;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) f32x4_t lds_f32x4;
+
+__device__ __forceinline__ float4 lds4(const lds_f32x4* __restrict__ S, unsigned int e) {
+    const f32x4_t v = S[e];
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+__device__ __forceinline__ int blk_tile() {
+    const int G = gridDim.x, b = blockIdx.x;
+    return (b % kXcd) * (G / kXcd) + b / kXcd;
+}
+
+// The block's table entry into tb (LDS) and blk; ends with a barrier
+__device__ __forceinline__ void blk_table(int tile, const int* __restrict__ key2, const int* __restrict__ cs, int n,
+                                          const PbfK& k, int* tb, int* __restrict__ blk) {
+    const int tid = (int)threadIdx.x;
+    const int s0 = tile * kBlkT, s1 = s0 + kBlkT < n ? s0 + kBlkT : n;
+    if (tid < 18) {
+        const int r = tid % 9, o = (r / 3 - 1) * k.gXZ + (r % 3 - 1) * k.gZ;
+        const int C = k.gXZ * k.gY;
+        int c = tid >= 9 ? (key2[s1 - 1] & ~kOvf) + o + 2 : (key2[s0] & ~kOvf) + o - 1;
+        c = c < 0 ? 0 : (c > C ? C : c);
+        tb[tid] = cs[c];
+    }
+    __syncthreads();
+    if (tid == 0) {
+        int acc = 0;
+        for (int L = 0; L < 9; L += 3) {
+            int end = 0;  // of the layer's copied slots (rows ascend)
+            for (int r = L; r < L + 3; ++r) {
+                const int a = tb[r], e = tb[9 + r];
+                const int from = r > L && a < end ? (end < e ? end : e) : a;
+                // rows that overlap share their places
+                tb[r] = r > L && a <= end ? tb[r - 1] : acc - a;
+                tb[9 + r] = from;
+                tb[18 + r] = e - from;
+                acc += e - from;
+                end = e > end ? e : end;
+            }
+        }
+        tb[kBlkStaged] = acc <= kBlkCap ? 1 : 0;
+    }
+    __syncthreads();
+    if (tid <= kBlkStaged) blk[(size_t)tile * kBlkInts + tid] = tb[tid];
+}
+
+// put(place, src[slot], slot) for the block's ranges (bt: its table entry); the
+// caller waits for the block
+template <class F>
+__device__ __forceinline__ void blk_copy(const int* __restrict__ bt, const float4* __restrict__ src, F&& put) {
+    const int tid = (int)threadIdx.x;
+    float4 v[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r)
+        if (tid < bt[18 + r]) v[r] = at4(src, bt[9 + r] + tid);
+#pragma unroll
+    for (int r = 0; r < 9; ++r)
+        if (tid < bt[18 + r]) put(bt[9 + r] + tid + bt[r], v[r], bt[9 + r] + tid);
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r)
+        for (int q = tid + kBlkT; q < bt[18 + r]; q += kBlkT)
+            put(bt[9 + r] + q + bt[r], at4(src, bt[9 + r] + q), bt[9 + r] + q);
+}
+
+// Walk the c (<= kNbrCap) entries of a block-staged list, calling f(e, p, a)
+// with p, a = get(e) in list order, eight reads in flight
+template <class G, class F>
+__device__ __forceinline__ void visit_list_blk(int c, int4 g, const int4* __restrict__ lst, G& get, F& f) {
+    if (c <= 0) return;
+    for (int t = 0; t < c; t += 8) {
+        const unsigned int w[4] = {(unsigned int)g.x, (unsigned int)g.y, (unsigned int)g.z, (unsigned int)g.w};
+        unsigned int e[8];
+        float4 p[8], a[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            e[u] = (u & 1) ? w[u >> 1] >> 16 : w[u >> 1] & 0xFFFFu;
+            get(e[u], p[u], a[u]);
+        }
+        const int gi = (t >> 3) + 1 < kNbrGroups ? (t >> 3) + 1 : kNbrGroups - 1;
+        g = lst[(size_t)gi * 64];
+        f((int)e[0], p[0], a[0]);
+#pragma unroll
+        for (int u = 1; u < 8; ++u)
+            if (t + u < c) f((int)e[u], p[u], a[u]);
+    }
+}
+
+// A particle's list as the pass begins: its header (count; flat: the layers
+// too) and first group, requested before the block waits for its copy
+struct BlkList {
+    const int4* __restrict__ lst;
+    int4 hd, g;
+    __device__ __forceinline__ BlkList(int i, int n, int tile, bool staged, unsigned long long* __restrict__ nb)
+        : lst(nbr_list(nb, n, i)) {
+        if (staged)
+            hd = make_int4(0, 0, 0, blk_counts(nb, tile)[threadIdx.x]);
+        else
+            hd = nbr_hdr(nb)[i];
+        g = lst[0];
+    }
+};
+
+// N(i): the staged copy's list (get), or the flat forms
+template <int kWalk, class G, class F>
+__device__ __forceinline__ void for_each_neighbor_blk(int i, const BlkList& l, bool staged,
+                                                      const int* __restrict__ key2, const int* __restrict__ cs,
+                                                      const float4* __restrict__ xp, const float4* __restrict__ cur,
+                                                      const float4* __restrict__ aux, const PbfK& k, G&& get, F&& f) {
+    if ((l.hd.w & 0xFFFF) > kNbrCap)
+        retest_neighbors(i, key2, cs, xp, cur, aux, k, f);
+    else if (staged)
+        visit_list_blk(l.hd.w, l.g, l.lst, get, f);
+    else
+        visit_list<kWalk>(l.hd, l.lst, cur, aux, f);
+}
+
+// The step's first pass: block table, lists and (kLambda) lambda, wave-staged
+// as the flat build; a staged block's entries are places in its copy.
+template <bool kFast, bool kLambda>
+__global__ __launch_bounds__(kBlkT) void k_pbf_build_blk(const float4* __restrict__ xp, const int* __restrict__ key2,
+                                                         const int* __restrict__ cs, int n, PbfK k,
+                                                         float4* __restrict__ xl, int* __restrict__ maxc,
+                                                         unsigned long long* __restrict__ nb,
+                                                         const int* __restrict__ gate, int* __restrict__ blk) {
+    if (gate && *gate == 0) return;  // uniform: before any barrier
+    __shared__ float stage[kBlkT / 64][kStageFloats<false>];
+    __shared__ int tb[kBlkInts];
+    const int tile = blk_tile();
+    float Ci = -1e30f;
+    if (tile * kBlkT < n) {
+        blk_table(tile, key2, cs, n, k, tb, blk);
+        lds_float* __restrict__ S = (lds_float*)stage[threadIdx.x >> 6];
+        if (tb[kBlkStaged])  // uniform
+            Ci = lambda_build_ws<kFast, false, kLambda, true>(xp, key2, cs, n, k, xl, nb, S, tb);
+        else
+            Ci = lambda_build_ws<kFast, false, kLambda>(xp, key2, cs, n, k, xl, nb, S);
+    }
+    if constexpr (kLambda) block_max_store(Ci, maxc);
+}
+
+template <bool kFast>
+__global__ __launch_bounds__(kBlkT) void k_pbf_lambda_blk(const float4* __restrict__ xa, const int* __restrict__ key2,
+                                                          const int* __restrict__ cs, int n, PbfK k,
+                                                          float4* __restrict__ xl, int* __restrict__ maxc,
+                                                          unsigned long long* __restrict__ nb,
+                                                          const float4* __restrict__ xp, const int* __restrict__ gate,
+                                                          const int* __restrict__ blk) {
+    if (gate && *gate == 0) return;  // uniform: before any barrier
+    __shared__ float4 copy[kBlkCap];
+    lds_f32x4* __restrict__ S = (lds_f32x4*)copy;
+    const int tile = blk_tile();
+    const int i = tile * kBlkT + (int)threadIdx.x;
+    float Ci = -1e30f;
+    if (tile * kBlkT < n) {
+        const int* __restrict__ bt = blk + (size_t)tile * kBlkInts;
+        const bool staged = bt[kBlkStaged] != 0;
+        const int ii = i < n ? i : n - 1;
+        const float4 pi = xa[ii];
+        const BlkList l(ii, n, tile, staged, nb);
+        if (staged) {
+            blk_copy(bt, xa, [&](int e, const float4 v, int) { S[e] = f32x4_t{v.x, v.y, v.z, 0.0f}; });
+            __syncthreads();
+        }
+        auto get = [&](unsigned int e, float4& p, float4&) { p = lds4(S, e); };
+        if (i < n)
+            Ci = lambda_body<kFast>(i, pi, xl, k, [&](auto&& f) {
+                for_each_neighbor_blk<kWalkWide>(i, l, staged, key2, cs, xp, xa, nullptr, k, get, f);
+            });
+    }
+    block_max_store(Ci, maxc);
+}
+
+template <bool kFast, int kNS>
+__global__ __launch_bounds__(kBlkT) void k_pbf_deltap_blk(const float4* __restrict__ xl, const int* __restrict__ key2,
+                                                          const int* __restrict__ cs, int n, PbfK k,
+                                                          float4* __restrict__ xa, const float4* __restrict__ xold,
+                                                          float4* __restrict__ vout, float dt,
+                                                          unsigned long long* __restrict__ nb,
+                                                          const float4* __restrict__ xp, const int* __restrict__ gate,
+                                                          const int* __restrict__ blk) {
+    if (gate && *gate == 0) return;
+    __shared__ float4 copy[kBlkCap];
+    lds_f32x4* __restrict__ S = (lds_f32x4*)copy;
+    const int tile = blk_tile();
+    const int i = tile * kBlkT + (int)threadIdx.x;
+    if (tile * kBlkT >= n) return;
+    const int* __restrict__ bt = blk + (size_t)tile * kBlkInts;
+    const bool staged = bt[kBlkStaged] != 0;
+    const int ii = i < n ? i : n - 1;
+    const float4 pi = xl[ii];
+    const BlkList l(ii, n, tile, staged, nb);
+    if (staged) {
+        blk_copy(bt, xl, [&](int e, const float4 v, int) { S[e] = f32x4_t{v.x, v.y, v.z, v.w}; });
+        __syncthreads();
+    }
+    if (i >= n) return;
+    deltap_body<kFast, kNS>(i, pi, k, xa, xold, vout, dt, [&](auto&& f) {
+        for_each_neighbor_blk<kWalkWide>(i, l, staged, key2, cs, xp, xl, nullptr, k,
+                                         [&](unsigned int e, float4& p, float4&) { p = lds4(S, e); }, f);
+    });
+}
+
+// The waves' maxima and sums of C, out[w] and out[waves + w] (wave w: slots
+// 64w .. 64w + 63); k_pbf_decide adds them as block_max_sum_store's blocks do
+__device__ __forceinline__ void wave_max_sum_store(float cmax, float csum, int i, int n, int* __restrict__ out) {
+    int m = ordered(cmax);
+    float s = csum;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const int o = __shfl_xor(m, d, 64);
+        m = o > m ? o : m;
+        s += __shfl_xor(s, d, 64);
+    }
+    if ((threadIdx.x & 63) == 0 && i < n) {
+        out[i >> 6] = m;
+        out[((n + 63) >> 6) + (i >> 6)] = __float_as_int(s);
+    }
+}
+
+template <bool kFast, bool kCheck>
+__global__ __launch_bounds__(kBlkT) void k_pbf_xsph_blk(const float4* __restrict__ xa, const float4* __restrict__ vt,
+                                                        const int* __restrict__ key2, const int* __restrict__ cs, int n,
+                                                        PbfK k, float4* __restrict__ vout, float4* __restrict__ xout,
+                                                        unsigned long long* __restrict__ nb,
+                                                        const float4* __restrict__ xp, int* __restrict__ maxd,
+                                                        const int* __restrict__ gate, NextKeys nk,
+                                                        const int* __restrict__ blk) {
+    if (gate && *gate == 0) return;  // uniform: before any barrier
+    __shared__ float4 copy[kBlkCap];  // x, y, z, slot (as bits)
+    lds_f32x4* __restrict__ S = (lds_f32x4*)copy;
+    const int tile = blk_tile();
+    const int i = tile * kBlkT + (int)threadIdx.x;
+    float Ci = -1e30f;
+    float4 xn = make_float4(0.0f, 0.0f, 0.0f, 0.0f), vn = xn;
+    if (tile * kBlkT < n) {
+        const int* __restrict__ bt = blk + (size_t)tile * kBlkInts;
+        const bool staged = bt[kBlkStaged] != 0;
+        const int ii = i < n ? i : n - 1;
+        const float4 pi = xa[ii], vi = vt[ii];
+        const BlkList l(ii, n, tile, staged, nb);
+        if (staged) {
+            blk_copy(bt, xa, [&](int e, const float4 v, int j) { S[e] = f32x4_t{v.x, v.y, v.z, __int_as_float(j)}; });
+            __syncthreads();
+        }
+        if (i < n)
+            Ci = xsph_body<kFast, kCheck>(i, pi, vi, k, vout, xout, [&](auto&& f) {
+                for_each_neighbor_blk<kWalkPairs>(i, l, staged, key2, cs, xp, xa, vt, k,
+                                                  [&](unsigned int e, float4& p, float4& a) {
+                                                      const f32x4_t v = S[e];
+                                                      p = make_float4(v.x, v.y, v.z, 0.0f);
+                                                      a = at4(vt, __float_as_int(v.w));
+                                                  },
+                                                  f);
+            }, &xn, &vn);
+    }
+    if (nk.key) next_key(i, i < n, xn, vn, k, nk);
+    if (kCheck) wave_max_sum_store(Ci, Ci > 0.0f ? Ci : 0.0f, i, n, maxd);
+}
+
+static hipError_t launch_build_blk(const float4* xp, const int* key2, const int* cs, int n, const PbfK& k, float4* xl,
+                                   int* maxc, unsigned long long* nb, const int* gate, int* blk, hipStream_t s) {
+    const dim3 g(grid_for(n, kBlkT)), b(kBlkT);
+    if (xl && k.exact)
+        launch_kernel((k_pbf_build_blk<false, true>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, nb, gate, blk);
+    else if (xl)
+        launch_kernel((k_pbf_build_blk<true, true>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, nb, gate, blk);
+    else if (k.exact)
+        launch_kernel((k_pbf_build_blk<false, false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, nb, gate, blk);
+    else
+        launch_kernel((k_pbf_build_blk<true, false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, nb, gate, blk);
+    return hipGetLastError();
+}
+
+static hipError_t launch_lambda_blk(const float4* xa, const int* key2, const int* cs, int n, const PbfK& k, float4* xl,
+                                    int* maxc, unsigned long long* nb, const float4* xp, const int* gate, const int* blk,
+                                    hipStream_t s) {
+    const dim3 g(grid_for(n, kBlkT)), b(kBlkT);
+    if (k.exact)
+        launch_kernel((k_pbf_lambda_blk<false>), g, b, 0, s, xa, key2, cs, n, k, xl, maxc, nb, xp, gate, blk);
+    else
+        launch_kernel((k_pbf_lambda_blk<true>), g, b, 0, s, xa, key2, cs, n, k, xl, maxc, nb, xp, gate, blk);
+    return hipGetLastError();
+}
+
+static hipError_t launch_deltap_blk(const float4* xl, const int* key2, const int* cs, int n, const PbfK& k, float4* xa,
+                                    const float4* xold, float4* vout, float dt, unsigned long long* nb,
+                                    const float4* xp, const int* gate, const int* blk, hipStream_t s) {
+    const dim3 g(grid_for(n, kBlkT)), b(kBlkT);
+    const bool n4 = k.n_scorr == 4;
+#define LUS_DP(F, N) \
+    launch_kernel((k_pbf_deltap_blk<F, N>), g, b, 0, s, xl, key2, cs, n, k, xa, xold, vout, dt, nb, xp, gate, blk)
+    if (k.exact && n4) LUS_DP(false, 4);
+    else if (k.exact) LUS_DP(false, 0);
+    else if (n4) LUS_DP(true, 4);
+    else LUS_DP(true, 0);
+#undef LUS_DP
+    return hipGetLastError();
+}
+
+static hipError_t launch_xsph_blk(const float4* xa, const float4* vt, const int* key2, const int* cs, int n,
+                                  const PbfK& k, float4* vout, float4* xout, unsigned long long* nb, const float4* xp,
+                                  int* maxd, const int* gate, const NextKeys& nk, const int* blk, hipStream_t s) {
+    const dim3 g(grid_for(n, kBlkT)), b(kBlkT);
+#define LUS_XS(F, C) \
+    launch_kernel((k_pbf_xsph_blk<F, C>), g, b, 0, s, xa, vt, key2, cs, n, k, vout, xout, nb, xp, maxd, gate, nk, blk)
+    if (k.exact && maxd) LUS_XS(false, true);
+    else if (k.exact) LUS_XS(false, false);
+    else if (maxd) LUS_XS(true, true);
+    else LUS_XS(true, false);
+#undef LUS_XS
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -2034,6 +2456,7 @@ hipError_t launch_pbf_xsph(const float4* xa, const float4* vt, int* key2, const 
     }
     if (ta.sub > 1 && !k.exact && !maxd)
         return launch_xsph_sub(xa, vt, key2, cs, n, k, vout, xout, masks, xp, gate, s, nk);
+    if (ta.blk) return launch_xsph_blk(xa, vt, key2, cs, n, k, vout, xout, masks, xp, maxd, gate, nk, ta.blk, s);
     const dim3 g(grid_for(n, ta.block)), b(ta.block);
     if (k.exact && maxd)
         launch_kernel((k_pbf_xsph<false, true>), g, b, 0, s, xa, vt, key2, cs, n, k, vout, xout, masks, xp, maxd, gate,
@@ -2454,11 +2877,41 @@ __device__ __forceinline__ void features_body(int i, const float4* __restrict__ 
     }
 }
 
+// Walk a staged block's list (header count c) with each place turned back into
+// its slot (the nine rows' copies ascend), calling f(j, cur[j], zeros): for the
+// features, whose bins take the LDS that a copy would need
+template <class F>
+__device__ __forceinline__ void visit_list_places(int c, const int4* __restrict__ lst, const int* __restrict__ bt,
+                                                  const float4* __restrict__ cur, F& f) {
+    if (c <= 0) return;
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int4 g = lst[0];
+    for (int t = 0; t < c; t += 8) {
+        const unsigned int w[4] = {(unsigned int)g.x, (unsigned int)g.y, (unsigned int)g.z, (unsigned int)g.w};
+        int j[8];
+        float4 p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = (int)((u & 1) ? w[u >> 1] >> 16 : w[u >> 1] & 0xFFFFu);
+            int shift = bt[0];
+#pragma unroll
+            for (int r = 1; r < 9; ++r) shift = e >= bt[9 + r] + bt[r] ? bt[r] : shift;
+            j[u] = e - shift;
+            p[u] = at4(cur, j[u]);
+        }
+        const int gi = (t >> 3) + 1 < kNbrGroups ? (t >> 3) + 1 : kNbrGroups - 1;
+        g = lst[(size_t)gi * 64];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (t + u < c) f(j[u], p[u], z);
+    }
+}
+
 // kBuild: the pass builds the lists from per-lane gathers; else it walks the
-// lists of k_pbf_list_build_ws
+// lists of k_pbf_list_build_ws (blk null) or k_pbf_build_blk
 template <bool kFast, bool kRecord, bool kBuild>
 __global__ __launch_bounds__(kBlock) void k_pbf_features(
-    int* __restrict__ key2, const int* __restrict__ cs, int n, PbfK k,
+    int* __restrict__ key2, const int* __restrict__ cs, int n, PbfK k, const int* __restrict__ blk,
     unsigned long long* __restrict__ masks, const float4* __restrict__ xp,
     const float4* __restrict__ xold, const float* __restrict__ mu, const float* __restrict__ inv_sigma,
     bf16x8_t* __restrict__ fbf, float* __restrict__ frec, int rec_stride, int rec_off, float inv_h) {
@@ -2467,6 +2920,19 @@ __global__ __launch_bounds__(kBlock) void k_pbf_features(
     if (i >= n) return;
     features_body<kFast, kRecord, true>(i, xp, xold, k, mu, inv_sigma, fbf, frec, rec_stride, rec_off, inv_h,
                                   [&](auto&& f) {
+        if constexpr (!kBuild) {
+            // uniform: a wave's slots lie in one block
+            const int tile = __builtin_amdgcn_readfirstlane(i / kBlkT);
+            const int* __restrict__ bt = blk + (size_t)tile * kBlkInts;
+            if (blk && bt[kBlkStaged]) {
+                const int c = blk_counts(masks, tile)[i - tile * kBlkT];
+                if (c <= kNbrCap)
+                    visit_list_places(c, nbr_list(masks, n, i), bt, xp, f);
+                else
+                    retest_neighbors(i, key2, cs, xp, xp, nullptr, k, f);
+                return;
+            }
+        }
         for_each_neighbor<kBuild, kWalkWide>(i, n, key2, cs, masks, xp, xp, nullptr, k, f);
     }, (lds_float4*)bins + threadIdx.x);
 }
@@ -2516,18 +2982,20 @@ hipError_t launch_pbf_features(int* key2, const int* cs, int n, PbfK k, unsigned
     // the staged build and a walk of its lists, or (lus_pbf_set_build(0)) both
     // in one pass of gathers
     const bool staged = ta.stage && n > 0;
-    if (staged && k.exact)
+    if (staged && ta.blk) {
+        if (hipError_t e = launch_build_blk(xp, key2, cs, n, k, nullptr, nullptr, masks, nullptr, ta.blk, s)) return e;
+    } else if (staged && k.exact)
         launch_kernel((k_pbf_list_build_ws<false>), g, b, 0, s, xp, (const int*)key2, cs, n, k, masks);
     else if (staged)
         launch_kernel((k_pbf_list_build_ws<true>), g, b, 0, s, xp, (const int*)key2, cs, n, k, masks);
 #define LUS_FEAT(F, R)                                                                                              \
     do {                                                                                                            \
         if (staged)                                                                                                 \
-            launch_kernel((k_pbf_features<F, R, false>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu, inv_sigma, \
-                          (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                                        \
+            launch_kernel((k_pbf_features<F, R, false>), g, b, 0, s, key2, cs, n, k, (const int*)ta.blk, masks, xp, xold, mu, \
+                          inv_sigma, (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                             \
         else                                                                                                        \
-            launch_kernel((k_pbf_features<F, R, true>), g, b, 0, s, key2, cs, n, k, masks, xp, xold, mu, inv_sigma, \
-                          (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                                        \
+            launch_kernel((k_pbf_features<F, R, true>), g, b, 0, s, key2, cs, n, k, (const int*)ta.blk, masks, xp, xold, mu, \
+                          inv_sigma, (bf16x8_t*)fbf, frec, rec_stride, rec_off, inv_h);                             \
     } while (0)
     if (frec)
         LUS_FEAT(false, true);
@@ -2567,7 +3035,9 @@ hipError_t launch_pbf_record_target(const float4* xa, const float4* xp, int n, i
 // hist[cap + step % cap], decide the rerun.  learned: 0 a plain step (record
 // only), 1 a learned attempt (record, set *flag when e > bound), 2 after the
 // gated rerun (when *flag is set, the rerun's e replaces the step's entry).
-__global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ maxd, int nblk, int n,
+// waves: maxd holds the waves' values (wave_max_sum_store), block b's being those
+// of its tile's four waves.
+__global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ maxd, int nblk, int n, int waves,
                                                        float bound, int learned, int* __restrict__ flag,
                                                        int* __restrict__ counters, float* __restrict__ hist,
                                                        int cap) {
@@ -2576,8 +3046,21 @@ __global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ m
     int m = INT_MIN;
     float s = 0.0f;
     for (int b = threadIdx.x; b < nblk; b += kBlock) {
-        m = maxd[b] > m ? maxd[b] : m;
-        s += __int_as_float(maxd[nblk + b]);
+        int bm = INT_MIN;
+        float bs = 0.0f;
+        if (waves) {
+            constexpr int kW = kBlock / 64;
+            const int w0 = ((b % kXcd) * (nblk / kXcd) + b / kXcd) * kW, nw = (n + 63) / 64;
+            for (int w = w0; w < w0 + kW && w < nw; ++w) {
+                bm = maxd[w] > bm ? maxd[w] : bm;
+                bs += __int_as_float(maxd[nw + w]);
+            }
+        } else {
+            bm = maxd[b];
+            bs = __int_as_float(maxd[nblk + b]);
+        }
+        m = bm > m ? bm : m;
+        s += bs;
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -2619,26 +3102,32 @@ __global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ m
     }
 }
 
-hipError_t launch_pbf_decide(const int* maxd, int nblk, int n, float bound, int learned, int* flag,
+hipError_t launch_pbf_decide(const int* maxd, int nblk, int n, int waves, float bound, int learned, int* flag,
                              int* counters, float* hist, int cap, hipStream_t s) {
-    launch_kernel(k_pbf_decide, dim3(1), dim3(kBlock), 0, s, maxd, nblk, n, bound, learned, flag,
+    launch_kernel(k_pbf_decide, dim3(1), dim3(kBlock), 0, s, maxd, nblk, n, waves, bound, learned, flag,
                        counters, hist, cap);
     return hipGetLastError();
 }
 
 // Particles of the last list-building pass whose list could not be stored
 // (header count kNbrRetest): they re-test their candidates in every pass.
-__global__ __launch_bounds__(kBlock) void k_pbf_count_retest(const int4* __restrict__ hdr, int n,
-                                                              int* __restrict__ out) {
+__global__ __launch_bounds__(kBlock) void k_pbf_count_retest(unsigned long long* __restrict__ nb, int n,
+                                                              const int* __restrict__ blk, int* __restrict__ out) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    int c = (i < n && (hdr[i].w & 0xFFFF) == kNbrRetest) ? 1 : 0;
+    int c = 0;
+    if (i < n) {
+        const int tile = i / kBlkT;
+        const int w = blk && blk[(size_t)tile * kBlkInts + kBlkStaged] ? blk_counts(nb, tile)[i - tile * kBlkT]
+                                                               : nbr_hdr(nb)[i].w & 0xFFFF;
+        c = w == kNbrRetest ? 1 : 0;
+    }
     for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
     if ((threadIdx.x & 63) == 0 && c) atomicAdd(out, c);
 }
 
-hipError_t launch_pbf_count_retest(const unsigned long long* nb, int n, int* out, hipStream_t s) {
+hipError_t launch_pbf_count_retest(const unsigned long long* nb, int n, const int* blk, int* out, hipStream_t s) {
     launch_kernel(k_pbf_count_retest, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                  reinterpret_cast<const int4*>(nb), n, out);
+                  const_cast<unsigned long long*>(nb), n, blk, out);
     return hipGetLastError();
 }
 

@@ -407,8 +407,9 @@ class Gpu:
 
     def pbf_set_build(self, staged=True):
         """staged: the list build tests wave-staged candidates in LDS; else
-        per-lane gathers (same results)."""
-        _check(self._lib.lus_pbf_set_build(self._h, int(bool(staged))), "lus_pbf_set_build")
+        per-lane gathers (same results).  2: block-staged lists at any size
+        (True: at the sizes where they are faster)."""
+        _check(self._lib.lus_pbf_set_build(self._h, int(staged)), "lus_pbf_set_build")
 
     def pbf_set_lanes(self, lanes=0):
         """Lanes per particle in fused list walks: 0 automatic, 1 or 4."""

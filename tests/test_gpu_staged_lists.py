@@ -1,5 +1,5 @@
-"""The list forms of a step against the gathered one (lus_pbf_set_build(0)):
-the same neighbour sets in the same order, so the same bits in every pass that
+"""The list forms of a step -- wave-staged build (lus_pbf_set_build(1)) and
+block-staged lists (2) -- against the gathered one (0): the same neighbour sets in the same order, so the same bits in every pass that
 walks them -- the plain solver, the learned step's features and the training
 rows -- at sizes around a wave and a block, for columns of cells shorter and
 longer than a block, dense cells (rows past what is staged) and lists past
@@ -48,7 +48,9 @@ def same(a, b):
 @pytest.mark.parametrize("k", range(len(SCENES)))
 def test_plain_steps(gpu_mod, k, exact):
     cfg, pos, vel = scene(*SCENES[k], seed=k)
-    same(plain(gpu_mod, cfg, pos, vel, True, exact), plain(gpu_mod, cfg, pos, vel, False, exact))
+    want = plain(gpu_mod, cfg, pos, vel, 0, exact)
+    for staged in (1, 2):
+        same(plain(gpu_mod, cfg, pos, vel, staged, exact), want)
 
 
 @pytest.mark.parametrize("exact", [True, False])
@@ -56,8 +58,9 @@ def test_plain_steps(gpu_mod, k, exact):
 def test_dense_scenes(gpu_mod, squeeze, exact):
     # 2 to 11 times the rest density: full cells, long rows, lists past 128 entries
     cfg, pos, vel = scene((24, 16, 24), (48, 32, 48), 0.05, 7, squeeze)
-    a = plain(gpu_mod, cfg, pos, vel, True, exact, steps=2)
-    same(a, plain(gpu_mod, cfg, pos, vel, False, exact, steps=2))
+    want = plain(gpu_mod, cfg, pos, vel, 0, exact, steps=2)
+    for staged in (1, 2):
+        same(plain(gpu_mod, cfg, pos, vel, staged, exact, steps=2), want)
 
 
 @pytest.mark.parametrize("k", [2, 5])
@@ -65,7 +68,7 @@ def test_learned_steps(gpu_mod, k):
     cfg, pos, vel = scene(*SCENES[k], seed=k)
     net = learned.load()[0]
     out = []
-    for staged in (True, False):
+    for staged in (0, 1, 2):
         with gpu_mod.Gpu(0) as g:
             g.pbf_set_build(staged)
             g.pbf_init(gpu_mod.pbf_params(cfg, iterations=6, exact=False), pos, vel)
@@ -73,14 +76,15 @@ def test_learned_steps(gpu_mod, k):
             g.pbf_set_mode(True, 2, 0.05)  # some steps rerun
             g.pbf_step(np.float32(cfg.dt), 4)
             out.append(g.pbf_download(order=0) + tuple(np.asarray(q) for q in g.pbf_learned_stats(True)))
-    same(*out)
+    same(out[0], out[1])
+    same(out[0], out[2])
 
 
 @pytest.mark.parametrize("exact", [True, False])
 def test_recorded_rows(gpu_mod, exact):
     cfg, pos, vel = scene(*SCENES[2], seed=3)
     out = []
-    for staged in (True, False):
+    for staged in (0, 1, 2):
         with gpu_mod.Gpu(0) as g:
             g.pbf_set_build(staged)
             g.pbf_init(gpu_mod.pbf_params(cfg, exact=exact), pos, vel)
@@ -89,7 +93,8 @@ def test_recorded_rows(gpu_mod, exact):
                 t.record_step(np.float32(cfg.dt), 3)
             out.append(t.download())
             t.close()
-    same(*out)
+    same(out[0], out[1])
+    same(out[0], out[2])
 
 
 def test_batch(gpu_mod):
@@ -97,11 +102,12 @@ def test_batch(gpu_mod):
     cfgs = [scenes.dam_break_of_size(n, n) for n in (40, 700, 2500, 90)]
     pos = np.concatenate([c.positions() for c in cfgs])
     out = []
-    for staged in (True, False):
+    for staged in (0, 1, 2):
         with gpu_mod.Gpu(0) as g:
             g.pbf_set_build(staged)
             g.pbf_set_lanes(1)
             g.pbf_batch_init(gpu_mod.pbf_params(cfgs[0], exact=False), [c.n for c in cfgs], [c.box for c in cfgs], pos)
             g.pbf_step(np.float32(cfgs[0].dt), 3)
             out.append(g.pbf_download(order=1))
-    same(*out)
+    same(out[0], out[1])
+    same(out[0], out[2])
