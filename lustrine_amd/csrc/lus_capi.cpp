@@ -246,11 +246,10 @@ struct SandState {
            *B = nullptr, *solid = nullptr;
     int *att = nullptr, *att2 = nullptr, *key = nullptr, *slot = nullptr, *tmp = nullptr,
         *perm = nullptr, *key2 = nullptr, *counts = nullptr, *cs = nullptr, *tiles = nullptr,
-        *ocs = nullptr, *solid_ref = nullptr, *nbr_off = nullptr, *nbr_cnt = nullptr,
-        *nbr_cnt1 = nullptr, *nbr_idx = nullptr, *ntiles = nullptr;
-    long nbr_cap = 0;
-    Arena nbr_mem;
-    float4* final_iter = nullptr;
+        *ocs = nullptr, *solid_ref = nullptr;
+    lus::SandLists L{};
+    Arena pool_mem;    // L.pool
+    int list_n = 0;    // sand slots when the lists were built
     int* qbuf = nullptr;  // one int: cell-box count
     int* err = nullptr;   // one int: a simulate_sand_v3 prediction left the grid
     float* stage = nullptr;  // 6 n floats: packed positions and velocities for downloads
@@ -713,7 +712,7 @@ void lus_gpu_destroy(LusGpu* c) {
     c->pbf.mem.release();
     c->net.mem.release();
     c->sand.mem.release();
-    c->sand.nbr_mem.release();
+    c->sand.pool_mem.release();
     lus::fluid_free(c->fluid);
     c->fluid = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1902,10 +1901,9 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
     LUS_HIP(hipStreamSynchronize(c->stream));
     sand_drop_graphs(S);
     S.mem.release();
-    S.nbr_mem.release();
+    S.pool_mem.release();
     // everything that pointed into the released memory
-    S.nbr_idx = nullptr;
-    S.nbr_cap = 0;
+    S.L = lus::SandLists{};
     S.fail = nullptr;
     S.fixed_cap = 0;
     S.use_graph = false;
@@ -1973,10 +1971,17 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
     LUS_HIP(m.alloc(&S.counts, S.C + 1));
     LUS_HIP(m.alloc(&S.cs, S.C + 1));
     LUS_HIP(m.alloc(&S.tiles, lus::scan_tile_count(S.C + 1) + 1));
-    LUS_HIP(m.alloc(&S.nbr_off, n + 1));
-    LUS_HIP(m.alloc(&S.nbr_cnt, n + 1));
-    LUS_HIP(m.alloc(&S.nbr_cnt1, n));
-    LUS_HIP(m.alloc(&S.ntiles, lus::scan_tile_count(n + 1) + 1));
+    {
+        // A list's fixed place holds three times the neighbours of unit
+        // spacing (4/3 pi (h/d)^3; grains in contact pack 1.4 times as
+        // densely), between 32 and 128 entries; longer lists go to the pool.
+        const double hd = (double)p->kernelRadius / (double)p->particleDiameter;
+        const double want = 3.0 * 4.18879 * hd * hd * hd / 4.0;
+        S.L.groups = !(want > 8.0) ? 8 : (want < 32.0 ? (int)std::ceil(want) : 32);
+        LUS_HIP(m.alloc(&S.L.hdr, n));
+        LUS_HIP(m.alloc(&S.L.lists, ((size_t)n + 63) / 64 * 64 * (size_t)S.L.groups));
+        LUS_HIP(m.alloc(&S.L.ctl, 2));
+    }
     LUS_HIP(m.alloc(&S.qbuf, 1));
     LUS_HIP(m.alloc(&S.err, 1));
     std::vector<float4> hx = to_f4(pos, n), hv = to_f4(vel, n);
@@ -1986,7 +1991,6 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
     LUS_HIP(hipMemcpy(S.v, hv.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
     LUS_HIP(hipMemcpy(S.att, ha.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     LUS_HIP(hipMemset(S.counts, 0, sizeof(int) * (S.C + 1)));
-    LUS_HIP(hipMemset(S.nbr_cnt, 0, sizeof(int) * (n + 1)));
     // the out-of-grid flag is read by every no-wait step's check, whatever the
     // variant: it starts clear (a new allocation may hold an old context's data)
     LUS_HIP(hipMemset(S.err, 0, sizeof(int)));
@@ -2046,9 +2050,20 @@ int sand_check(LusGpu* c) {
     return LUS_OK;
 }
 
+// Room for `groups` int4 in the pool of long lists
+int sand_pool(SandState& S, long groups) {
+    S.pool_mem.release();
+    S.L.pool = nullptr;
+    S.L.pool_groups = 0;
+    LUS_HIP(S.pool_mem.alloc(&S.L.pool, (size_t)groups));
+    S.L.pool_groups = groups;
+    return LUS_OK;
+}
+
 // Enqueues one simulate_sand step.  Without a fixed capacity it waits once
-// for the lists' total length (it sizes their buffer); with one it does not
-// wait, and a step whose lists do not fit is reported by sand_check.  The
+// for the lists' lengths (lists longer than their place size the pool); with
+// one it does not wait, and a step whose lists do not fit is reported by
+// sand_check.  The
 // host-side buffer swaps are applied by sand_after.
 int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
     SandState& S = c->sand;
@@ -2061,47 +2076,42 @@ int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
     LUS_HIP(mark(0));
     if (k.variant == 2 && !fixed) LUS_HIP(lus::launch_zero_ints(S.err, 1, s));
     LUS_HIP(lus::launch_sand_predict_key(S.x, S.v, S.att, n, k, dt, S.err, S.xs, S.key, S.slot, S.counts,
-                                         s));
+                                         S.L.ctl, s));
     LUS_HIP(mark(1));
     LUS_HIP(lus::launch_exclusive_scan(S.counts, S.cs, S.C + 1, S.tiles, 1, s));
     LUS_HIP(lus::launch_scatter(S.key, S.slot, S.cs, n, S.tmp, s));
-    LUS_HIP(lus::launch_sand_permute(S.tmp, S.key, S.cs, S.x, S.xs, S.v, S.att, n, S.x2, S.A, S.v2,
-                                     S.att2, S.perm, S.key2, s));
-    // neighbor lists: count, scan, fill
-    LUS_HIP(lus::launch_sand_nbr(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, nullptr, S.nbr_cnt,
-                                 S.nbr_cnt1, nullptr, 0, s));
-    LUS_HIP(lus::launch_exclusive_scan(S.nbr_cnt, S.nbr_off, n + 1, S.ntiles, 0, s));
-    if (!fixed) {
-        int total = 0, bad_key = 0;
-        LUS_HIP(hipMemcpyAsync(&total, S.nbr_off + n, sizeof(int), hipMemcpyDeviceToHost, s));
+    LUS_HIP(lus::launch_sand_permute(S.tmp, S.key, S.cs, S.x, S.xs, S.att, n, S.x2, S.A, S.att2, S.perm, S.key2,
+                                     s));
+    for (;;) {
+        LUS_HIP(lus::launch_sand_lists(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, S.L, s));
+        if (fixed) break;  // lists within the capacity fit the pool
+        unsigned long long ctl[2] = {0ull, 0ull};
+        int bad_key = 0;
+        LUS_HIP(hipMemcpyAsync(ctl, S.L.ctl, sizeof(ctl), hipMemcpyDeviceToHost, s));
         if (k.variant == 2) LUS_HIP(hipMemcpyAsync(&bad_key, S.err, sizeof(int), hipMemcpyDeviceToHost, s));
         LUS_HIP(hipStreamSynchronize(s));
         if (bad_key)
             return set_error(LUS_EINVAL,
                              "lus_sand_step: a predicted position's cell lies outside the grid (simulate_sand_v3 "
                              "does not clamp; the reference indexes outside its cell vector there)");
-        if (total < 0) return set_error(LUS_EHIP, "lus_sand_step: neighbor count overflow");
-        if ((long)total > S.nbr_cap || !S.nbr_idx) {
-            S.nbr_mem.release();
-            long cap = std::max<long>((long)total + total / 4, 64);
-            LUS_HIP(S.nbr_mem.alloc(&S.nbr_idx, (size_t)cap));
-            S.nbr_cap = cap;
-        }
+        if (ctl[0] > (unsigned long long)INT_MAX) return set_error(LUS_EHIP, "lus_sand_step: neighbor count overflow");
+        if (ctl[1] <= (unsigned long long)S.L.pool_groups) break;
+        if (int r = sand_pool(S, (long)(ctl[1] + ctl[1] / 4))) return r;
+        LUS_HIP(lus::launch_zero_ints(reinterpret_cast<int*>(S.L.ctl), 4, s));
     }
-    LUS_HIP(lus::launch_sand_nbr(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, S.nbr_off, S.nbr_cnt,
-                                 S.nbr_cnt1, S.nbr_idx, 1, s, S.nbr_cap, fixed ? S.fail : nullptr));
     LUS_HIP(mark(2));
     float4* A = S.A;
     float4* B = S.B;
     // simulate_sand_v3's substeps all read the same positions_tmp: one pass
     const int passes = k.variant == 2 ? (S.p.substeps > 0 ? 1 : 0) : S.p.substeps;
+    int* fail = fixed ? S.fail : nullptr;
     for (int it = 0; it < passes; ++it) {
-        LUS_HIP(lus::launch_sand_substep(A, S.x2, S.solid, S.nbr_off, S.nbr_idx, n, k, B, S.att2, s,
-                                         fixed ? S.fail : nullptr));
+        LUS_HIP(lus::launch_sand_substep(A, S.x2, S.solid, S.L, n, k, B, it + 1 == passes ? S.v2 : nullptr, dt, S.att2,
+                                         s, S.fixed_cap, fail));
         std::swap(A, B);
     }
     LUS_HIP(mark(3));
-    LUS_HIP(lus::launch_sand_vupdate(A, S.x2, S.v2, n, dt, s));
+    if (passes == 0) LUS_HIP(lus::launch_sand_velocity(A, S.x2, S.v2, n, dt, S.L, s, S.fixed_cap, fail));
     LUS_HIP(mark(4));
     if (c->profiling) {
         // slots of simulate_sand_v1 (src/Simulate.cpp:669-802): 0 the call,
@@ -2120,12 +2130,13 @@ int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
 // replayed graph of it)
 void sand_after(SandState& S, const lus::SandK& k) {
     const int passes = k.variant == 2 ? (S.p.substeps > 0 ? 1 : 0) : S.p.substeps;
-    if (passes & 1) std::swap(S.A, S.B);
-    S.final_iter = S.A;
-    std::swap(S.x, S.x2);
+    // the last substep's positions are the new ones, the old ones' buffer is
+    // free (a swap: two assignments alternate, as the graphs' key has them)
+    std::swap(S.x, (passes & 1) ? S.B : S.A);
     std::swap(S.v, S.v2);
     std::swap(S.att, S.att2);
     if (k.variant != 2) S.prev_attract = k.attract;  // v3 keeps no previous flag
+    S.list_n = S.n;
     S.stepped = true;
 }
 
@@ -2210,11 +2221,9 @@ int lus_sand_set_list_capacity(LusGpu* c, long entries) {
         S.use_graph = false;
         return LUS_OK;
     }
-    S.nbr_mem.release();
-    S.nbr_idx = nullptr;
-    S.nbr_cap = 0;
-    LUS_HIP(S.nbr_mem.alloc(&S.nbr_idx, (size_t)entries));
-    S.nbr_cap = entries;
+    // Lists of at most `entries` in total always fit: those in the pool have
+    // more than 4 groups (32 at least) entries each, rounded up to a group
+    if (int r = sand_pool(S, entries / 4 + entries / 32 + 1)) return r;
     if (!S.fail) LUS_HIP(S.mem.alloc(&S.fail, 1));
     LUS_HIP(hipMemset(S.fail, 0, sizeof(int)));
     S.fixed_cap = entries;
@@ -2367,15 +2376,14 @@ int lus_sand_sink_evict(LusGpu* c, const int* cells, int ncells, int* n_sand) {
         const int m = (int)mv.size();
         if (m > 0) {
             int2* d_mv;
-            float4 *t0, *t1, *t2;
-            int* t3;
+            float4 *t0, *t1;
+            int* t2;
             LUS_HIP(tmp.alloc(&d_mv, m));
             LUS_HIP(tmp.alloc(&t0, m));
             LUS_HIP(tmp.alloc(&t1, m));
             LUS_HIP(tmp.alloc(&t2, m));
-            LUS_HIP(tmp.alloc(&t3, m));
             LUS_HIP(hipMemcpyAsync(d_mv, mv.data(), sizeof(int2) * m, hipMemcpyHostToDevice, s));
-            LUS_HIP(lus::launch_slot_moves(d_mv, m, S.x, S.final_iter, S.v, S.att, t0, t1, t2, t3, s));
+            LUS_HIP(lus::launch_slot_moves(d_mv, m, S.x, S.v, S.att, t0, t1, t2, s));
             LUS_HIP(hipStreamSynchronize(s));
         }
         S.n = end;
@@ -2525,18 +2533,27 @@ int lus_sand_neighbors(LusGpu* c, long* off, int* idx, long cap, long* total) {
     LUS_HIP(hipStreamSynchronize(c->stream));
     if (int r = sand_check(c)) return r;
     const int n = S.n;
+    hipStream_t s = c->stream;
+    Arena tmp;
+    int *cnt, *d_off, *tiles, *d_idx;
+    LUS_HIP(tmp.alloc(&cnt, n + 1));
+    LUS_HIP(tmp.alloc(&d_off, n + 1));
+    LUS_HIP(tmp.alloc(&tiles, lus::scan_tile_count(n + 1) + 1));
+    LUS_HIP(hipMemsetAsync(cnt + n, 0, sizeof(int), s));
+    LUS_HIP(lus::launch_sand_rows(S.L, S.list_n, n, S.k.sym_limit, S.solid_ref, nullptr, cnt, s));
+    LUS_HIP(lus::launch_exclusive_scan(cnt, d_off, n + 1, tiles, 0, s));
     std::vector<int> o((size_t)n + 1);
-    LUS_HIP(hipMemcpy(o.data(), S.nbr_off, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
+    LUS_HIP(hipMemcpyAsync(o.data(), d_off, sizeof(int) * (n + 1), hipMemcpyDeviceToHost, s));
+    LUS_HIP(hipStreamSynchronize(s));
     for (int i = 0; i <= n; ++i) off[i] = o[i];
     *total = o[n];
     if (*total > cap || (*total > 0 && !idx))
         return set_error(LUS_EINVAL, "lus_sand_neighbors: capacity %ld < %ld", cap, *total);
     if (*total == 0) return LUS_OK;
-    LUS_HIP(hipMemcpy(idx, S.nbr_idx, sizeof(int) * (size_t)*total, hipMemcpyDeviceToHost));
-    std::vector<int> ref((size_t)std::max(S.ns, 1));
-    if (S.ns) LUS_HIP(hipMemcpy(ref.data(), S.solid_ref, sizeof(int) * S.ns, hipMemcpyDeviceToHost));
-    for (long t = 0; t < *total; ++t)
-        if (idx[t] >= n) idx[t] = ref[idx[t] - n];
+    LUS_HIP(tmp.alloc(&d_idx, (size_t)*total));
+    LUS_HIP(lus::launch_sand_rows(S.L, S.list_n, n, S.k.sym_limit, S.solid_ref, d_off, d_idx, s));
+    LUS_HIP(hipMemcpyAsync(idx, d_idx, sizeof(int) * (size_t)*total, hipMemcpyDeviceToHost, s));
+    LUS_HIP(hipStreamSynchronize(s));
     return LUS_OK;
 }
 

@@ -310,24 +310,36 @@ int col_stats_part(int w);
 hipError_t launch_col_stats(const float* x, long rows, int w, double* part, double* out, hipStream_t s);
 
 // sand (simulate_sand)
+// The neighbour lists of a sand step.  Slot i's header: its entry count and,
+// when that exceeds 4 groups, its first int4 in the pool; its entries, four to
+// an int4, lie there contiguously, else lane-blocked in lists: group g of slot
+// i at ((i / 64) * groups + g) * 64 + i % 64.  The last group is filled up
+// with i.  ctl: the lists' total length as the reference counts it, and the
+// pool groups asked for (both zeroed by launch_sand_predict_key).
+struct SandLists {
+    int2* hdr;
+    int4* lists;
+    int4* pool;
+    unsigned long long* ctl;
+    long pool_groups;
+    int groups;
+};
 hipError_t launch_sand_predict_key(float4* x, float4* v, int* att, int n, SandK k, float dt, int* err,
-                                   float4* xs, int* key, int* slot, int* counts, hipStream_t s);
-hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_start,
-                               const float4* x, const float4* xs, const float4* v, const int* att,
-                               int n, float4* x2, float4* xs2, float4* v2, int* att2, int* perm,
-                               int* key2, hipStream_t s);
-// fill with fail non-null: idx holds cap entries; a total past cap (or a
-// negative one) writes nothing and sets *fail, and a substep with *fail set
-// does nothing
-hipError_t launch_sand_nbr(const float4* xs, const int* key2, const int* sand_cs, int n,
-                           const float4* solid, const int* solid_cs, SandK k, const int* off,
-                           int* cnt, int* cnt1, int* idx, int fill, hipStream_t s, long cap = 0,
-                           int* fail = nullptr);
-hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid,
-                               const int* off, const int* idx, int n, SandK k, float4* B, int* att,
-                               hipStream_t s, const int* fail = nullptr);
-hipError_t launch_sand_vupdate(const float4* A, float4* xold_to_new, float4* vout, int n, float dt,
-                               hipStream_t s);
+                                   float4* xs, int* key, int* slot, int* counts, unsigned long long* ctl,
+                                   hipStream_t s);
+hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_start, const float4* x,
+                               const float4* xs, const int* att, int n, float4* x2, float4* xs2, int* att2,
+                               int* perm, int* key2, hipStream_t s);
+hipError_t launch_sand_lists(const float4* xs, const int* key2, const int* sand_cs, int n, const float4* solid,
+                             const int* solid_cs, SandK k, SandLists L, hipStream_t s);
+hipError_t launch_sand_rows(SandLists L, int n, int rows, int sym_limit, const int* solid_ref, const int* off,
+                            int* out, hipStream_t s);
+// v non-null: the last substep, which also forms the velocities.  fail
+// non-null: lists longer than cap in total set *fail and move nothing
+hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid, SandLists L, int n, SandK k,
+                               float4* B, float4* v, float dt, int* att, hipStream_t s, long cap, int* fail);
+hipError_t launch_sand_velocity(const float4* A, const float4* xold, float4* v, int n, float dt, SandLists L,
+                                hipStream_t s, long cap, int* fail);
 
 // grid-state consumers (lus_kernels.hip).  Cell box lo..hi (x, y, z; inclusive)
 // of a grid with cell starts cs (sand slots) and ocs (static solids, reference
@@ -357,8 +369,8 @@ hipError_t launch_chunk_write(const int* cells, const float4* cell_colors, int X
 // voxel model -> grid cells and colours; *occupied += set voxels
 hipError_t launch_grid_from_voxels(const unsigned char* vox, int sx, int sy, int sz, const uchar4* palette,
                                    int* cells, float4* colors, int* occupied, hipStream_t s);
-// a[mv[k].x] = a_old[mv[k].y] for the four arrays; t*: m staging entries each
-hipError_t launch_slot_moves(const int2* mv, int m, float4* a0, float4* a1, float4* a2, int* a3,
-                             float4* t0, float4* t1, float4* t2, int* t3, hipStream_t s);
+// a[mv[k].x] = a_old[mv[k].y] for the three arrays; t*: m staging entries each
+hipError_t launch_slot_moves(const int2* mv, int m, float4* a0, float4* a1, int* a2, float4* t0, float4* t1, int* t2,
+                             hipStream_t s);
 
 }  // namespace lus

@@ -662,10 +662,12 @@ __global__ __launch_bounds__(kBlock) void k_sand_predict_key(float4* __restrict_
                                                               float4* __restrict__ xs,
                                                               int* __restrict__ key,
                                                               int* __restrict__ slot,
-                                                              int* __restrict__ counts) {
+                                                              int* __restrict__ counts,
+                                                              unsigned long long* __restrict__ ctl) {
     const int i = xcd_index();
     const bool active = i < n;
     int c = 0;
+    if (i == 0) ctl[0] = ctl[1] = 0ull;  // the lists' counters (SandLists)
     if (active)
         c = k.variant == 2 ? sand_predict_v3(i, x, v, k, dt, xs, key, err) : sand_predict(i, x, v, att, k, dt, xs, key);
     // one atomic per run of equal keys in the wave (every lane calls it)
@@ -674,19 +676,20 @@ __global__ __launch_bounds__(kBlock) void k_sand_predict_key(float4* __restrict_
 }
 
 hipError_t launch_sand_predict_key(float4* x, float4* v, int* att, int n, SandK k, float dt, int* err,
-                                   float4* xs, int* key, int* slot, int* counts, hipStream_t s) {
+                                   float4* xs, int* key, int* slot, int* counts, unsigned long long* ctl,
+                                   hipStream_t s) {
     launch_kernel(k_sand_predict_key, dim3(grid_for(n)), dim3(kBlock), 0, s, x, v, att, n, k,
-                       dt, err, xs, key, slot, counts);
+                       dt, err, xs, key, slot, counts, ctl);
     return hipGetLastError();
 }
 
-// stable counting sort permutation of x, x*, v, attracted
-// (src/neighbors/Neighbors.cpp:280-304)
+// stable counting sort permutation of x, x*, attracted
+// (src/neighbors/Neighbors.cpp:280-304; the velocity, which the step replaces
+// and nothing reads until then, is not moved)
 __global__ __launch_bounds__(kBlock) void k_sand_permute(
     const int* __restrict__ tmp, const int* __restrict__ key, const int* __restrict__ cell_start,
-    const float4* __restrict__ x, const float4* __restrict__ xs, const float4* __restrict__ v,
-    const int* __restrict__ att, int n, float4* __restrict__ x2, float4* __restrict__ xs2,
-    float4* __restrict__ v2, int* __restrict__ att2, int* __restrict__ perm,
+    const float4* __restrict__ x, const float4* __restrict__ xs, const int* __restrict__ att, int n,
+    float4* __restrict__ x2, float4* __restrict__ xs2, int* __restrict__ att2, int* __restrict__ perm,
     int* __restrict__ key2) {
     const int p = xcd_index();
     if (p >= n) return;
@@ -695,18 +698,16 @@ __global__ __launch_bounds__(kBlock) void k_sand_permute(
     const int o = stable_slot(tmp, cell_start, c, i);
     x2[o] = x[i];
     xs2[o] = xs[i];
-    v2[o] = v[i];
     att2[o] = att[i];
     perm[o] = i;
     key2[o] = c;
 }
 
-hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_start,
-                               const float4* x, const float4* xs, const float4* v, const int* att,
-                               int n, float4* x2, float4* xs2, float4* v2, int* att2, int* perm,
-                               int* key2, hipStream_t s) {
-    launch_kernel(k_sand_permute, dim3(grid_for(n)), dim3(kBlock), 0, s, tmp, key, cell_start,
-                       x, xs, v, att, n, x2, xs2, v2, att2, perm, key2);
+hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_start, const float4* x,
+                               const float4* xs, const int* att, int n, float4* x2, float4* xs2, int* att2,
+                               int* perm, int* key2, hipStream_t s) {
+    launch_kernel(k_sand_permute, dim3(grid_for(n)), dim3(kBlock), 0, s, tmp, key, cell_start, x, xs, att, n, x2,
+                  xs2, att2, perm, key2);
     return hipGetLastError();
 }
 
@@ -715,8 +716,18 @@ hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_s
 // them: entries pushed by earlier slots k < i (the symmetric push of :351-352)
 // come first, in ascending k, then slot i's own scan of the clamped 27 cells
 // in (y, x, z) order, each cell holding its solids first (the cached static
-// lists, :293) then its sand slots; j = i is pushed twice.
+// lists, :293) then its sand slots; j = i, pushed twice, is stored once.
 // Solid entries are stored as n + (solid sorted position).
+//
+// One pass writes them: a list's first `groups` int4 groups have a fixed place
+// (lane-blocked: group g of the 64 slots of a wave is one 1 KB segment, so a
+// walk's loads are whole segments), and a slot with more entries takes a
+// contiguous run of the pool, which its wave scans its stencil a second time
+// to fill.  Counting first and filling exact CSR rows, as before, scanned
+// every stencil twice and left each walk's index loads a line per lane:
+// 1M slots 2 x 118 us + the scan of the counts -> @BUILD@ us, and a substep
+// 77 -> @SUB@ us.
+//
 // Wave-staged: the slots of a wave lie in a few (y, x) cell columns, and
 // within a column their z windows ascend with the slot, so for each stencil
 // row the union of the wave's windows is one slot range per column run, in
@@ -724,6 +735,8 @@ hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_s
 // z of each slot) into LDS with coalesced loads and its lanes test their
 // candidates there, in the same order with the same arithmetic; a row whose
 // ranges exceed kSandStage slots or kSandSegs runs is read from global memory.
+// What bounds it is vector issue: the tests, then one trip of the writer per
+// entry of the wave's fullest lane.
 constexpr int kSandStage = 256;
 constexpr int kSandSegs = 4;
 
@@ -749,53 +762,47 @@ __device__ __forceinline__ unsigned int sand_hits32(const float4 me, const lds_f
     return ~o;
 }
 
-// A slot's list entries as its scan finds them: part 1 (sand slots j < i,
-// pushed by j's own scan in the reference) from o1, part 2 (the own scan)
-// from o2; counted only when not filling
-struct SandHits {
-    int o1 = 0, o2 = 0, n1 = 0, n2 = 0;
-    __device__ __forceinline__ void solid(int js, int n, int fill, int* __restrict__ idx) {
-        if (fill) idx[o2 + n2] = n + js;
-        ++n2;
+// A slot's list as its scan finds it: the last four entries, stored as a
+// group of four to lst[group * stride] while there is room (lim entries, a
+// multiple of four); entries past that are counted only
+struct SandWriter {
+    int c = 0, lim, stride;
+    int4* lst;
+    int q0 = 0, q1 = 0, q2 = 0, q3 = 0;
+    __device__ __forceinline__ void push(int j) {
+        q0 = q1;
+        q1 = q2;
+        q2 = q3;
+        q3 = j;
+        ++c;
+        if ((c & 3) == 0 && c <= lim) lst[(size_t)((c >> 2) - 1) * stride] = make_int4(q0, q1, q2, q3);
     }
-    __device__ __forceinline__ void sand(int j, int i, int fill, int* __restrict__ idx, const SandK& k) {
-        if (j < i) {
-            if (i < k.sym_limit) {
-                if (fill) idx[o1 + n1] = j;
-                ++n1;
-            }
-        } else {
-            if (fill) idx[o2 + n2] = j;
-            ++n2;
-            if (j == i && i < k.sym_limit) {  // j = i is pushed twice
-                if (fill) idx[o2 + n2] = j;
-                ++n2;
-            }
-        }
+    // the last, partial group, filled up with the slot itself
+    __device__ __forceinline__ void finish(int i) {
+        const int rem = c & 3;
+        if (rem == 0 || c > lim) return;
+        const int4 g = rem == 1 ? make_int4(q3, i, i, i) : (rem == 2 ? make_int4(q2, q3, i, i) : make_int4(q1, q2, q3, i));
+        lst[(size_t)(c >> 2) * stride] = g;
     }
 };
 
-__global__ __launch_bounds__(kBlock) void k_sand_nbr(const float4* __restrict__ xs,
-                                                      const int* __restrict__ key2,
-                                                      const int* __restrict__ scs, int n,
-                                                      const float4* __restrict__ solid,
-                                                      const int* __restrict__ ocs, SandK k,
-                                                      const int* __restrict__ off,
-                                                      int* __restrict__ cnt,
-                                                      int* __restrict__ cnt1,
-                                                      int* __restrict__ idx, int fill,
-                                                      long cap, int* __restrict__ fail) {
-    // per wave: the staged sand and solid ranges of a row
-    __shared__ float stage[kBlock / 64][2][3 * kSandStage];
-    // a fixed index buffer (fail non-null): a total past its capacity (or
-    // past the int range) writes nothing and marks the step failed (uniform)
-    if (fill && fail) {
-        const int tot = off[n];
-        if (tot < 0 || (long)tot > cap) {
-            if (xcd_index() == 0) *fail = 1;
-            return;
-        }
-    }
+// group 0 of slot i's list and the distance of its groups
+__device__ __forceinline__ const int4* sand_list(const SandLists& L, int i, int2 h, int& stride) {
+    const bool big = h.x > 4 * L.groups;
+    stride = big ? 1 : 64;
+    return big ? L.pool + h.y : L.lists + (size_t)(i >> 6) * (64 * (size_t)L.groups) + (i & 63);
+}
+
+template <bool kSolid>
+__global__ __launch_bounds__(kBlock) void k_sand_lists(const float4* __restrict__ xs, const int* __restrict__ key2,
+                                                       const int* __restrict__ scs, int n,
+                                                       const float4* __restrict__ solid,
+                                                       const int* __restrict__ ocs, SandK k, SandLists L) {
+    // per wave: the staged sand (and solid) ranges of a row
+    __shared__ float stage[kBlock / 64][kSolid ? 2 : 1][3 * kSandStage];
+    __shared__ int block_total;
+    if (threadIdx.x == 0) block_total = 0;
+    __syncthreads();
     const int i = xcd_index();
     const int lane = (int)(threadIdx.x & 63);
     // every lane of the wave takes part in the staging; a lane past n has no
@@ -803,7 +810,7 @@ __global__ __launch_bounds__(kBlock) void k_sand_nbr(const float4* __restrict__ 
     const bool act = i < n;
     const int ii = act ? i : n - 1;
     lds_float* __restrict__ SS = (lds_float*)stage[threadIdx.x >> 6][0];
-    lds_float* __restrict__ SO = (lds_float*)stage[threadIdx.x >> 6][1];
+    lds_float* __restrict__ SO = (lds_float*)stage[threadIdx.x >> 6][kSolid ? 1 : 0];
     const float4 me = xs[ii];
     const int c = key2[ii];
     const int yy = c / k.gXZ;
@@ -818,167 +825,250 @@ __global__ __launch_bounds__(kBlock) void k_sand_nbr(const float4* __restrict__ 
     if (zz + zl < 0) zl = 0;
     if (zz + zu >= k.gZ) zu = 0;
     const int nz = zu - zl + 1;  // z cells of a row (1 to 3)
-    SandHits h;
-    h.o1 = (fill && act) ? off[i] : 0;            // part 1: sand k < i
-    h.o2 = (fill && act) ? off[i] + cnt1[i] : 0;  // part 2: own scan
-    const unsigned long long below = (1ull << lane) - 1ull;  // lanes before this one
+    const bool sym = ii < k.sym_limit;
+    const unsigned long long upto = (1ull << lane) | ((1ull << lane) - 1ull);  // lanes through this one
+    const int room = 4 * L.groups;
+    SandWriter w;
+    w.lim = act ? room : 0;
+    w.stride = 64;
+    w.lst = L.lists + (size_t)(ii >> 6) * (64 * (size_t)L.groups) + (ii & 63);
+    int base = 0;
+    bool big = false;
 #pragma unroll 1
-    for (int r = 0; r < 9; ++r) {
-        const int y = r / 3 - 1, x = r % 3 - 1;
-        const bool valid = act && y >= yl && y <= yu && x >= xl && x <= xu;
-        // the row's z cells are consecutive: their 2 to 4 boundaries in
-        // both cell tables are requested together
-        const int row = valid ? (yy + y) * k.gXZ + (xx + x) * k.gZ + zz : 0;
-        int sb[4], ob[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const bool in = valid && q <= nz;
-            sb[q] = in ? scs[row + zl + q] : 0;
-            ob[q] = (in && solid) ? ocs[row + zl + q] : 0;
-        }
-        const int s_hi = nz == 1 ? sb[1] : (nz == 2 ? sb[2] : sb[3]);
-        const int o_hi = nz == 1 ? ob[1] : (nz == 2 ? ob[2] : ob[3]);
-        // runs of lanes whose row lies in one cell column (their windows
-        // ascend with the slot)
-        const int col = valid ? (yy + y) * k.gX + (xx + x) : -1;
-        const int pcol = __shfl_up(col, 1, 64);
-        const int ncol = __shfl_down(col, 1, 64);
-        const unsigned long long fm = __ballot(valid && (lane == 0 || pcol != col));
-        const unsigned long long lm = __ballot(valid && (lane == 63 || ncol != col));
-        const int nseg = __popcll(fm);
-        if (nseg == 0) continue;  // uniform: no lane has this row
-        // the runs' sand and solid ranges, packed in LDS at offsets s_off / o_off
-        int s_start[kSandSegs], s_off[kSandSegs + 1], o_start[kSandSegs], o_off[kSandSegs + 1];
-        int tot_s = 0, tot_o = 0;
-        {
-            unsigned long long fq = fm, lq = lm;
-#pragma unroll
-            for (int g = 0; g < kSandSegs; ++g) {
-                s_off[g] = tot_s;
-                o_off[g] = tot_o;
-                s_start[g] = 0;
-                o_start[g] = 0;
-                if (g < nseg) {
-                    const int lf = __ffsll((long long)fq) - 1, ll = __ffsll((long long)lq) - 1;
-                    fq &= fq - 1ull;
-                    lq &= lq - 1ull;
-                    s_start[g] = __builtin_amdgcn_readlane(sb[0], lf);
-                    tot_s += __builtin_amdgcn_readlane(s_hi, ll) - s_start[g];
-                    o_start[g] = __builtin_amdgcn_readlane(ob[0], lf);
-                    tot_o += __builtin_amdgcn_readlane(o_hi, ll) - o_start[g];
-                }
-            }
-            s_off[kSandSegs] = tot_s;
-            o_off[kSandSegs] = tot_o;
-        }
-        // uniform
-        const bool staged = nseg <= kSandSegs && tot_s <= kSandStage && tot_o <= kSandStage;
-        if (staged) {
-            for (int q = lane; q < tot_s; q += 64) {
-                int j = q - s_off[0] + s_start[0];
-#pragma unroll
-                for (int g = 1; g < kSandSegs; ++g)
-                    if (q >= s_off[g]) j = q - s_off[g] + s_start[g];
-                const float4 p = xs[j];
-                SS[3 * q] = p.x;
-                SS[3 * q + 1] = p.y;
-                SS[3 * q + 2] = p.z;
-            }
-            for (int q = lane; q < tot_o; q += 64) {
-                int j = q - o_off[0] + o_start[0];
-#pragma unroll
-                for (int g = 1; g < kSandSegs; ++g)
-                    if (q >= o_off[g]) j = q - o_off[g] + o_start[g];
-                const float4 p = solid[j];
-                SO[3 * q] = p.x;
-                SO[3 * q + 1] = p.y;
-                SO[3 * q + 2] = p.z;
-            }
-            wave_lds_sync();
-            // this lane's run: LDS place of slot j is j + ls (sand), j + lo (solid)
-            const int seg = __popcll(fm & (below | (1ull << lane))) - 1;
-            int ls = s_off[0] - s_start[0], lo = o_off[0] - o_start[0];
-#pragma unroll
-            for (int g = 1; g < kSandSegs; ++g)
-                if (seg == g) {
-                    ls = s_off[g] - s_start[g];
-                    lo = o_off[g] - o_start[g];
-                }
+    for (int pass = 0; pass < 2; ++pass) {
+        // Slots ascend in scan order, so the pushed entries (sand j < i) are
+        // those of rows 0 to 3 and the first ones of row 4.  With solids:
+        // steps 0 to 4 take the sand below i of rows 0 to 4, steps 5 to 8 the
+        // solids of rows 0 to 3, steps 9 to 13 rows 4 to 8 (cell by cell, the
+        // solids and the sand from i on).  Without: the nine rows.
+#pragma unroll 1
+        for (int st = 0; st < (kSolid ? 14 : 9); ++st) {
+            const int r = (kSolid && st >= 5) ? st - 5 : st;
+            const bool want_s = !kSolid || st < 5 || st >= 9, want_o = kSolid && st >= 5;
+            const int y = r / 3 - 1, x = r % 3 - 1;
+            const bool valid = act && y >= yl && y <= yu && x >= xl && x <= xu;
+            const int row = valid ? (yy + y) * k.gXZ + (xx + x) * k.gZ + zz + zl : 0;
+            // the lane's windows in both tables (the row's z cells are
+            // consecutive)
+            int s_lo = 0, s_hi = 0, o_lo = 0, o_hi = 0;
             if (valid) {
+                if (want_s) {
+                    s_lo = scs[row];
+                    s_hi = scs[row + nz];
+                }
+                if (want_o) {
+                    o_lo = ocs[row];
+                    o_hi = ocs[row + nz];
+                }
+            }
+            // runs of lanes whose row lies in one cell column (their windows
+            // ascend with the slot)
+            const int col = valid ? (yy + y) * k.gX + (xx + x) : -1;
+            const int pcol = __shfl_up(col, 1, 64);
+            const int ncol = __shfl_down(col, 1, 64);
+            const unsigned long long fm = __ballot(valid && (lane == 0 || pcol != col));
+            const unsigned long long lm = __ballot(valid && (lane == 63 || ncol != col));
+            const int nseg = __popcll(fm);
+            if (nseg == 0) continue;  // uniform: no lane has this row
+            // the runs' sand and solid ranges, packed in LDS at offsets s_off / o_off
+            int s_start[kSandSegs], s_off[kSandSegs + 1], o_start[kSandSegs], o_off[kSandSegs + 1];
+            int tot_s = 0, tot_o = 0;
+            {
+                unsigned long long fq = fm, lq = lm;
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    if (q >= nz) break;
-                    // each cell's solids then sand slots, 32 candidates a mask
-                    for (int t0 = ob[q]; t0 < ob[q + 1]; t0 += 32) {
-                        const int cn = ob[q + 1] - t0 < 32 ? ob[q + 1] - t0 : 32;
-                        unsigned int m = sand_hits32(me, SO + 3 * (t0 + lo), cn, k.h2);
-                        if (!fill) {
-                            h.n2 += __popc(m);
-                            continue;
+                for (int g = 0; g < kSandSegs; ++g) {
+                    s_off[g] = tot_s;
+                    o_off[g] = tot_o;
+                    s_start[g] = 0;
+                    o_start[g] = 0;
+                    if (g < nseg) {
+                        const int lf = __ffsll((long long)fq) - 1, ll = __ffsll((long long)lq) - 1;
+                        fq &= fq - 1ull;
+                        lq &= lq - 1ull;
+                        s_start[g] = __builtin_amdgcn_readlane(s_lo, lf);
+                        tot_s += __builtin_amdgcn_readlane(s_hi, ll) - s_start[g];
+                        if (kSolid) {
+                            o_start[g] = __builtin_amdgcn_readlane(o_lo, lf);
+                            tot_o += __builtin_amdgcn_readlane(o_hi, ll) - o_start[g];
                         }
-                        for (; m; m &= m - 1u) h.solid(t0 + __builtin_ctz(m), n, fill, idx);
-                    }
-                    for (int t0 = sb[q]; t0 < sb[q + 1]; t0 += 32) {
-                        const int cn = sb[q + 1] - t0 < 32 ? sb[q + 1] - t0 : 32;
-                        unsigned int m = sand_hits32(me, SS + 3 * (t0 + ls), cn, k.h2);
-                        if (!fill) {
-                            // part 1: slots below i (if i receives pushes); part
-                            // 2: the rest, and i itself once more
-                            const int below_i = i - t0;  // candidates of this mask below slot i
-                            const unsigned int lowm =
-                                below_i <= 0 ? 0u : (below_i >= 32 ? ~0u : (1u << below_i) - 1u);
-                            const bool sym = i < k.sym_limit;
-                            h.n1 += sym ? __popc(m & lowm) : 0;
-                            h.n2 += __popc(m & ~lowm);
-                            if (sym && below_i >= 0 && below_i < 32 && ((m >> below_i) & 1u)) ++h.n2;
-                            continue;
-                        }
-                        for (; m; m &= m - 1u) h.sand(t0 + __builtin_ctz(m), i, fill, idx, k);
                     }
                 }
             }
-            wave_lds_sync();  // the next row's staging overwrites this one's
-        } else if (valid) {
+            // uniform: every window is empty (the totals cover every run only
+            // when there are at most kSandSegs)
+            if (nseg <= kSandSegs && tot_s == 0 && tot_o == 0) continue;
+            // uniform
+            const bool staged = nseg <= kSandSegs && tot_s <= kSandStage && tot_o <= kSandStage;
+            // the sand this step takes of the window: [t_lo, t_hi)
+            int t_lo = s_lo, t_hi = s_hi;
+            if (kSolid && st < 5) {
+                if (t_hi > ii) t_hi = ii;
+                if (!sym) t_hi = t_lo;
+            } else if ((kSolid || !sym) && t_lo < ii) {
+                t_lo = ii;
+            }
+            int ls = 0, lo = 0;  // LDS place of slot j: j + ls (sand), j + lo (solid)
+            if (staged) {
+                for (int q = lane; q < tot_s; q += 64) {
+                    int j = q - s_off[0] + s_start[0];
+                    if (nseg > 1) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                if (q >= nz) break;
-                // candidates four at a time: the four loads are requested
-                // together, then tested in slot order (the last candidate of
-                // the cell stands in for places past its end)
-                if (solid) {
-                    const int je = ob[q + 1];
-                    for (int j0 = ob[q]; j0 < je; j0 += 4) {
+                        for (int g = 1; g < kSandSegs; ++g)
+                            if (q >= s_off[g]) j = q - s_off[g] + s_start[g];
+                    }
+                    const float4 p = xs[j];
+                    SS[3 * q] = p.x;
+                    SS[3 * q + 1] = p.y;
+                    SS[3 * q + 2] = p.z;
+                }
+                if (kSolid)
+                    for (int q = lane; q < tot_o; q += 64) {
+                        int j = q - o_off[0] + o_start[0];
+                        if (nseg > 1) {
+#pragma unroll
+                            for (int g = 1; g < kSandSegs; ++g)
+                                if (q >= o_off[g]) j = q - o_off[g] + o_start[g];
+                        }
+                        const float4 p = solid[j];
+                        SO[3 * q] = p.x;
+                        SO[3 * q + 1] = p.y;
+                        SO[3 * q + 2] = p.z;
+                    }
+                wave_lds_sync();
+                ls = s_off[0] - s_start[0];
+                lo = o_off[0] - o_start[0];
+                if (nseg > 1) {  // uniform
+                    const int seg = __popcll(fm & upto) - 1;
+#pragma unroll
+                    for (int g = 1; g < kSandSegs; ++g)
+                        if (seg == g) {
+                            ls = s_off[g] - s_start[g];
+                            lo = o_off[g] - o_start[g];
+                        }
+                }
+            }
+            if (valid) {
+                // sand slots [a, b) / solids [a, b), in order
+                auto sands = [&](int a, int b) {
+                    if (staged) {
+                        for (int t0 = a; t0 < b; t0 += 32) {
+                            unsigned int m = sand_hits32(me, SS + 3 * (t0 + ls), b - t0 < 32 ? b - t0 : 32, k.h2);
+                            for (; m; m &= m - 1u) w.push(t0 + __builtin_ctz(m));
+                        }
+                        return;
+                    }
+                    // four loads requested together, then tested in slot order
+                    // (the last candidate stands in for places past the end)
+                    for (int j0 = a; j0 < b; j0 += 4) {
                         float4 p4[4];
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) p4[u] = solid[j0 + u < je ? j0 + u : je - 1];
+                        for (int u = 0; u < 4; ++u) p4[u] = xs[j0 + u < b ? j0 + u : b - 1];
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
-                            if (j0 + u < je && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) h.solid(j0 + u, n, fill, idx);
+                            if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(j0 + u);
+                    }
+                };
+                auto solids = [&](int a, int b) {
+                    if (staged) {
+                        for (int t0 = a; t0 < b; t0 += 32) {
+                            unsigned int m = sand_hits32(me, SO + 3 * (t0 + lo), b - t0 < 32 ? b - t0 : 32, k.h2);
+                            for (; m; m &= m - 1u) w.push(n + t0 + __builtin_ctz(m));
+                        }
+                        return;
+                    }
+                    for (int j0 = a; j0 < b; j0 += 4) {
+                        float4 p4[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) p4[u] = solid[j0 + u < b ? j0 + u : b - 1];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(n + j0 + u);
+                    }
+                };
+                if (!kSolid || st < 5 || (nseg <= kSandSegs && tot_o == 0)) {  // uniform: sand only
+                    sands(t_lo, t_hi);
+                } else if (st < 9) {
+                    solids(o_lo, o_hi);
+                } else {
+                    // cell by cell: its solids, then its sand
+                    int so = o_lo, ss = s_lo;
+#pragma unroll 1
+                    for (int q = 1; q <= nz; ++q) {
+                        const int eo = ocs[row + q], es = scs[row + q];
+                        solids(so, eo);
+                        sands(ss < t_lo ? t_lo : ss, es < t_hi ? es : t_hi);
+                        so = eo;
+                        ss = es;
                     }
                 }
-                const int je = sb[q + 1];
-                for (int j0 = sb[q]; j0 < je; j0 += 4) {
-                    float4 p4[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) p4[u] = xs[j0 + u < je ? j0 + u : je - 1];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (j0 + u < je && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) h.sand(j0 + u, i, fill, idx, k);
-                }
             }
+            if (staged) wave_lds_sync();  // the next step's staging overwrites this one's
         }
+        if (act && w.lim > 0) w.finish(ii);
+        if (pass == 1) break;
+        big = act && w.c > room;
+        if (__ballot(big) == 0ull) break;  // uniform: every list fits its place
+        // room in the pool for the long ones; without it (the host looks at
+        // what was asked for) the list stays empty
+        const int need = (w.c + 3) >> 2;
+        unsigned long long at = 0ull;
+        if (big) at = atomicAdd(&L.ctl[1], (unsigned long long)need);
+        const bool got = big && at + (unsigned long long)need <= (unsigned long long)L.pool_groups;
+        base = got ? (int)at : -1;
+        w.lim = got ? 4 * need : 0;
+        w.stride = 1;
+        w.lst = got ? L.pool + at : L.pool;
+        if (__ballot(got) == 0ull) break;  // uniform
+        w.c = 0;
     }
-    if (!fill && act) {
-        cnt[i] = h.n1 + h.n2;
-        cnt1[i] = h.n1;
-    }
+    if (act) L.hdr[i] = big ? make_int2(base < 0 ? 0 : w.c, base < 0 ? 0 : base) : make_int2(w.c, 0);
+    // the lists' total length as the reference counts them (slot i twice when
+    // it receives pushes)
+    const float sx = me.x - me.x, sy = me.y - me.y, sz = me.z - me.z;
+    const bool self = (__float_as_uint(k.h2 - dot3(sx, sy, sz, sx, sy, sz)) >> 31) == 0u;
+    int mine = act ? w.c + ((sym && self) ? 1 : 0) : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+    if (lane == 0) atomicAdd(&block_total, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&L.ctl[0], (unsigned long long)block_total);
 }
 
-hipError_t launch_sand_nbr(const float4* xs, const int* key2, const int* sand_cs, int n,
-                           const float4* solid, const int* solid_cs, SandK k, const int* off,
-                           int* cnt, int* cnt1, int* idx, int fill, hipStream_t s, long cap, int* fail) {
-    launch_kernel(k_sand_nbr, dim3(grid_for(n)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid,
-                       solid_cs, k, off, cnt, cnt1, idx, fill, cap, fail);
+hipError_t launch_sand_lists(const float4* xs, const int* key2, const int* sand_cs, int n, const float4* solid,
+                             const int* solid_cs, SandK k, SandLists L, hipStream_t s) {
+    if (solid)
+        launch_kernel(k_sand_lists<true>, dim3(grid_for(n)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid,
+                      solid_cs, k, L);
+    else
+        launch_kernel(k_sand_lists<false>, dim3(grid_for(n)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid,
+                      solid_cs, k, L);
+    return hipGetLastError();
+}
+
+// The lists as the reference holds them (slot i twice when it receives pushes,
+// solids as reference slots), for lus_sand_neighbors: counts, or with off the
+// rows.  n: the slots of the scene at the step; rows [0, rows).
+__global__ __launch_bounds__(kBlock) void k_sand_rows(SandLists L, int n, int rows, int sym_limit,
+                                                      const int* __restrict__ solid_ref,
+                                                      const int* __restrict__ off, int* __restrict__ out) {
+    const int i = xcd_index();
+    if (i >= rows) return;
+    const int2 h = L.hdr[i];
+    int stride;
+    const int4* __restrict__ lst = sand_list(L, i, h, stride);
+    int o = off ? off[i] : 0;
+    for (int t = 0; t < h.x; ++t) {
+        const int j = reinterpret_cast<const int*>(lst + (size_t)(t >> 2) * stride)[t & 3];
+        const int times = (j == i && i < sym_limit) ? 2 : 1;
+        for (int u = 0; u < times; ++u, ++o)
+            if (off) out[o] = j < n ? j : solid_ref[j - n];
+    }
+    if (!off) out[i] = o;
+}
+
+hipError_t launch_sand_rows(SandLists L, int n, int rows, int sym_limit, const int* solid_ref, const int* off,
+                            int* out, hipStream_t s) {
+    launch_kernel(k_sand_rows, dim3(grid_for(rows)), dim3(kBlock), 0, s, L, n, rows, sym_limit, solid_ref, off, out);
     return hipGetLastError();
 }
 
@@ -1087,10 +1177,12 @@ __device__ __forceinline__ void sand_walls_v3(const float4 q, const SandK& k, fl
 }
 
 // One Jacobi substep of contact + friction (src/Simulate.cpp:228-308).  The
-// list is walked four entries at a time (their indices and positions all
-// requested before the four are tested; places past the list end read slot
-// i, in bounds and unused), collecting the possible contacts, which a second
-// loop projects in list order.
+// list is walked a group of four at a time (their positions requested
+// together, then the next group's entries, before the four are tested; the
+// last group is filled up with slot i, never a contact), collecting the
+// possible contacts, which a second loop projects in list order.  The last
+// substep also forms the velocity v = (x* - x) / dt (:316-319), which a pass
+// of its own read and wrote 64 B a slot for (11 us at 1M slots).
 //
 // simulate_sand_credits: a particle flagged 2 loses the flag at its first
 // contact (:463-469; the three rand() draws there are not used).
@@ -1099,42 +1191,52 @@ __device__ __forceinline__ void sand_walls_v3(const float4 q, const SandK& k, fl
 // projections of positions_tmp are added and nothing is clamped (:566-616).
 constexpr int kSandContacts = 16;  // contacts of a lane held between its walk and its projection loop
 
+template <bool kSolid>
 __global__ __launch_bounds__(kBlock) void k_sand_substep(const float4* __restrict__ A,
-                                                          const float4* __restrict__ xold,
-                                                          const float4* __restrict__ solid,
-                                                          const int* __restrict__ off,
-                                                          const int* __restrict__ idx, int n,
-                                                          SandK k, float4* __restrict__ B,
-                                                          int* __restrict__ att,
-                                                          const int* __restrict__ fail) {
+                                                         const float4* __restrict__ xold,
+                                                         const float4* __restrict__ solid, SandLists L, int n,
+                                                         SandK k, float4* __restrict__ B, float4* __restrict__ v,
+                                                         float dt, int* __restrict__ att, long cap,
+                                                         int* __restrict__ fail) {
     // the lane's contacts in list order: contact[u * kBlock + thread]
     __shared__ int contact[kSandContacts * kBlock];
-    if (fail && *fail) return;  // the lists were not written (uniform)
     const int i = xcd_index();
     if (i >= n) return;
     const float4 pi = A[i];
     const float4 xoi = xold[i];
+    // a fixed capacity (fail non-null) that the lists exceed: the step is
+    // marked failed and its positions stay as predicted (uniform)
+    const bool over = fail && L.ctl[0] > (unsigned long long)cap;
+    if (over && i == 0) *fail = 1;
     float dpx = 0.0f, dpy = 0.0f, dpz = 0.0f;
     bool contact_any = false;
-    const int t0 = off[i], t1 = off[i + 1];
-    auto at = [&](int j) { return j < n ? A[j] : solid[j - n]; };
+    auto at = [&](int j) {
+        if constexpr (kSolid) return j < n ? A[j] : solid[j - n];
+        return A[j];
+    };
+    int2 h = L.hdr[i];
+    if (over) h.x = 0;
+    int stride;
+    const int4* __restrict__ lst = sand_list(L, i, h, stride);
+    const int ng = (h.x + 3) >> 2;
     // Most neighbours lie beyond d, but over a wave some lane has a contact
     // at almost every step of the walk: the walk only collects the
     // neighbours whose squared length can give a length within d (d2_far),
     // and a second loop, as long as the wave's largest contact count,
     // projects them in list order (the same sums in the same order).
     int nc = 0;
-    for (int t = t0; t < t1; t += 4) {
-        int j[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) j[u] = (t + u < t1) ? idx[t + u] : i;
+    int4 e = make_int4(i, i, i, i);
+    if (ng > 0) e = lst[0];
+    for (int g = 0; g < ng; ++g) {
+        const int j[4] = {e.x, e.y, e.z, e.w};
         float4 pj[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) pj[u] = at(j[u]);
+        e = lst[(size_t)(g + 1 < ng ? g + 1 : g) * stride];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const float ijx = pi.x - pj[u].x, ijy = pi.y - pj[u].y, ijz = pi.z - pj[u].z;
-            if (t + u < t1 && j[u] != i && dot3(ijx, ijy, ijz, ijx, ijy, ijz) <= k.d2_far) {
+            if (j[u] != i && dot3(ijx, ijy, ijz, ijx, ijy, ijz) <= k.d2_far) {
                 if (nc < kSandContacts) contact[nc * kBlock + (int)threadIdx.x] = j[u];
                 ++nc;
             }
@@ -1160,14 +1262,18 @@ __global__ __launch_bounds__(kBlock) void k_sand_substep(const float4* __restric
         }
     } else {
         // more than the buffer holds: every neighbour again
-        for (int t = t0; t < t1; ++t) {
-            const int j = idx[t];
-            if (j != i)
-                contact_any |= sand_pair(pi, xoi, at(j), [&] { return xold[j]; }, j < n, k, dpx, dpy, dpz);
+        for (int g = 0; g < ng; ++g) {
+            const int4 q = lst[(size_t)g * stride];
+            const int j[4] = {q.x, q.y, q.z, q.w};
+            for (int u = 0; u < 4; ++u)
+                if (j[u] != i)
+                    contact_any |= sand_pair(pi, xoi, at(j[u]), [&] { return xold[j[u]]; }, j[u] < n, k, dpx, dpy, dpz);
         }
     }
     float4 r;
-    if (k.variant == 2) {
+    if (over) {
+        r = pi;
+    } else if (k.variant == 2) {
         float wx, wy, wz;
         sand_walls_v3(pi, k, wx, wy, wz);
         r.x = (pi.x + dpx) + wx;
@@ -1180,37 +1286,41 @@ __global__ __launch_bounds__(kBlock) void k_sand_substep(const float4* __restric
     }
     r.w = 0.0f;
     B[i] = r;
+    if (v) v[i] = make_float4((r.x - xoi.x) / dt, (r.y - xoi.y) / dt, (r.z - xoi.z) / dt, 0.0f);
     if (k.variant == 1 && contact_any) {
         const int a = att[i];
         if (a & 2) att[i] = a & ~2;
     }
 }
 
-hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid,
-                               const int* off, const int* idx, int n, SandK k, float4* B, int* att,
-                               hipStream_t s, const int* fail) {
-    launch_kernel(k_sand_substep, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, solid, off,
-                       idx, n, k, B, att, fail);
+hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid, SandLists L, int n, SandK k,
+                               float4* B, float4* v, float dt, int* att, hipStream_t s, long cap, int* fail) {
+    if (solid)
+        launch_kernel(k_sand_substep<true>, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, solid, L, n, k, B, v, dt,
+                      att, cap, fail);
+    else
+        launch_kernel(k_sand_substep<false>, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, solid, L, n, k, B, v, dt,
+                      att, cap, fail);
     return hipGetLastError();
 }
 
-// v = (x* - x) / dt; x = x*  (src/Simulate.cpp:316-319)
-__global__ __launch_bounds__(kBlock) void k_sand_vupdate(const float4* __restrict__ A,
-                                                          float4* __restrict__ x,
-                                                          float4* __restrict__ v, int n,
-                                                          float dt) {
+// the velocity of a step without substeps: v = (x* - x) / dt
+// (src/Simulate.cpp:316-319)
+__global__ __launch_bounds__(kBlock) void k_sand_velocity(const float4* __restrict__ A,
+                                                          const float4* __restrict__ xold,
+                                                          float4* __restrict__ v, int n, float dt, SandLists L,
+                                                          long cap, int* __restrict__ fail) {
     const int i = xcd_index();
     if (i >= n) return;
+    if (i == 0 && fail && L.ctl[0] > (unsigned long long)cap) *fail = 1;
     const float4 a = A[i];
-    const float4 p = x[i];
+    const float4 p = xold[i];
     v[i] = make_float4((a.x - p.x) / dt, (a.y - p.y) / dt, (a.z - p.z) / dt, 0.0f);
-    x[i] = a;
 }
 
-hipError_t launch_sand_vupdate(const float4* A, float4* xold_to_new, float4* vout, int n, float dt,
-                               hipStream_t s) {
-    launch_kernel(k_sand_vupdate, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold_to_new, vout,
-                       n, dt);
+hipError_t launch_sand_velocity(const float4* A, const float4* xold, float4* v, int n, float dt, SandLists L,
+                                hipStream_t s, long cap, int* fail) {
+    launch_kernel(k_sand_velocity, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, v, n, dt, L, cap, fail);
     return hipGetLastError();
 }
 
@@ -1279,34 +1389,28 @@ hipError_t launch_cell_ranges(const int* cs, const int* cells, int n, int2* out,
 // written (two launches), so moves may chain and overlap.
 __global__ __launch_bounds__(kBlock) void k_moves_gather(const int2* __restrict__ mv, int m,
                                                          const float4* __restrict__ a0,
-                                                         const float4* __restrict__ a1,
-                                                         const float4* __restrict__ a2,
-                                                         const int* __restrict__ a3,
+                                                         const float4* __restrict__ a1, const int* __restrict__ a2,
                                                          float4* __restrict__ t0, float4* __restrict__ t1,
-                                                         float4* __restrict__ t2, int* __restrict__ t3) {
+                                                         int* __restrict__ t2) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= m) return;
     const int src = mv[k].y;
     t0[k] = a0[src];
     t1[k] = a1[src];
     t2[k] = a2[src];
-    t3[k] = a3[src];
 }
 
 __global__ __launch_bounds__(kBlock) void k_moves_scatter(const int2* __restrict__ mv, int m,
                                                           float4* __restrict__ a0, float4* __restrict__ a1,
-                                                          float4* __restrict__ a2, int* __restrict__ a3,
-                                                          const float4* __restrict__ t0,
+                                                          int* __restrict__ a2, const float4* __restrict__ t0,
                                                           const float4* __restrict__ t1,
-                                                          const float4* __restrict__ t2,
-                                                          const int* __restrict__ t3) {
+                                                          const int* __restrict__ t2) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= m) return;
     const int dst = mv[k].x;
     a0[dst] = t0[k];
     a1[dst] = t1[k];
     a2[dst] = t2[k];
-    a3[dst] = t3[k];
 }
 
 // Particles inside the player's collision box (Bullet coupling,
@@ -1475,12 +1579,12 @@ hipError_t launch_grid_from_voxels(const unsigned char* vox, int sx, int sy, int
     return hipGetLastError();
 }
 
-hipError_t launch_slot_moves(const int2* mv, int m, float4* a0, float4* a1, float4* a2, int* a3,
-                             float4* t0, float4* t1, float4* t2, int* t3, hipStream_t s) {
+hipError_t launch_slot_moves(const int2* mv, int m, float4* a0, float4* a1, int* a2, float4* t0, float4* t1, int* t2,
+                             hipStream_t s) {
     if (m <= 0) return hipSuccess;
     const dim3 g((m + kBlock - 1) / kBlock), b(kBlock);
-    launch_kernel(k_moves_gather, g, b, 0, s, mv, m, a0, a1, a2, a3, t0, t1, t2, t3);
-    launch_kernel(k_moves_scatter, g, b, 0, s, mv, m, a0, a1, a2, a3, t0, t1, t2, t3);
+    launch_kernel(k_moves_gather, g, b, 0, s, mv, m, a0, a1, a2, t0, t1, t2);
+    launch_kernel(k_moves_scatter, g, b, 0, s, mv, m, a0, a1, a2, t0, t1, t2);
     return hipGetLastError();
 }
 
