@@ -753,13 +753,16 @@ __device__ __forceinline__ bool sand_within(const float4 me, float qx, float qy,
 // candidate to the first, so one funnel shift replaces compare and branch.
 __device__ __forceinline__ unsigned int sand_hits32(const float4 me, const lds_float* __restrict__ b, int cnt,
                                                     float h2) {
-    unsigned int o = ~0u;  // outside bits; ones above bit cnt - 1
-    for (int t = cnt - 1; t >= 0; --t) {
-        const lds_float* __restrict__ p = b + 3 * t;
-        const float dx = me.x - p[0], dy = me.y - p[1], dz = me.z - p[2];
-        o = __builtin_amdgcn_alignbit(o, __float_as_uint(h2 - dot3(dx, dy, dz, dx, dy, dz)), 31u);
+    unsigned int o = 0u;  // outside bits
+    for (int t = (cnt + 3) & ~3; t > 0; t -= 4) {
+        const lds_float* __restrict__ p = b + 3 * (t - 4);
+#pragma unroll
+        for (int u = 3; u >= 0; --u) {
+            const float dx = me.x - p[3 * u], dy = me.y - p[3 * u + 1], dz = me.z - p[3 * u + 2];
+            o = __builtin_amdgcn_alignbit(o, __float_as_uint(h2 - dot3(dx, dy, dz, dx, dy, dz)), 31u);
+        }
     }
-    return ~o;
+    return ~o & (~0u >> (32 - cnt));
 }
 
 // A slot's list as its scan finds it: the last four entries, stored as a
@@ -799,7 +802,7 @@ __global__ __launch_bounds__(kBlock) void k_sand_lists(const float4* __restrict_
                                                        const float4* __restrict__ solid,
                                                        const int* __restrict__ ocs, SandK k, SandLists L) {
     // per wave: the staged sand (and solid) ranges of a row
-    __shared__ float stage[kBlock / 64][kSolid ? 2 : 1][3 * kSandStage];
+    __shared__ float stage[kBlock / 64][kSolid ? 2 : 1][3 * (kSandStage + 3)];
     __shared__ int block_total;
     if (threadIdx.x == 0) block_total = 0;
     __syncthreads();
