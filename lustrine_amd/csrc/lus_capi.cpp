@@ -162,7 +162,7 @@ struct PbfState {
     lus::PbfK k{};
     int n = 0, C = 0;
     Arena mem;
-    float* stage = nullptr;  // 6 n floats: packed positions and velocities for downloads
+    float* stage = nullptr;  // 7 n words: a download's packed arrays
     float4 *x = nullptr, *x2 = nullptr, *v = nullptr, *v2 = nullptr, *xa = nullptr, *xl = nullptr,
            *xp = nullptr;
     int *id = nullptr, *id2 = nullptr, *key = nullptr, *slot = nullptr, *tmp = nullptr,
@@ -252,7 +252,7 @@ struct SandState {
     int list_n = 0;    // sand slots when the lists were built
     int* qbuf = nullptr;  // one int: cell-box count
     int* err = nullptr;   // one int: a simulate_sand_v3 prediction left the grid
-    float* stage = nullptr;  // 6 n floats: packed positions and velocities for downloads
+    float* stage = nullptr;  // 8 n words: a download's packed arrays
     bool stepped = false;
     // fixed index-buffer capacity (lus_sand_set_list_capacity): the step
     // enqueues without waiting; *fail marks a step whose lists did not fit
@@ -289,12 +289,14 @@ struct LusGpu {
     NetState net;
     SandState sand;
     lus::FluidState* fluid = nullptr;      // simulate_fluid state (lus_fluid.hip)
+    lus::HostPull* pull = nullptr;         // pinned memory of downloads (lus_pull.cpp)
     std::vector<LusMlpTrainer*> trainers;  // live trainers, detached on destroy
 };
 
 int lus::ctx_device(const LusGpu* c) { return c->device; }
 hipStream_t lus::ctx_stream(const LusGpu* c) { return c->stream; }
 lus::FluidState*& lus::ctx_fluid(LusGpu* c) { return c->fluid; }
+lus::HostPull*& lus::ctx_pull(LusGpu* c) { return c->pull; }
 
 // A trainer belongs to one context.  Destroying the context first frees the
 // trainer's device memory and detaches it (ctx = nullptr): later calls on it
@@ -692,6 +694,7 @@ int lus_gpu_create(LusGpu** out, int device) {
         delete c;
         return set_error(LUS_EHIP, "hipStreamCreateWithFlags: %s", hipGetErrorString(e));
     }
+    lus::pull_prepare(c->pull);
     *out = c;
     return LUS_OK;
 }
@@ -715,6 +718,8 @@ void lus_gpu_destroy(LusGpu* c) {
     c->sand.pool_mem.release();
     lus::fluid_free(c->fluid);
     c->fluid = nullptr;
+    lus::pull_free(c->pull);
+    c->pull = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1297,26 +1302,35 @@ int lus_pbf_download(LusGpu* c, int order, float* pos, float* vel, int* ids) {
     if (!c || !c->pbf.ready) return set_error(LUS_ESTATE, "lus_pbf_download: no PBF scene");
     PbfState& P = c->pbf;
     LUS_HIP(hipSetDevice(c->device));
-    LUS_HIP(hipStreamSynchronize(c->stream));
     if (order != 0 && order != 1) return set_error(LUS_EINVAL, "lus_pbf_download: order must be 0 or 1");
     const int n = P.n;
     hipStream_t s = c->stream;
     // vec3 rows packed (and for order 1 put back in input order by id) on
-    // the device: each array is one copy into the caller's memory
-    if ((pos || vel) && !P.stage) LUS_HIP(P.mem.alloc(&P.stage, 6 * (size_t)n));
-    const int* by = order == 1 ? P.id : nullptr;
+    // the device, one block for all arrays
+    if (!P.stage) LUS_HIP(P.mem.alloc(&P.stage, 7 * (size_t)n));
+    lus::PackArgs pk{};
+    lus::HostPiece pc[3];
+    int np = 0;
+    float* at = P.stage;
+    pk.by = order == 1 ? P.id : nullptr;
     if (pos) {
-        LUS_HIP(lus::launch_pack3(P.x, by, n, P.stage, s));
-        LUS_HIP(hipMemcpyAsync(pos, P.stage, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s));
+        pk.f[0] = {P.x, at, 0, n};
+        pc[np++] = {pos, nullptr, sizeof(float) * 3 * (size_t)n};
+        at += 3 * (size_t)n;
     }
     if (vel) {
-        LUS_HIP(lus::launch_pack3(P.v, by, n, P.stage + 3 * (size_t)n, s));
-        LUS_HIP(hipMemcpyAsync(vel, P.stage + 3 * (size_t)n, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s));
+        pk.f[1] = {P.v, at, 0, n};
+        pc[np++] = {vel, nullptr, sizeof(float) * 3 * (size_t)n};
+        at += 3 * (size_t)n;
     }
-    if (ids && order == 0) LUS_HIP(hipMemcpyAsync(ids, P.id, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-    LUS_HIP(hipStreamSynchronize(s));
-    if (ids && order == 1)
-        for (int r = 0; r < n; ++r) ids[r] = r;
+    if (ids && order == 0) {
+        pk.i[0] = {P.id, reinterpret_cast<int*>(at), n};
+        pc[np++] = {ids, nullptr, sizeof(int) * (size_t)n};
+    }
+    if (np) LUS_HIP(lus::launch_pack(pk, n, s));
+    const bool iota = ids && order == 1;
+    LUS_HIP(lus::pull_to_host(c, P.stage, pc, np, iota ? ids : nullptr, iota ? n : 0));
+    if (!np) LUS_HIP(hipStreamSynchronize(s));
     return LUS_OK;
 }
 
@@ -2272,25 +2286,41 @@ int lus_sand_download(LusGpu* c, float* pos, float* pos_star, float* vel, int* a
     LUS_HIP(hipSetDevice(c->device));
     hipStream_t s = c->stream;
     const int n = S.n;
-    // vec3 rows are packed on the device and each array is one copy into the
-    // caller's memory; the stream is waited for once
-    if ((pos || pos_star || vel) && !S.stage) LUS_HIP(S.mem.alloc(&S.stage, 6 * (size_t)n));
+    // the arrays are packed on the device into one block; positions_star
+    // equals positions after a step (src/Simulate.cpp:316-319) and before the
+    // first one (both are the uploaded positions)
+    if (!S.stage) LUS_HIP(S.mem.alloc(&S.stage, 8 * (size_t)n));
+    lus::PackArgs pk{};
+    lus::HostPiece pc[4];
+    int np = 0;
+    float* at = S.stage;
     if (pos || pos_star) {
-        LUS_HIP(lus::launch_pack3(S.x, nullptr, n, S.stage, s));
-        LUS_HIP(hipMemcpyAsync(pos ? pos : pos_star, S.stage, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s));
+        pk.f[0] = {S.x, at, 0, n};
+        pc[np++] = {pos ? pos : pos_star, pos ? pos_star : nullptr, sizeof(float) * 3 * (size_t)n};
+        at += 3 * (size_t)n;
     }
     if (vel) {
-        LUS_HIP(lus::launch_pack3(S.v, nullptr, n, S.stage + 3 * (size_t)n, s));
-        LUS_HIP(hipMemcpyAsync(vel, S.stage + 3 * (size_t)n, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s));
+        pk.f[1] = {S.v, at, 0, n};
+        pc[np++] = {vel, nullptr, sizeof(float) * 3 * (size_t)n};
+        at += 3 * (size_t)n;
     }
-    if (attracted) LUS_HIP(hipMemcpyAsync(attracted, S.att, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-    if (perm) LUS_HIP(hipMemcpyAsync(perm, S.perm, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-    LUS_HIP(hipStreamSynchronize(s));
-    if (int r = sand_check(c)) return r;
-    // positions_star equals positions after a step (src/Simulate.cpp:316-319)
-    // and before the first one (both are the uploaded positions)
-    if (pos && pos_star) memcpy(pos_star, pos, sizeof(float) * 3 * (size_t)n);
-    return LUS_OK;
+    int* q = reinterpret_cast<int*>(at);
+    if (attracted) {
+        pk.i[0] = {S.att, q, n};
+        pc[np++] = {attracted, nullptr, sizeof(int) * (size_t)n};
+        q += n;
+    }
+    if (perm) {
+        pk.i[1] = {S.perm, q, n};
+        pc[np++] = {perm, nullptr, sizeof(int) * (size_t)n};
+    }
+    if (np && n > 0) {
+        LUS_HIP(lus::launch_pack(pk, n, s));
+        LUS_HIP(lus::pull_to_host(c, S.stage, pc, np));
+    } else {
+        LUS_HIP(hipStreamSynchronize(s));
+    }
+    return sand_check(c);
 }
 
 // get_cell_indices (src/neighbors/Utils.hpp:13-21): clamp to

@@ -69,6 +69,7 @@ struct FluidState {
     float4* xs2 = nullptr;    // the sweep's output; swapped with xs after it
     int* ctl = nullptr;       // see kCtl*
     int* host_ctl = nullptr;  // pinned mirror of ctl
+    float* stage = nullptr;   // a download's packed arrays
 };
 
 constexpr int kCtlTicket = 0;    // next block of the sweep
@@ -896,24 +897,37 @@ int lus_fluid_download(LusGpu* c, float* positions, float* positions_star, float
     if (!F) return lus::report_error(LUS_ESTATE, "lus_fluid_download: lus_fluid_init first");
     hipStream_t s = lus::ctx_stream(c);
     FL_HIP(hipSetDevice(lus::ctx_device(c)));
-    std::vector<float4> h((size_t)F->total);
-    auto pull = [&](const float4* src, float* dst, int a, int b) -> hipError_t {
-        if (!dst) return hipSuccess;
-        hipError_t e = hipMemcpyAsync(h.data(), src, sizeof(float4) * F->total, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        for (int i = a; i < b; ++i) {
-            dst[3 * (size_t)i] = h[i].x;
-            dst[3 * (size_t)i + 1] = h[i].y;
-            dst[3 * (size_t)i + 2] = h[i].z;
-        }
-        return hipSuccess;
-    };
-    FL_HIP(pull(F->x, positions, 0, F->total));
-    FL_HIP(pull(F->xs, positions_star, 0, F->total));
-    FL_HIP(pull(F->v, velocities, F->s0, F->s1));
-    if (lambdas && F->k.nl) {
-        FL_HIP(hipMemcpyAsync(lambdas, F->lam, sizeof(float) * F->k.nl, hipMemcpyDeviceToHost, s));
+    // the arrays are packed on the device into one block: positions,
+    // positions_star, the moving slots' velocities, lambdas
+    const int total = F->total, moving = F->s1 - F->s0, nl = F->k.nl;
+    if (!F->stage) FL_HIP(fl_alloc(F, &F->stage, 6 * (size_t)total + 3 * (size_t)moving + (size_t)nl));
+    lus::PackArgs pk{};
+    lus::HostPiece pc[4];
+    int np = 0;
+    float* at = F->stage;
+    if (positions) {
+        pk.f[0] = {F->x, at, 0, total};
+        pc[np++] = {positions, nullptr, sizeof(float) * 3 * (size_t)total};
+        at += 3 * (size_t)total;
+    }
+    if (positions_star) {
+        pk.f[1] = {F->xs, at, 0, total};
+        pc[np++] = {positions_star, nullptr, sizeof(float) * 3 * (size_t)total};
+        at += 3 * (size_t)total;
+    }
+    if (velocities) {
+        pk.f[2] = {F->v, at, F->s0, F->s1};
+        pc[np++] = {velocities + 3 * (size_t)F->s0, nullptr, sizeof(float) * 3 * (size_t)moving};
+        at += 3 * (size_t)moving;
+    }
+    if (lambdas && nl) {
+        pk.i[0] = {reinterpret_cast<const int*>(F->lam), reinterpret_cast<int*>(at), nl};
+        pc[np++] = {lambdas, nullptr, sizeof(float) * (size_t)nl};
+    }
+    if (np) {
+        FL_HIP(lus::launch_pack(pk, std::max(total, nl), s));
+        FL_HIP(lus::pull_to_host(c, F->stage, pc, np));
+    } else {
         FL_HIP(hipStreamSynchronize(s));
     }
     return LUS_OK;

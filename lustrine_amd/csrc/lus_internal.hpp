@@ -90,6 +90,22 @@ int ctx_device(const LusGpu* c);
 hipStream_t ctx_stream(const LusGpu* c);
 FluidState*& ctx_fluid(LusGpu* c);
 
+// ---- downloads (lus_pull.cpp) ----
+// The next `bytes` of a packed device block go to dst (and to also)
+struct HostPiece {
+    void* dst;
+    void* also;
+    size_t bytes;
+};
+// A context's pinned memory for downloads
+struct HostPull;
+void pull_prepare(HostPull*& hp);
+void pull_free(HostPull* hp);
+HostPull*& ctx_pull(LusGpu* c);
+// Waits for the stream's work and copies the block `dev` (np pieces, one after
+// the other) to their places; iota[r] = r for r < n_iota.
+hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np, int* iota = nullptr, int n_iota = 0);
+
 // ---- launchers (lus_kernels.hip); all enqueue on `s` and return hipError_t ----
 // prefix scan of m ints: out[k] = sum in[0..k); zero_in clears `in` after use.
 // tile: the sort tile, ints per scan block (1024, 2048 or 4096); tile_sums
@@ -120,8 +136,23 @@ hipError_t launch_scatter(const int* key, const int* slot, const int* cell_start
 hipError_t launch_stable_rank(const int* tmp, const int* key, const int* cell_start, int n,
                               int* perm, int* key_sorted, hipStream_t s);
 hipError_t launch_gather4(const float4* src, const int* perm, int n, float4* dst, hipStream_t s);
-// dst[3 q .. 3 q + 2] = src[r].xyz, q = ids ? ids[r] : r (ids a permutation of 0..n-1)
-hipError_t launch_pack3(const float4* src, const int* ids, int n, float* dst, hipStream_t s);
+// Packs a download's arrays into one block, in one launch.  f[a]: rows
+// [f_lo, f_hi) of src, row r at dst[3 (q - f_lo)], q = by ? by[r] : r (by a
+// permutation of 0..n-1); i[a]: n ints copied.  Unused: src nullptr.
+struct PackArgs {
+    struct Rows {
+        const float4* src;
+        float* dst;
+        int lo, hi;
+    } f[3];
+    struct Ints {
+        const int* src;
+        int* dst;
+        int n;
+    } i[2];
+    const int* by;
+};
+hipError_t launch_pack(const PackArgs& p, int n, hipStream_t s);
 // *out += particles of the neighbour-list buffer nb whose header marks the
 // re-test path (*out must be cleared by the caller)
 // (blk: the block table of block-staged lists, nullptr for flat ones)

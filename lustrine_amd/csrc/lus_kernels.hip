@@ -383,21 +383,28 @@ __global__ __launch_bounds__(kBlock) void k_gather4(const float4* __restrict__ s
     dst[i] = src[perm[i]];
 }
 
-// AoS float[3] rows from float4: row q = ids ? ids[r] : r receives src[r]
-// (the host's vec3 layout, written on the device so a download is one copy)
-__global__ __launch_bounds__(kBlock) void k_pack3(const float4* __restrict__ src, const int* __restrict__ ids,
-                                                   int n, float* __restrict__ dst) {
+// AoS float[3] rows from float4 and the int arrays beside them (the host's
+// layout, written on the device so that a download is one copy and one launch)
+__global__ __launch_bounds__(kBlock) void k_pack(PackArgs p, int n) {
     const int r = xcd_index();
     if (r >= n) return;
-    const float4 a = src[r];
-    const int q = ids ? ids[r] : r;
-    dst[3 * (size_t)q] = a.x;
-    dst[3 * (size_t)q + 1] = a.y;
-    dst[3 * (size_t)q + 2] = a.z;
+    const int q = p.by ? p.by[r] : r;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (!p.f[a].src || r < p.f[a].lo || r >= p.f[a].hi) continue;
+        const float4 v = p.f[a].src[r];
+        float* __restrict__ d = p.f[a].dst + 3 * (size_t)(q - p.f[a].lo);
+        d[0] = v.x;
+        d[1] = v.y;
+        d[2] = v.z;
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+        if (p.i[a].src && r < p.i[a].n) p.i[a].dst[r] = p.i[a].src[r];
 }
 
-hipError_t launch_pack3(const float4* src, const int* ids, int n, float* dst, hipStream_t s) {
-    launch_kernel(k_pack3, dim3(grid_for(n)), dim3(kBlock), 0, s, src, ids, n, dst);
+hipError_t launch_pack(const PackArgs& p, int n, hipStream_t s) {
+    launch_kernel(k_pack, dim3(grid_for(n)), dim3(kBlock), 0, s, p, n);
     return hipGetLastError();
 }
 
