@@ -369,6 +369,15 @@ hipError_t launch_sand_rows(SandLists L, int n, int rows, int sym_limit, const i
 // non-null: lists longer than cap in total set *fail and move nothing
 hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid, SandLists L, int n, SandK k,
                                float4* B, float4* v, float dt, int* att, hipStream_t s, long cap, int* fail);
+// Scenes of at most kSandSubMaxN particles build their lists with four waves
+// per 64 slots and take a substep with four lanes per particle.  us per launch
+// over a solid floor, lists one wave then four, substep one lane then four:
+//     512   40.7 -> 16.3    9.3 ->  5.9
+//     32K   32.3 -> 16.9   10.5 ->  7.1
+//     65K   31.1 -> 25.5   10.9 ->  9.4
+//    110K   32.6 -> 36.2   12.5 -> 13.3
+//    131K   32.7 -> 40.6   12.9 -> 14.4
+constexpr int kSandSubMaxN = 65536;
 hipError_t launch_sand_velocity(const float4* A, const float4* xold, float4* v, int n, float dt, SandLists L,
                                 hipStream_t s, long cap, int* fail);
 

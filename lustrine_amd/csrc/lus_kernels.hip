@@ -732,8 +732,8 @@ hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_s
 // contiguous run of the pool, which its wave scans its stencil a second time
 // to fill.  Counting first and filling exact CSR rows, as before, scanned
 // every stencil twice and left each walk's index loads a line per lane:
-// 1M slots 2 x 118 us + the scan of the counts -> @BUILD@ us, and a substep
-// 77 -> @SUB@ us.
+// 1M slots 2 x 118 us + the scan of the counts -> 79 us, and a substep
+// 77 -> 49 us.
 //
 // Wave-staged: the slots of a wave lie in a few (y, x) cell columns, and
 // within a column their z windows ascend with the slot, so for each stencil
@@ -741,7 +741,7 @@ hipError_t launch_sand_permute(const int* tmp, const int* key, const int* cell_s
 // the sand table and in the solid table.  The wave copies those ranges (x, y,
 // z of each slot) into LDS with coalesced loads and its lanes test their
 // candidates there, in the same order with the same arithmetic; a row whose
-// ranges exceed kSandStage slots or kSandSegs runs is read from global memory.
+// ranges exceed kStage slots or kSandSegs runs is read from global memory.
 // What bounds it is vector issue: the tests, then one trip of the writer per
 // entry of the wave's fullest lane.
 constexpr int kSandStage = 256;
@@ -803,6 +803,268 @@ __device__ __forceinline__ const int4* sand_list(const SandLists& L, int i, int2
     return big ? L.pool + h.y : L.lists + (size_t)(i >> 6) * (64 * (size_t)L.groups) + (i & 63);
 }
 
+// A wave's scan of its 64 slots' stencils, step by step.  Slots ascend in
+// scan order, so the pushed entries (sand j < i) are those of rows 0 to 3 and
+// the first ones of row 4.  With solids: steps 0 to 4 take the sand below i of
+// rows 0 to 4, steps 5 to 8 the solids of rows 0 to 3, steps 9 to 13 rows 4 to
+// 8 (cell by cell, the solids and the sand from i on).  Without: the nine rows.
+// Every lane of the wave takes part in the staging; a lane past n has no rows.
+template <bool kSolid, int kStage>
+struct SandScan {
+    static constexpr int kSteps = kSolid ? 14 : 9;
+    const float4* __restrict__ xs;
+    const int* __restrict__ scs;
+    const float4* __restrict__ solid;
+    const int* __restrict__ ocs;
+    const SandK& k;
+    int n, ii, lane;
+    bool act, sym;
+    lds_float* __restrict__ SS;  // the staged sand and solid ranges of a row
+    lds_float* __restrict__ SO;
+    float4 me;
+    int yy, xx, zz, yl = -1, yu = 1, xl = -1, xu = 1, zl = -1, zu = 1, nz;
+    unsigned long long upto;  // lanes through this one
+
+    __device__ __forceinline__ SandScan(int i, const float4* __restrict__ xs_, const int* __restrict__ key2,
+                                        const int* __restrict__ scs_, int n_, const float4* __restrict__ solid_,
+                                        const int* __restrict__ ocs_, const SandK& k_, lds_float* __restrict__ SS_,
+                                        lds_float* __restrict__ SO_)
+        : xs(xs_), scs(scs_), solid(solid_), ocs(ocs_), k(k_), n(n_), SS(SS_), SO(SO_) {
+        lane = (int)(threadIdx.x & 63);
+        act = i < n;
+        ii = act ? i : n - 1;
+        me = xs[ii];
+        const int c = key2[ii];
+        yy = c / k.gXZ;
+        const int tm = c - yy * k.gXZ;
+        zz = tm % k.gZ;
+        xx = tm / k.gZ;
+        if (yy + yl < 0) yl = 0;
+        if (yy + yu >= k.gY) yu = 0;
+        if (xx + xl < 0) xl = 0;
+        if (xx + xu >= k.gX) xu = 0;
+        if (zz + zl < 0) zl = 0;
+        if (zz + zu >= k.gZ) zu = 0;
+        nz = zu - zl + 1;  // z cells of a row (1 to 3)
+        sym = ii < k.sym_limit;
+        upto = (1ull << lane) | ((1ull << lane) - 1ull);
+    }
+
+    template <class W>
+    __device__ __forceinline__ void step(int st, W& w) const {
+        const int r = (kSolid && st >= 5) ? st - 5 : st;
+        const bool want_s = !kSolid || st < 5 || st >= 9, want_o = kSolid && st >= 5;
+        const int y = r / 3 - 1, x = r % 3 - 1;
+        const bool valid = act && y >= yl && y <= yu && x >= xl && x <= xu;
+        const int row = valid ? (yy + y) * k.gXZ + (xx + x) * k.gZ + zz + zl : 0;
+        // the lane's windows in both tables (the row's z cells are
+        // consecutive)
+        int s_lo = 0, s_hi = 0, o_lo = 0, o_hi = 0;
+        if (valid) {
+            if (want_s) {
+                s_lo = scs[row];
+                s_hi = scs[row + nz];
+            }
+            if (want_o) {
+                o_lo = ocs[row];
+                o_hi = ocs[row + nz];
+            }
+        }
+        // runs of lanes whose row lies in one cell column (their windows
+        // ascend with the slot)
+        const int col = valid ? (yy + y) * k.gX + (xx + x) : -1;
+        const int pcol = __shfl_up(col, 1, 64);
+        const int ncol = __shfl_down(col, 1, 64);
+        const unsigned long long fm = __ballot(valid && (lane == 0 || pcol != col));
+        const unsigned long long lm = __ballot(valid && (lane == 63 || ncol != col));
+        const int nseg = __popcll(fm);
+        if (nseg == 0) return;  // uniform: no lane has this row
+        // the runs' sand and solid ranges, packed in LDS at offsets s_off / o_off
+        int s_start[kSandSegs], s_off[kSandSegs + 1], o_start[kSandSegs], o_off[kSandSegs + 1];
+        int tot_s = 0, tot_o = 0;
+        {
+            unsigned long long fq = fm, lq = lm;
+#pragma unroll
+            for (int g = 0; g < kSandSegs; ++g) {
+                s_off[g] = tot_s;
+                o_off[g] = tot_o;
+                s_start[g] = 0;
+                o_start[g] = 0;
+                if (g < nseg) {
+                    const int lf = __ffsll((long long)fq) - 1, ll = __ffsll((long long)lq) - 1;
+                    fq &= fq - 1ull;
+                    lq &= lq - 1ull;
+                    s_start[g] = __builtin_amdgcn_readlane(s_lo, lf);
+                    tot_s += __builtin_amdgcn_readlane(s_hi, ll) - s_start[g];
+                    if (kSolid) {
+                        o_start[g] = __builtin_amdgcn_readlane(o_lo, lf);
+                        tot_o += __builtin_amdgcn_readlane(o_hi, ll) - o_start[g];
+                    }
+                }
+            }
+        }
+        // uniform: every window is empty (the totals cover every run only
+        // when there are at most kSandSegs)
+        if (nseg <= kSandSegs && tot_s == 0 && tot_o == 0) return;
+        // uniform
+        const bool staged = nseg <= kSandSegs && tot_s <= kStage && tot_o <= kStage;
+        // the sand this step takes of the window: [t_lo, t_hi)
+        int t_lo = s_lo, t_hi = s_hi;
+        if (kSolid && st < 5) {
+            if (t_hi > ii) t_hi = ii;
+            if (!sym) t_hi = t_lo;
+        } else if ((kSolid || !sym) && t_lo < ii) {
+            t_lo = ii;
+        }
+        int ls = 0, lo = 0;  // LDS place of slot j: j + ls (sand), j + lo (solid)
+        if (staged) {
+            for (int q = lane; q < tot_s; q += 64) {
+                int j = q - s_off[0] + s_start[0];
+                if (nseg > 1) {
+#pragma unroll
+                    for (int g = 1; g < kSandSegs; ++g)
+                        if (q >= s_off[g]) j = q - s_off[g] + s_start[g];
+                }
+                const float4 p = xs[j];
+                SS[3 * q] = p.x;
+                SS[3 * q + 1] = p.y;
+                SS[3 * q + 2] = p.z;
+            }
+            if (kSolid)
+                for (int q = lane; q < tot_o; q += 64) {
+                    int j = q - o_off[0] + o_start[0];
+                    if (nseg > 1) {
+#pragma unroll
+                        for (int g = 1; g < kSandSegs; ++g)
+                            if (q >= o_off[g]) j = q - o_off[g] + o_start[g];
+                    }
+                    const float4 p = solid[j];
+                    SO[3 * q] = p.x;
+                    SO[3 * q + 1] = p.y;
+                    SO[3 * q + 2] = p.z;
+                }
+            wave_lds_sync();
+            ls = s_off[0] - s_start[0];
+            lo = o_off[0] - o_start[0];
+            if (nseg > 1) {  // uniform
+                const int seg = __popcll(fm & upto) - 1;
+#pragma unroll
+                for (int g = 1; g < kSandSegs; ++g)
+                    if (seg == g) {
+                        ls = s_off[g] - s_start[g];
+                        lo = o_off[g] - o_start[g];
+                    }
+            }
+        }
+        if (valid) {
+            // sand slots [a, b) / solids [a, b), in order
+            auto sands = [&](int a, int b) {
+                if (staged) {
+                    for (int t0 = a; t0 < b; t0 += 32) {
+                        unsigned int m = sand_hits32(me, SS + 3 * (t0 + ls), b - t0 < 32 ? b - t0 : 32, k.h2);
+                        for (; m; m &= m - 1u) w.push(t0 + __builtin_ctz(m));
+                    }
+                    return;
+                }
+                // four loads requested together, then tested in slot order
+                // (the last candidate stands in for places past the end)
+                for (int j0 = a; j0 < b; j0 += 4) {
+                    float4 p4[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) p4[u] = xs[j0 + u < b ? j0 + u : b - 1];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(j0 + u);
+                }
+            };
+            auto solids = [&](int a, int b) {
+                if (staged) {
+                    for (int t0 = a; t0 < b; t0 += 32) {
+                        unsigned int m = sand_hits32(me, SO + 3 * (t0 + lo), b - t0 < 32 ? b - t0 : 32, k.h2);
+                        for (; m; m &= m - 1u) w.push(n + t0 + __builtin_ctz(m));
+                    }
+                    return;
+                }
+                for (int j0 = a; j0 < b; j0 += 4) {
+                    float4 p4[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) p4[u] = solid[j0 + u < b ? j0 + u : b - 1];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(n + j0 + u);
+                }
+            };
+            if (!kSolid || st < 5 || (nseg <= kSandSegs && tot_o == 0)) {  // uniform: sand only
+                sands(t_lo, t_hi);
+            } else if (st < 9) {
+                solids(o_lo, o_hi);
+            } else {
+                // cell by cell: its solids, then its sand
+                int so = o_lo, ss = s_lo;
+#pragma unroll 1
+                for (int q = 1; q <= nz; ++q) {
+                    const int eo = ocs[row + q], es = scs[row + q];
+                    solids(so, eo);
+                    sands(ss < t_lo ? t_lo : ss, es < t_hi ? es : t_hi);
+                    so = eo;
+                    ss = es;
+                }
+            }
+        }
+        if (staged) wave_lds_sync();  // the next step's staging overwrites this one's
+    }
+
+    // the lists' length of a slot with c entries as the reference counts them
+    // (slot i twice when it receives pushes)
+    __device__ __forceinline__ int length(int c) const {
+        const float sx = me.x - me.x, sy = me.y - me.y, sz = me.z - me.z;
+        const bool self = (__float_as_uint(k.h2 - dot3(sx, sy, sz, sx, sy, sz)) >> 31) == 0u;
+        return act ? c + ((sym && self) ? 1 : 0) : 0;
+    }
+
+    // The whole scan into the lists; the entries of slot i
+    __device__ __forceinline__ int write(const SandLists& L) const {
+        const int room = 4 * L.groups;
+        SandWriter w;
+        w.lim = act ? room : 0;
+        w.stride = 64;
+        w.lst = L.lists + (size_t)(ii >> 6) * (64 * (size_t)L.groups) + (ii & 63);
+        int base = 0;
+        bool big = false;
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll 1
+            for (int st = 0; st < kSteps; ++st) step(st, w);
+            if (act && w.lim > 0) w.finish(ii);
+            if (pass == 1) break;
+            big = act && w.c > room;
+            if (__ballot(big) == 0ull) break;  // uniform: every list fits its place
+            // room in the pool for the long ones; without it (the host looks
+            // at what was asked for) the list stays empty
+            const int need = (w.c + 3) >> 2;
+            unsigned long long at = 0ull;
+            if (big) at = atomicAdd(&L.ctl[1], (unsigned long long)need);
+            const bool got = big && at + (unsigned long long)need <= (unsigned long long)L.pool_groups;
+            base = got ? (int)at : -1;
+            w.lim = got ? 4 * need : 0;
+            w.stride = 1;
+            w.lst = got ? L.pool + at : L.pool;
+            if (__ballot(got) == 0ull) break;  // uniform
+            w.c = 0;
+        }
+        if (act) L.hdr[ii] = big ? make_int2(base < 0 ? 0 : w.c, base < 0 ? 0 : base) : make_int2(w.c, 0);
+        return w.c;
+    }
+};
+
+// the wave sums of the lists' lengths to block_total, that to ctl[0]; a
+// barrier between the two is the caller's
+__device__ __forceinline__ void sand_total(int mine, int* block_total) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(block_total, mine);
+}
+
 template <bool kSolid>
 __global__ __launch_bounds__(kBlock) void k_sand_lists(const float4* __restrict__ xs, const int* __restrict__ key2,
                                                        const int* __restrict__ scs, int n,
@@ -813,245 +1075,94 @@ __global__ __launch_bounds__(kBlock) void k_sand_lists(const float4* __restrict_
     __shared__ int block_total;
     if (threadIdx.x == 0) block_total = 0;
     __syncthreads();
-    const int i = xcd_index();
-    const int lane = (int)(threadIdx.x & 63);
-    // every lane of the wave takes part in the staging; a lane past n has no
-    // rows and writes nothing
-    const bool act = i < n;
-    const int ii = act ? i : n - 1;
-    lds_float* __restrict__ SS = (lds_float*)stage[threadIdx.x >> 6][0];
-    lds_float* __restrict__ SO = (lds_float*)stage[threadIdx.x >> 6][kSolid ? 1 : 0];
-    const float4 me = xs[ii];
-    const int c = key2[ii];
-    const int yy = c / k.gXZ;
-    const int tm = c - yy * k.gXZ;
-    const int zz = tm % k.gZ;
-    const int xx = tm / k.gZ;
-    int yl = -1, yu = 1, xl = -1, xu = 1, zl = -1, zu = 1;
-    if (yy + yl < 0) yl = 0;
-    if (yy + yu >= k.gY) yu = 0;
-    if (xx + xl < 0) xl = 0;
-    if (xx + xu >= k.gX) xu = 0;
-    if (zz + zl < 0) zl = 0;
-    if (zz + zu >= k.gZ) zu = 0;
-    const int nz = zu - zl + 1;  // z cells of a row (1 to 3)
-    const bool sym = ii < k.sym_limit;
-    const unsigned long long upto = (1ull << lane) | ((1ull << lane) - 1ull);  // lanes through this one
-    const int room = 4 * L.groups;
-    SandWriter w;
-    w.lim = act ? room : 0;
-    w.stride = 64;
-    w.lst = L.lists + (size_t)(ii >> 6) * (64 * (size_t)L.groups) + (ii & 63);
-    int base = 0;
-    bool big = false;
-#pragma unroll 1
-    for (int pass = 0; pass < 2; ++pass) {
-        // Slots ascend in scan order, so the pushed entries (sand j < i) are
-        // those of rows 0 to 3 and the first ones of row 4.  With solids:
-        // steps 0 to 4 take the sand below i of rows 0 to 4, steps 5 to 8 the
-        // solids of rows 0 to 3, steps 9 to 13 rows 4 to 8 (cell by cell, the
-        // solids and the sand from i on).  Without: the nine rows.
-#pragma unroll 1
-        for (int st = 0; st < (kSolid ? 14 : 9); ++st) {
-            const int r = (kSolid && st >= 5) ? st - 5 : st;
-            const bool want_s = !kSolid || st < 5 || st >= 9, want_o = kSolid && st >= 5;
-            const int y = r / 3 - 1, x = r % 3 - 1;
-            const bool valid = act && y >= yl && y <= yu && x >= xl && x <= xu;
-            const int row = valid ? (yy + y) * k.gXZ + (xx + x) * k.gZ + zz + zl : 0;
-            // the lane's windows in both tables (the row's z cells are
-            // consecutive)
-            int s_lo = 0, s_hi = 0, o_lo = 0, o_hi = 0;
-            if (valid) {
-                if (want_s) {
-                    s_lo = scs[row];
-                    s_hi = scs[row + nz];
-                }
-                if (want_o) {
-                    o_lo = ocs[row];
-                    o_hi = ocs[row + nz];
-                }
-            }
-            // runs of lanes whose row lies in one cell column (their windows
-            // ascend with the slot)
-            const int col = valid ? (yy + y) * k.gX + (xx + x) : -1;
-            const int pcol = __shfl_up(col, 1, 64);
-            const int ncol = __shfl_down(col, 1, 64);
-            const unsigned long long fm = __ballot(valid && (lane == 0 || pcol != col));
-            const unsigned long long lm = __ballot(valid && (lane == 63 || ncol != col));
-            const int nseg = __popcll(fm);
-            if (nseg == 0) continue;  // uniform: no lane has this row
-            // the runs' sand and solid ranges, packed in LDS at offsets s_off / o_off
-            int s_start[kSandSegs], s_off[kSandSegs + 1], o_start[kSandSegs], o_off[kSandSegs + 1];
-            int tot_s = 0, tot_o = 0;
-            {
-                unsigned long long fq = fm, lq = lm;
-#pragma unroll
-                for (int g = 0; g < kSandSegs; ++g) {
-                    s_off[g] = tot_s;
-                    o_off[g] = tot_o;
-                    s_start[g] = 0;
-                    o_start[g] = 0;
-                    if (g < nseg) {
-                        const int lf = __ffsll((long long)fq) - 1, ll = __ffsll((long long)lq) - 1;
-                        fq &= fq - 1ull;
-                        lq &= lq - 1ull;
-                        s_start[g] = __builtin_amdgcn_readlane(s_lo, lf);
-                        tot_s += __builtin_amdgcn_readlane(s_hi, ll) - s_start[g];
-                        if (kSolid) {
-                            o_start[g] = __builtin_amdgcn_readlane(o_lo, lf);
-                            tot_o += __builtin_amdgcn_readlane(o_hi, ll) - o_start[g];
-                        }
-                    }
-                }
-            }
-            // uniform: every window is empty (the totals cover every run only
-            // when there are at most kSandSegs)
-            if (nseg <= kSandSegs && tot_s == 0 && tot_o == 0) continue;
-            // uniform
-            const bool staged = nseg <= kSandSegs && tot_s <= kSandStage && tot_o <= kSandStage;
-            // the sand this step takes of the window: [t_lo, t_hi)
-            int t_lo = s_lo, t_hi = s_hi;
-            if (kSolid && st < 5) {
-                if (t_hi > ii) t_hi = ii;
-                if (!sym) t_hi = t_lo;
-            } else if ((kSolid || !sym) && t_lo < ii) {
-                t_lo = ii;
-            }
-            int ls = 0, lo = 0;  // LDS place of slot j: j + ls (sand), j + lo (solid)
-            if (staged) {
-                for (int q = lane; q < tot_s; q += 64) {
-                    int j = q - s_off[0] + s_start[0];
-                    if (nseg > 1) {
-#pragma unroll
-                        for (int g = 1; g < kSandSegs; ++g)
-                            if (q >= s_off[g]) j = q - s_off[g] + s_start[g];
-                    }
-                    const float4 p = xs[j];
-                    SS[3 * q] = p.x;
-                    SS[3 * q + 1] = p.y;
-                    SS[3 * q + 2] = p.z;
-                }
-                if (kSolid)
-                    for (int q = lane; q < tot_o; q += 64) {
-                        int j = q - o_off[0] + o_start[0];
-                        if (nseg > 1) {
-#pragma unroll
-                            for (int g = 1; g < kSandSegs; ++g)
-                                if (q >= o_off[g]) j = q - o_off[g] + o_start[g];
-                        }
-                        const float4 p = solid[j];
-                        SO[3 * q] = p.x;
-                        SO[3 * q + 1] = p.y;
-                        SO[3 * q + 2] = p.z;
-                    }
-                wave_lds_sync();
-                ls = s_off[0] - s_start[0];
-                lo = o_off[0] - o_start[0];
-                if (nseg > 1) {  // uniform
-                    const int seg = __popcll(fm & upto) - 1;
-#pragma unroll
-                    for (int g = 1; g < kSandSegs; ++g)
-                        if (seg == g) {
-                            ls = s_off[g] - s_start[g];
-                            lo = o_off[g] - o_start[g];
-                        }
-                }
-            }
-            if (valid) {
-                // sand slots [a, b) / solids [a, b), in order
-                auto sands = [&](int a, int b) {
-                    if (staged) {
-                        for (int t0 = a; t0 < b; t0 += 32) {
-                            unsigned int m = sand_hits32(me, SS + 3 * (t0 + ls), b - t0 < 32 ? b - t0 : 32, k.h2);
-                            for (; m; m &= m - 1u) w.push(t0 + __builtin_ctz(m));
-                        }
-                        return;
-                    }
-                    // four loads requested together, then tested in slot order
-                    // (the last candidate stands in for places past the end)
-                    for (int j0 = a; j0 < b; j0 += 4) {
-                        float4 p4[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) p4[u] = xs[j0 + u < b ? j0 + u : b - 1];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(j0 + u);
-                    }
-                };
-                auto solids = [&](int a, int b) {
-                    if (staged) {
-                        for (int t0 = a; t0 < b; t0 += 32) {
-                            unsigned int m = sand_hits32(me, SO + 3 * (t0 + lo), b - t0 < 32 ? b - t0 : 32, k.h2);
-                            for (; m; m &= m - 1u) w.push(n + t0 + __builtin_ctz(m));
-                        }
-                        return;
-                    }
-                    for (int j0 = a; j0 < b; j0 += 4) {
-                        float4 p4[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) p4[u] = solid[j0 + u < b ? j0 + u : b - 1];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (j0 + u < b && sand_within(me, p4[u].x, p4[u].y, p4[u].z, k)) w.push(n + j0 + u);
-                    }
-                };
-                if (!kSolid || st < 5 || (nseg <= kSandSegs && tot_o == 0)) {  // uniform: sand only
-                    sands(t_lo, t_hi);
-                } else if (st < 9) {
-                    solids(o_lo, o_hi);
-                } else {
-                    // cell by cell: its solids, then its sand
-                    int so = o_lo, ss = s_lo;
-#pragma unroll 1
-                    for (int q = 1; q <= nz; ++q) {
-                        const int eo = ocs[row + q], es = scs[row + q];
-                        solids(so, eo);
-                        sands(ss < t_lo ? t_lo : ss, es < t_hi ? es : t_hi);
-                        so = eo;
-                        ss = es;
-                    }
-                }
-            }
-            if (staged) wave_lds_sync();  // the next step's staging overwrites this one's
-        }
-        if (act && w.lim > 0) w.finish(ii);
-        if (pass == 1) break;
-        big = act && w.c > room;
-        if (__ballot(big) == 0ull) break;  // uniform: every list fits its place
-        // room in the pool for the long ones; without it (the host looks at
-        // what was asked for) the list stays empty
-        const int need = (w.c + 3) >> 2;
-        unsigned long long at = 0ull;
-        if (big) at = atomicAdd(&L.ctl[1], (unsigned long long)need);
-        const bool got = big && at + (unsigned long long)need <= (unsigned long long)L.pool_groups;
-        base = got ? (int)at : -1;
-        w.lim = got ? 4 * need : 0;
-        w.stride = 1;
-        w.lst = got ? L.pool + at : L.pool;
-        if (__ballot(got) == 0ull) break;  // uniform
-        w.c = 0;
+    const SandScan<kSolid, kSandStage> scan(xcd_index(), xs, key2, scs, n, solid, ocs, k,
+                                (lds_float*)stage[threadIdx.x >> 6][0],
+                                (lds_float*)stage[threadIdx.x >> 6][kSolid ? 1 : 0]);
+    sand_total(scan.length(scan.write(L)), &block_total);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&L.ctl[0], (unsigned long long)block_total);
+}
+
+// The lists of a small scene: a block of four waves takes 64 slots, each wave
+// a consecutive part of the scan's steps.  Its hits wait in LDS (kSandSeg per
+// slot and wave) until the parts' counts are known, then go to their places.
+// If a part holds more hits or a list exceeds its place, the first wave scans
+// alone.  Few waves are on the chip, and one wave's chain of 14 steps takes
+// 31 us at any size to 65K.  Times: kSandSubMaxN.
+constexpr int kSandSeg = 23;
+constexpr int kSandSubStage = 160;  // four blocks' LDS per CU
+struct SandSegWriter {
+    int c = 0;
+    int* seg;  // this slot's place t is seg[64 t]
+    __device__ __forceinline__ void push(int j) {
+        if (c < kSandSeg) seg[64 * c] = j;
+        ++c;
     }
-    if (act) L.hdr[i] = big ? make_int2(base < 0 ? 0 : w.c, base < 0 ? 0 : base) : make_int2(w.c, 0);
-    // the lists' total length as the reference counts them (slot i twice when
-    // it receives pushes)
-    const float sx = me.x - me.x, sy = me.y - me.y, sz = me.z - me.z;
-    const bool self = (__float_as_uint(k.h2 - dot3(sx, sy, sz, sx, sy, sz)) >> 31) == 0u;
-    int mine = act ? w.c + ((sym && self) ? 1 : 0) : 0;
+};
+
+template <bool kSolid>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sand_lists_sub(const float4* __restrict__ xs,
+                                                           const int* __restrict__ key2,
+                                                           const int* __restrict__ scs, int n,
+                                                           const float4* __restrict__ solid,
+                                                           const int* __restrict__ ocs, SandK k, SandLists L) {
+    __shared__ float stage[kBlock / 64][kSolid ? 2 : 1][3 * (kSandSubStage + 3)];
+    __shared__ int seg[4][kSandSeg * 64];
+    __shared__ int cnt[4][64];
+    __shared__ int block_total;
+    if (threadIdx.x == 0) block_total = 0;
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int b = (int)blockIdx.x, G = (int)gridDim.x;
+    const int i = ((b % kXcd) * (G / kXcd) + b / kXcd) * 64 + lane;
+    const SandScan<kSolid, kSandSubStage> scan(i, xs, key2, scs, n, solid, ocs, k, (lds_float*)stage[wv][0],
+                                (lds_float*)stage[wv][kSolid ? 1 : 0]);
+    // steps [first, last): a quarter of the rows that hold entries
+    const int first = kSolid ? (wv == 0 ? 0 : (wv == 1 ? 4 : (wv == 2 ? 9 : 11))) : (wv == 0 ? 0 : 2 * wv + 1);
+    const int last = kSolid ? (wv == 0 ? 4 : (wv == 1 ? 9 : (wv == 2 ? 11 : 14))) : 2 * wv + 3;
+    SandSegWriter w;
+    w.seg = seg[wv] + lane;
+#pragma unroll 1
+    for (int st = first; st < last; ++st) scan.step(st, w);
+    cnt[wv][lane] = w.c;
+    __syncthreads();
+    int at = 0, c = 0;
+    bool fits = true;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
-    if (lane == 0) atomicAdd(&block_total, mine);
+    for (int q = 0; q < 4; ++q) {
+        const int cq = cnt[q][lane];
+        if (q < wv) at += cq;
+        c += cq;
+        fits = fits && cq <= kSandSeg;
+    }
+    fits = fits && c <= 4 * L.groups;
+    if (__ballot(scan.act && !fits) != 0ull) {  // the same in every wave
+        if (wv == 0) c = scan.write(L);
+    } else if (scan.act) {
+        int4* __restrict__ lst = L.lists + (size_t)(i >> 6) * (64 * (size_t)L.groups) + lane;
+        auto put = [&](int t, int j) { reinterpret_cast<int*>(lst + (size_t)(t >> 2) * 64)[t & 3] = j; };
+        for (int t = 0; t < w.c; ++t) put(at + t, seg[wv][64 * t + lane]);
+        if (wv == 3)
+            for (int t = c; t & 3; ++t) put(t, i);  // the last group is filled up
+        if (wv == 0) L.hdr[i] = make_int2(c, 0);
+    }
+    if (wv == 0) sand_total(scan.length(c), &block_total);
     __syncthreads();
     if (threadIdx.x == 0) atomicAdd(&L.ctl[0], (unsigned long long)block_total);
 }
 
 hipError_t launch_sand_lists(const float4* xs, const int* key2, const int* sand_cs, int n, const float4* solid,
                              const int* solid_cs, SandK k, SandLists L, hipStream_t s) {
-    if (solid)
-        launch_kernel(k_sand_lists<true>, dim3(grid_for(n)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid,
-                      solid_cs, k, L);
-    else
-        launch_kernel(k_sand_lists<false>, dim3(grid_for(n)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid,
-                      solid_cs, k, L);
+#define LUS_LISTS(K, T) \
+    launch_kernel((K), dim3(grid_for(n, T)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid, solid_cs, k, L)
+    if (n <= kSandSubMaxN) {
+        if (solid) LUS_LISTS(k_sand_lists_sub<true>, 64);
+        else LUS_LISTS(k_sand_lists_sub<false>, 64);
+    } else {
+        if (solid) LUS_LISTS(k_sand_lists<true>, kBlock);
+        else LUS_LISTS(k_sand_lists<false>, kBlock);
+    }
+#undef LUS_LISTS
     return hipGetLastError();
 }
 
@@ -1082,13 +1193,14 @@ hipError_t launch_sand_rows(SandLists L, int n, int rows, int sym_limit, const i
     return hipGetLastError();
 }
 
-// The contact + friction projection of particle (pi, xoi) against a neighbour
-// at pj into dp (src/Simulate.cpp:240-300); xoj_of() gives the neighbour's
-// old position, asked for only for a sand contact.
-// Returns whether the pair is in contact (within the diameter).
+// The contact (t) and friction (f) displacements of particle (pi, xoi) against
+// a neighbour at pj (src/Simulate.cpp:240-300), which dp loses in this order;
+// xoj_of() gives the neighbour's old position, asked for only for a sand
+// contact.  Returns whether the pair is in contact (within the diameter).
 template <class XoJ>
-__device__ __forceinline__ bool sand_pair(const float4 pi, const float4 xoi, const float4 pj, XoJ&& xoj_of,
-                                          bool sand, const SandK& k, float& dpx, float& dpy, float& dpz) {
+__device__ __forceinline__ bool sand_terms(const float4 pi, const float4 xoi, const float4 pj, XoJ&& xoj_of,
+                                           bool sand, const SandK& k, float& tx, float& ty, float& tz, float& fx,
+                                           float& fy, float& fz) {
     float ijx = pi.x - pj.x, ijy = pi.y - pj.y, ijz = pi.z - pj.z;
     // |ij| == 0 -> ij = (0, 1e-5, 0) (src/Simulate.cpp:236-239; not in
     // simulate_sand_v3); the length is computed again only then
@@ -1108,12 +1220,9 @@ __device__ __forceinline__ bool sand_pair(const float4 pi, const float4 xoi, con
     } else {
         sc = k.collision * (len - k.d);
     }
-    const float tx = (sc * ijx) / len;
-    const float ty = (sc * ijy) / len;
-    const float tz = (sc * ijz) / len;
-    dpx = dpx - tx;
-    dpy = dpy - ty;
-    dpz = dpz - tz;
+    tx = (sc * ijx) / len;
+    ty = (sc * ijy) / len;
+    tz = (sc * ijz) / len;
     const float d = sqrtf(dot3(tx, ty, tz, tx, ty, tz));
     float xidx = (pi.x - tx) - xoi.x;
     float xidy = (pi.y - ty) - xoi.y;
@@ -1144,16 +1253,30 @@ __device__ __forceinline__ bool sand_pair(const float4 pi, const float4 xoi, con
     const float xtx = rx - rd * nx, xty = ry - rd * ny, xtz = rz - rd * nz;
     const float lt = sqrtf(dot3(xtx, xty, xtz, xtx, xty, xtz));
     if ((d * k.mu_s) > (lt + 1e-9f)) {
-        dpx = dpx - k.friction * xtx;
-        dpy = dpy - k.friction * xty;
-        dpz = dpz - k.friction * xtz;
+        fx = k.friction * xtx;
+        fy = k.friction * xty;
+        fz = k.friction * xtz;
     } else {
         const float q = (k.mu_k * d) / (lt + 1e-9f);
         const float ratio = q < 1.0f ? q : 1.0f;
-        dpx = dpx - (k.friction * xtx) * ratio;
-        dpy = dpy - (k.friction * xty) * ratio;
-        dpz = dpz - (k.friction * xtz) * ratio;
+        fx = (k.friction * xtx) * ratio;
+        fy = (k.friction * xty) * ratio;
+        fz = (k.friction * xtz) * ratio;
     }
+    return true;
+}
+
+template <class XoJ>
+__device__ __forceinline__ bool sand_pair(const float4 pi, const float4 xoi, const float4 pj, XoJ&& xoj_of,
+                                          bool sand, const SandK& k, float& dpx, float& dpy, float& dpz) {
+    float tx, ty, tz, fx, fy, fz;
+    if (!sand_terms(pi, xoi, pj, xoj_of, sand, k, tx, ty, tz, fx, fy, fz)) return false;
+    dpx = dpx - tx;
+    dpy = dpy - ty;
+    dpz = dpz - tz;
+    dpx = dpx - fx;
+    dpy = dpy - fy;
+    dpz = dpz - fz;
     return true;
 }
 
@@ -1200,6 +1323,33 @@ __device__ __forceinline__ void sand_walls_v3(const float4 q, const SandK& k, fl
 // and give the same bits, so one pass computes them; then the half-space
 // projections of positions_tmp are added and nothing is clamped (:566-616).
 constexpr int kSandContacts = 16;  // contacts of a lane held between its walk and its projection loop
+
+// a substep's result for slot i (over: nothing moves)
+__device__ __forceinline__ void sand_finish(int i, const float4 pi, const float4 xoi, float dpx, float dpy, float dpz,
+                                            bool contact_any, bool over, const SandK& k, float4* __restrict__ B,
+                                            float4* __restrict__ v, float dt, int* __restrict__ att) {
+    float4 r;
+    if (over) {
+        r = pi;
+    } else if (k.variant == 2) {
+        float wx, wy, wz;
+        sand_walls_v3(pi, k, wx, wy, wz);
+        r.x = (pi.x + dpx) + wx;
+        r.y = (pi.y + dpy) + wy;
+        r.z = (pi.z + dpz) + wz;
+    } else {
+        r.x = rclamp(pi.x + dpx, k.r, k.hi[0]);
+        r.y = rclamp(pi.y + dpy, k.r, k.hi[1]);
+        r.z = rclamp(pi.z + dpz, k.r, k.hi[2]);
+    }
+    r.w = 0.0f;
+    B[i] = r;
+    if (v) v[i] = make_float4((r.x - xoi.x) / dt, (r.y - xoi.y) / dt, (r.z - xoi.z) / dt, 0.0f);
+    if (k.variant == 1 && contact_any) {
+        const int a = att[i];
+        if (a & 2) att[i] = a & ~2;
+    }
+}
 
 template <bool kSolid>
 __global__ __launch_bounds__(kBlock) void k_sand_substep(const float4* __restrict__ A,
@@ -1280,37 +1430,136 @@ __global__ __launch_bounds__(kBlock) void k_sand_substep(const float4* __restric
                     contact_any |= sand_pair(pi, xoi, at(j[u]), [&] { return xold[j[u]]; }, j[u] < n, k, dpx, dpy, dpz);
         }
     }
-    float4 r;
-    if (over) {
-        r = pi;
-    } else if (k.variant == 2) {
-        float wx, wy, wz;
-        sand_walls_v3(pi, k, wx, wy, wz);
-        r.x = (pi.x + dpx) + wx;
-        r.y = (pi.y + dpy) + wy;
-        r.z = (pi.z + dpz) + wz;
-    } else {
-        r.x = rclamp(pi.x + dpx, k.r, k.hi[0]);
-        r.y = rclamp(pi.y + dpy, k.r, k.hi[1]);
-        r.z = rclamp(pi.z + dpz, k.r, k.hi[2]);
+    sand_finish(i, pi, xoi, dpx, dpy, dpz, contact_any, over, k, B, v, dt, att);
+}
+
+// The substep of a small scene with four lanes per particle.  65K particles
+// are one wave per SIMD, and a substep takes as long as one wave's chain of
+// loads; here a particle's lanes walk its groups 0, 4, .., 1, 5, .. and its
+// contacts likewise.  The contacts keep their places in list order, and every
+// lane subtracts all displacements in that order (no contact: zero, which
+// leaves dp as it is): the same bits.  Times: kSandSubMaxN.
+__device__ __forceinline__ int quad_bcast(int x, int l) {
+    switch (l) {  // (unrolled: l is a constant)
+        case 0: return __builtin_amdgcn_mov_dpp(x, 0x00, 0xf, 0xf, true);
+        case 1: return __builtin_amdgcn_mov_dpp(x, 0x55, 0xf, 0xf, true);
+        case 2: return __builtin_amdgcn_mov_dpp(x, 0xaa, 0xf, 0xf, true);
+        default: return __builtin_amdgcn_mov_dpp(x, 0xff, 0xf, 0xf, true);
     }
-    r.w = 0.0f;
-    B[i] = r;
-    if (v) v[i] = make_float4((r.x - xoi.x) / dt, (r.y - xoi.y) / dt, (r.z - xoi.z) / dt, 0.0f);
-    if (k.variant == 1 && contact_any) {
-        const int a = att[i];
-        if (a & 2) att[i] = a & ~2;
+}
+__device__ __forceinline__ float quad_bcast(float x, int l) {
+    return __int_as_float(quad_bcast(__float_as_int(x), l));
+}
+
+template <bool kSolid>
+__global__ __launch_bounds__(kBlock) void k_sand_substep_sub(const float4* __restrict__ A,
+                                                             const float4* __restrict__ xold,
+                                                             const float4* __restrict__ solid, SandLists L, int n,
+                                                             SandK k, float4* __restrict__ B, float4* __restrict__ v,
+                                                             float dt, int* __restrict__ att, long cap,
+                                                             int* __restrict__ fail) {
+    // a particle's contacts in list order: contact[u * kBlock / 4 + particle]
+    __shared__ int contact[kSandContacts * kBlock / 4];
+    const int t = xcd_index();
+    const int i = t / 4, sub = t % 4;
+    if (i >= n) return;  // (whole quads)
+    int* __restrict__ mine = contact + (int)threadIdx.x / 4;
+    const float4 pi = A[i];
+    const float4 xoi = xold[i];
+    const bool over = fail && L.ctl[0] > (unsigned long long)cap;
+    if (over && i == 0) *fail = 1;
+    float dpx = 0.0f, dpy = 0.0f, dpz = 0.0f;
+    bool contact_any = false;
+    auto at = [&](int j) {
+        if constexpr (kSolid) return j < n ? A[j] : solid[j - n];
+        return A[j];
+    };
+    // the lane's first group is requested with the header (groups >= 4)
+    int2 h = L.hdr[i];
+    int4 e = L.lists[((size_t)(i >> 6) * (size_t)L.groups + sub) * 64 + (i & 63)];
+    if (over) h.x = 0;
+    int stride;
+    const int4* __restrict__ lst = sand_list(L, i, h, stride);
+    const int ng = (h.x + 3) >> 2;
+    if (stride == 1 && sub < ng) e = lst[sub];
+    int nc = 0;
+    for (int g0 = 0; g0 < ng; g0 += 4) {
+        const int g = g0 + sub;
+        int j[4] = {i, i, i, i};
+        if (g < ng) {
+            j[0] = e.x;
+            j[1] = e.y;
+            j[2] = e.z;
+            j[3] = e.w;
+        }
+        float4 pj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) pj[u] = at(j[u]);
+        if (g + 4 < ng) e = lst[(size_t)(g + 4) * stride];
+        unsigned int m = 0u;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float ijx = pi.x - pj[u].x, ijy = pi.y - pj[u].y, ijz = pi.z - pj[u].z;
+            if (j[u] != i && dot3(ijx, ijy, ijz, ijx, ijy, ijz) <= k.d2_far) m |= 1u << u;
+        }
+        const int mc = __popc(m);
+        const int m0 = quad_bcast(mc, 0), m1 = quad_bcast(mc, 1), m2 = quad_bcast(mc, 2), m3 = quad_bcast(mc, 3);
+        int p = nc + (sub > 0 ? m0 : 0) + (sub > 1 ? m1 : 0) + (sub > 2 ? m2 : 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (m >> u & 1u) {
+                if (p < kSandContacts) mine[p * (kBlock / 4)] = j[u];
+                ++p;
+            }
+        nc += m0 + m1 + m2 + m3;
     }
+    wave_lds_sync();  // the contacts are seen by the particle's other lanes
+    if (nc <= kSandContacts) {
+        for (int u0 = 0; u0 < nc; u0 += 4) {
+            float tx = 0.0f, ty = 0.0f, tz = 0.0f, fx = 0.0f, fy = 0.0f, fz = 0.0f;
+            const int u = u0 + sub;
+            if (u < nc) {
+                const int j = mine[u * (kBlock / 4)];
+                const float4 pj = at(j), xoj = xold[j < n ? j : i];
+                contact_any |= sand_terms(pi, xoi, pj, [&] { return xoj; }, j < n, k, tx, ty, tz, fx, fy, fz);
+            }
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                dpx = dpx - quad_bcast(tx, l);
+                dpy = dpy - quad_bcast(ty, l);
+                dpz = dpz - quad_bcast(tz, l);
+                dpx = dpx - quad_bcast(fx, l);
+                dpy = dpy - quad_bcast(fy, l);
+                dpz = dpz - quad_bcast(fz, l);
+            }
+        }
+    } else if (sub == 0) {
+        // more than the buffer holds: every neighbour again
+        for (int g = 0; g < ng; ++g) {
+            const int4 q = lst[(size_t)g * stride];
+            const int j[4] = {q.x, q.y, q.z, q.w};
+            for (int u = 0; u < 4; ++u)
+                if (j[u] != i)
+                    contact_any |= sand_pair(pi, xoi, at(j[u]), [&] { return xold[j[u]]; }, j[u] < n, k, dpx, dpy, dpz);
+        }
+    }
+    const int any = contact_any ? 1 : 0;
+    contact_any = (quad_bcast(any, 0) | quad_bcast(any, 1) | quad_bcast(any, 2) | quad_bcast(any, 3)) != 0;
+    if (sub == 0) sand_finish(i, pi, xoi, dpx, dpy, dpz, contact_any, over, k, B, v, dt, att);
 }
 
 hipError_t launch_sand_substep(const float4* A, const float4* xold, const float4* solid, SandLists L, int n, SandK k,
                                float4* B, float4* v, float dt, int* att, hipStream_t s, long cap, int* fail) {
-    if (solid)
-        launch_kernel(k_sand_substep<true>, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, solid, L, n, k, B, v, dt,
-                      att, cap, fail);
-    else
-        launch_kernel(k_sand_substep<false>, dim3(grid_for(n)), dim3(kBlock), 0, s, A, xold, solid, L, n, k, B, v, dt,
-                      att, cap, fail);
+#define LUS_SUBSTEP(K, M)                                                                                          \
+    launch_kernel((K), dim3(grid_for((M)*n)), dim3(kBlock), 0, s, A, xold, solid, L, n, k, B, v, dt, att, cap, fail)
+    if (n <= kSandSubMaxN) {
+        if (solid) LUS_SUBSTEP(k_sand_substep_sub<true>, 4);
+        else LUS_SUBSTEP(k_sand_substep_sub<false>, 4);
+    } else {
+        if (solid) LUS_SUBSTEP(k_sand_substep<true>, 1);
+        else LUS_SUBSTEP(k_sand_substep<false>, 1);
+    }
+#undef LUS_SUBSTEP
     return hipGetLastError();
 }
 

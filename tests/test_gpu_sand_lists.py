@@ -108,3 +108,48 @@ def test_no_substeps_keeps_the_prediction(gpu_mod):
     want = x0 + (np.array([sp.gravity[a] for a in range(3)], np.float32) * DT) * DT
     assert np.array_equal(x, want) and np.array_equal(xs, x)
     assert np.array_equal(v, (want - x0) / DT)
+
+
+def _heap(n, seed, spacing=0.9):
+    side = int(np.ceil(n ** (1.0 / 3.0))) + 1
+    lat = scenes.jittered_lattice(side, side, side, cell=spacing, origin=(3.0, 3.0, 3.0), amplitude=0.25, seed=seed)
+    return lat[:n].astype(np.float32)
+
+
+@pytest.mark.parametrize("solids", [False, True])
+@pytest.mark.parametrize("spacing", [0.9, 0.6])
+def test_small_and_large_scene_forms_agree(gpu_mod, solids, spacing):
+    # the same heap alone (four waves per 64 slots, four lanes per particle)
+    # and beside a far layer that takes the scene past the small form's size
+    from lustrine_amd.gpu import sand_params
+
+    box = (200, 60, 200)
+    sol = scenes.lattice(40, 2, 40, origin=(0.0, 0.0, 0.0)) if solids else None
+    heap = _heap(5003, 3, spacing)
+    far = scenes.lattice(180, 2, 200, origin=(60.0, 20.0, 1.0))[:61000]
+    far = far[far[:, 0] < box[0] - 2]
+    far2 = scenes.lattice(130, 2, 190, origin=(62.0, 30.0, 2.0))
+    big = np.concatenate([heap, far, far2]).astype(np.float32)
+    assert len(heap) <= 65536 < len(big)
+    out = []
+    for pos in (heap, big):
+        ns = 0 if sol is None else len(sol)
+        total = max(len(pos) + ns, box[0] * box[1] * box[2])
+        sp = sand_params(*box, kernel_radius_scale=3.1)
+        sp.ptr_solid_start = total - ns
+        index = np.arange(total - 1, total - 1 - ns, -1, dtype=np.int32) if ns else None
+        with gpu_mod.Gpu(0) as g:
+            g.sand_init(sp, pos, None, None, sol, index)
+            g.sand_step(DT, False, False, None)
+            x, _, v, _, perm = g.sand_download()
+            off, idx = g.sand_neighbors()
+        back = np.argsort(perm)  # slot of input particle i
+        lists = []
+        for i in range(len(heap)):
+            row = idx[off[back[i]]:off[back[i] + 1]]
+            # solids by their offset from the top of the reference's slots
+            lists.append(np.where(row < len(pos), perm[np.minimum(row, len(pos) - 1)], row - total))
+        out.append((x[back[:len(heap)]], v[back[:len(heap)]], lists))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    for a, b in zip(out[0][2], out[1][2]):
+        assert np.array_equal(a, b)
