@@ -249,6 +249,10 @@ struct SandState {
         *ocs = nullptr, *solid_ref = nullptr;
     lus::SandLists L{};
     Arena pool_mem;    // L.pool
+    // pinned: L.ctl and err of a waiting step, copied when the lists are built
+    // (listed), so the wait for them does not hold back the substeps
+    unsigned long long* host_ctl = nullptr;
+    hipEvent_t listed = nullptr;
     int list_n = 0;    // sand slots when the lists were built
     int* qbuf = nullptr;  // one int: cell-box count
     int* err = nullptr;   // one int: a simulate_sand_v3 prediction left the grid
@@ -716,6 +720,8 @@ void lus_gpu_destroy(LusGpu* c) {
     c->net.mem.release();
     c->sand.mem.release();
     c->sand.pool_mem.release();
+    if (c->sand.host_ctl) (void)hipHostFree(c->sand.host_ctl);
+    if (c->sand.listed) (void)hipEventDestroy(c->sand.listed);
     lus::fluid_free(c->fluid);
     c->fluid = nullptr;
     lus::pull_free(c->pull);
@@ -1995,6 +2001,8 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
         LUS_HIP(m.alloc(&S.L.hdr, n));
         LUS_HIP(m.alloc(&S.L.lists, ((size_t)n + 63) / 64 * 64 * (size_t)S.L.groups));
         LUS_HIP(m.alloc(&S.L.ctl, 2));
+        if (!S.host_ctl) LUS_HIP(hipHostMalloc((void**)&S.host_ctl, 3 * sizeof(*S.host_ctl), hipHostMallocDefault));
+        if (!S.listed) LUS_HIP(hipEventCreateWithFlags(&S.listed, hipEventDisableTiming));
     }
     LUS_HIP(m.alloc(&S.qbuf, 1));
     LUS_HIP(m.alloc(&S.err, 1));
@@ -2075,8 +2083,8 @@ int sand_pool(SandState& S, long groups) {
 }
 
 // Enqueues one simulate_sand step.  Without a fixed capacity it waits once
-// for the lists' lengths (lists longer than their place size the pool); with
-// one it does not wait, and a step whose lists do not fit is reported by
+// for the lists' lengths (lists longer than their place size the pool), with
+// the substeps enqueued; with one it does not wait, and a step whose lists do not fit is reported by
 // sand_check.  The
 // host-side buffer swaps are applied by sand_after.
 int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
@@ -2094,35 +2102,41 @@ int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
     LUS_HIP(mark(1));
     LUS_HIP(lus::launch_exclusive_scan(S.counts, S.cs, S.C + 1, S.tiles, 1, s));
     LUS_HIP(lus::launch_scatter(S.key, S.slot, S.cs, n, S.tmp, s));
-    LUS_HIP(lus::launch_sand_permute(S.tmp, S.key, S.cs, S.x, S.xs, S.att, n, S.x2, S.A, S.att2, S.perm, S.key2,
-                                     s));
-    for (;;) {
-        LUS_HIP(lus::launch_sand_lists(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, S.L, s));
-        if (fixed) break;  // lists within the capacity fit the pool
-        unsigned long long ctl[2] = {0ull, 0ull};
-        int bad_key = 0;
-        LUS_HIP(hipMemcpyAsync(ctl, S.L.ctl, sizeof(ctl), hipMemcpyDeviceToHost, s));
-        if (k.variant == 2) LUS_HIP(hipMemcpyAsync(&bad_key, S.err, sizeof(int), hipMemcpyDeviceToHost, s));
-        LUS_HIP(hipStreamSynchronize(s));
-        if (bad_key)
-            return set_error(LUS_EINVAL,
-                             "lus_sand_step: a predicted position's cell lies outside the grid (simulate_sand_v3 "
-                             "does not clamp; the reference indexes outside its cell vector there)");
-        if (ctl[0] > (unsigned long long)INT_MAX) return set_error(LUS_EHIP, "lus_sand_step: neighbor count overflow");
-        if (ctl[1] <= (unsigned long long)S.L.pool_groups) break;
-        if (int r = sand_pool(S, (long)(ctl[1] + ctl[1] / 4))) return r;
-        LUS_HIP(lus::launch_zero_ints(reinterpret_cast<int*>(S.L.ctl), 4, s));
-    }
-    LUS_HIP(mark(2));
-    float4* A = S.A;
-    float4* B = S.B;
     // simulate_sand_v3's substeps all read the same positions_tmp: one pass
     const int passes = k.variant == 2 ? (S.p.substeps > 0 ? 1 : 0) : S.p.substeps;
     int* fail = fixed ? S.fail : nullptr;
-    for (int it = 0; it < passes; ++it) {
-        LUS_HIP(lus::launch_sand_substep(A, S.x2, S.solid, S.L, n, k, B, it + 1 == passes ? S.v2 : nullptr, dt, S.att2,
-                                         s, S.fixed_cap, fail));
-        std::swap(A, B);
+    float4 *A, *B;
+    for (;;) {
+        LUS_HIP(lus::launch_sand_permute(S.tmp, S.key, S.cs, S.x, S.xs, S.att, n, S.x2, S.A, S.att2, S.perm,
+                                         S.key2, s));
+        LUS_HIP(lus::launch_sand_lists(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, S.L, s));
+        LUS_HIP(mark(2));
+        if (!fixed) {
+            LUS_HIP(hipMemcpyAsync(S.host_ctl, S.L.ctl, 2 * sizeof(*S.host_ctl), hipMemcpyDeviceToHost, s));
+            if (k.variant == 2) LUS_HIP(hipMemcpyAsync(S.host_ctl + 2, S.err, sizeof(int), hipMemcpyDeviceToHost, s));
+            LUS_HIP(hipEventRecord(S.listed, s));
+        }
+        A = S.A;
+        B = S.B;
+        for (int it = 0; it < passes; ++it) {
+            LUS_HIP(lus::launch_sand_substep(A, S.x2, S.solid, S.L, n, k, B, it + 1 == passes ? S.v2 : nullptr, dt,
+                                             S.att2, s, S.fixed_cap, fail));
+            std::swap(A, B);
+        }
+        if (fixed) break;  // lists within the capacity fit the pool
+        LUS_HIP(hipEventSynchronize(S.listed));
+        if (k.variant == 2 && *reinterpret_cast<const int*>(S.host_ctl + 2))
+            return set_error(LUS_EINVAL,
+                             "lus_sand_step: a predicted position's cell lies outside the grid (simulate_sand_v3 "
+                             "does not clamp; the reference indexes outside its cell vector there)");
+        if (S.host_ctl[0] > (unsigned long long)INT_MAX)
+            return set_error(LUS_EHIP, "lus_sand_step: neighbor count overflow");
+        const unsigned long long need = S.host_ctl[1];
+        if (need <= (unsigned long long)S.L.pool_groups) break;
+        // long lists that had no room: once more from the sort, with room
+        LUS_HIP(hipStreamSynchronize(s));
+        if (int r = sand_pool(S, (long)(need + need / 4))) return r;
+        LUS_HIP(lus::launch_zero_ints(reinterpret_cast<int*>(S.L.ctl), 4, s));
     }
     LUS_HIP(mark(3));
     if (passes == 0) LUS_HIP(lus::launch_sand_velocity(A, S.x2, S.v2, n, dt, S.L, s, S.fixed_cap, fail));
