@@ -698,7 +698,6 @@ int lus_gpu_create(LusGpu** out, int device) {
         delete c;
         return set_error(LUS_EHIP, "hipStreamCreateWithFlags: %s", hipGetErrorString(e));
     }
-    lus::pull_prepare(c->pull);
     *out = c;
     return LUS_OK;
 }
@@ -1144,6 +1143,7 @@ int pbf_setup(LusGpu* c, const LusPbfParams* p, int n, const float* pos, const f
     LUS_HIP(hipMemcpy(P.maxc, mc.data(), sizeof(int) * mc.size(), hipMemcpyHostToDevice));
     // the context stream does not order against the null stream used above
     LUS_HIP(hipDeviceSynchronize());
+    lus::pull_prepare(c->pull, 28 * (size_t)n);  // lus_pbf_download
     P.ready = true;
     return LUS_OK;
 }
@@ -2036,6 +2036,7 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
     LUS_HIP(m.alloc(&S.solid_ref, n_solid));
     if (n_solid) LUS_HIP(hipMemcpy(S.solid_ref, oref.data(), sizeof(int) * n_solid, hipMemcpyHostToDevice));
     LUS_HIP(hipDeviceSynchronize());
+    lus::pull_prepare(c->pull, 32 * (size_t)n);  // lus_sand_download
     S.ready = true;
     return LUS_OK;
 }

@@ -99,7 +99,8 @@ struct HostPiece {
 };
 // A context's pinned memory for downloads
 struct HostPull;
-void pull_prepare(HostPull*& hp);
+// Reserves it for a download of `total` bytes (a scene's, when it is made)
+void pull_prepare(HostPull*& hp, size_t total);
 void pull_free(HostPull* hp);
 HostPull*& ctx_pull(LusGpu* c);
 // Waits for the stream's work and copies the block `dev` (np pieces, one after

@@ -28,8 +28,6 @@ constexpr size_t kPullSplit = (size_t)8 << 20;
 constexpr size_t kPullChunk = (size_t)2 << 20;
 constexpr size_t kPullSmallChunk = (size_t)1 << 20;
 constexpr int kPullThreads = 4;
-// what a new context reserves: a small scene's download allocates nothing
-constexpr size_t kPullFirst = (size_t)64 << 10;
 
 struct HostPull {
     char* pin = nullptr;
@@ -127,9 +125,23 @@ bool known_memory(const void* p) {
 
 }  // namespace
 
-void pull_prepare(HostPull*& hp) {
-    hp = new (std::nothrow) HostPull;
-    if (hp && pull_reserve(hp, kPullFirst, 1) != hipSuccess) (void)hipGetLastError();
+// threads, chunk and pinned bytes for a block of `total` bytes (and `more`
+// written by the host alone)
+static size_t pull_plan(size_t total, size_t more, int* threads, size_t* chunk) {
+    *threads = total + more >= kPullSplit ? kPullThreads : 1;
+    *chunk = *threads > 1 ? kPullChunk : kPullSmallChunk;
+    // one chunk (a small download) needs no more than its own size
+    if (*threads == 1 && total <= *chunk) return (total + 4095) & ~(size_t)4095;
+    return (size_t)2 * *threads * *chunk;
+}
+
+void pull_prepare(HostPull*& hp, size_t total) {
+    if (!hp) hp = new (std::nothrow) HostPull;
+    int threads;
+    size_t chunk;
+    const size_t need = pull_plan(total, 0, &threads, &chunk);
+    // (without it the download falls back)
+    if (hp && pull_reserve(hp, need, threads) != hipSuccess) (void)hipGetLastError();
 }
 
 hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np, int* iota, int n_iota) {
@@ -148,15 +160,10 @@ hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np,
         p.total += pc[k].bytes;
         direct = direct || known_memory(pc[k].dst) || (pc[k].also && known_memory(pc[k].also));
     }
-    const size_t work = p.total + sizeof(int) * (size_t)n_iota;
-    p.threads = work >= kPullSplit ? kPullThreads : 1;
-    p.chunk = p.threads > 1 ? kPullChunk : kPullSmallChunk;
+    const size_t need = pull_plan(p.total, sizeof(int) * (size_t)n_iota, &p.threads, &p.chunk);
     p.chunks = (int)((p.total + p.chunk - 1) / p.chunk);
     if (!direct) {
         if (!hp) hp = new (std::nothrow) HostPull;
-        const size_t slots = (size_t)2 * p.threads * p.chunk;
-        // one chunk (a small download) needs no more than its own size
-        const size_t need = p.chunks <= 1 && p.threads == 1 ? (p.total + 4095) & ~(size_t)4095 : slots;
         if (!hp || pull_reserve(hp, need, p.threads) != hipSuccess) {
             (void)hipGetLastError();
             direct = true;
