@@ -212,6 +212,18 @@ struct TileArgs {
 constexpr int kBlkT = 512;
 constexpr int kBlkInts = 32;
 constexpr int kBlkMinN = 2 * 256 * kBlkT;
+// Flat lists (one lane per particle in the walks) of at most kLayMaxN particles
+// are built with a wave per stencil layer, and lambda summed by a walk of
+// them.  The build in one pass, a lane per particle, is one wave's chain of 46
+// us at 106K particles (1.6 waves per SIMD); this is 24 and the walk 13.  us per
+// step, in one pass then this way, exact and fused:
+//     512   133 -> 120   105 ->  95
+//     32K   155 -> 133   123 -> 107
+//    106K   184 -> 172   145 -> 138
+//    131K   187 -> 177   149 -> 146
+//    205K   266 -> 254   212 -> 214
+//    258K   276 -> 272   226 -> 234
+constexpr int kLayMaxN = 131072;
 // A fused plain scene of at most kSubMaxN particles walks its lists with
 // kSubLanes lanes per particle (lus_pbf.hip, "Small scenes").
 constexpr int kSubLanes = 4;

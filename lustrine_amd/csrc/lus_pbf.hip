@@ -1385,6 +1385,179 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) 
     lambda_build_ws<kFast, true>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
 }
 
+// The flat lists of a scene that leaves the SIMDs one or two waves: a block of
+// three waves takes 64 slots, one wave per stencil layer (rows 3L..3L+2, the
+// layers of the list's header), staged row by row as in lambda_build_ws.  A
+// layer's hits stay masks (a row of more than 64 slots is tested again) until
+// the layers' counts are known, then go to their places as 16-bit entries:
+// the same lists.  lambda is then a walk of them, the same sums in the same
+// order.  Times: kLayMaxN.
+constexpr int kLayT = 192;
+
+template <bool kFast>
+__global__ __launch_bounds__(kLayT) void k_pbf_list_build_lay(const float4* __restrict__ xp,
+                                                              const int* __restrict__ key2,
+                                                              const int* __restrict__ cs, int n, PbfK k,
+                                                              unsigned long long* __restrict__ nb,
+                                                              const int* __restrict__ gate) {
+    if (gate && *gate == 0) return;  // uniform: before any barrier
+    __shared__ float stage[3][kStageFloats<false>];
+    __shared__ int part[3][3][64];  // a layer's count, first and last neighbour
+    const int lane = (int)(threadIdx.x & 63);
+    const int layer = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    lds_float* __restrict__ S = (lds_float*)stage[layer];
+    const int b = (int)blockIdx.x, G = (int)gridDim.x;
+    const int i = ((b % kXcd) * (G / kXcd) + b / kXcd) * 64 + lane;
+    const bool act = i < n;
+    const int ii = act ? i : n - 1;
+    int cy, cx, cz;
+    key_cell(key2[ii] & ~kOvf, k, cy, cx, cz);
+    const float4 pi = xp[ii];
+    const int z0 = cz > 0 ? cz - 1 : 0;
+    const int z1 = cz + 1 < k.gZ ? cz + 1 : k.gZ - 1;
+    const int y = cy + layer - 1;
+    int row_j0[3], row_L[3];
+    unsigned long long row_m[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int x = cx + d - 1;
+        row_j0[d] = row_L[d] = 0;
+        row_m[d] = 0ull;
+        if (act && y >= 0 && y < k.gY && x >= 0 && x < k.gX) {
+            const int row = row_key(y, x, 0, k);
+            row_j0[d] = cs[row + z0];
+            row_L[d] = cs[row + z1 + 1] - row_j0[d];
+        }
+    }
+    const unsigned long long upto = (1ull << lane) | ((1ull << lane) - 1ull);  // lanes through this one
+    int cnt = 0, first = -1, last = -1;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int x = cx + d - 1;
+        const bool valid = act && y >= 0 && y < k.gY && x >= 0 && x < k.gX;
+        const int j0 = row_j0[d], L = row_L[d];
+        // runs of lanes whose row lies in one column (their windows ascend
+        // with the slot)
+        const int col = valid ? y * k.gX + x : -1;
+        const int pcol = __shfl_up(col, 1, 64);
+        const int ncol = __shfl_down(col, 1, 64);
+        const unsigned long long fm = __ballot(valid && (lane == 0 || pcol != col));
+        const unsigned long long lm = __ballot(valid && (lane == 63 || ncol != col));
+        const int nseg = __popcll(fm);
+        if (nseg == 0) continue;  // uniform: no lane has this row
+        int s_start[kStageSegs], s_off[kStageSegs];
+        int tot = 0;
+        {
+            unsigned long long f = fm, l = lm;
+#pragma unroll
+            for (int s = 0; s < kStageSegs; ++s) {
+                s_off[s] = tot;
+                s_start[s] = 0;
+                if (s < nseg) {
+                    const int lf = __ffsll((long long)f) - 1, ll = __ffsll((long long)l) - 1;
+                    f &= f - 1ull;
+                    l &= l - 1ull;
+                    s_start[s] = __builtin_amdgcn_readlane(j0, lf);
+                    tot += __builtin_amdgcn_readlane(j0 + L, ll) - s_start[s];
+                }
+            }
+        }
+        // uniform: every window is empty (tot covers every run only when there
+        // are at most kStageSegs)
+        if (tot == 0 && nseg <= kStageSegs) continue;
+        unsigned long long m = 0ull;
+        if (nseg <= kStageSegs && tot <= kStageCap) {  // uniform
+            for (int q = lane; q < tot; q += 64) {
+                int j = q - s_off[0] + s_start[0];
+                if (nseg > 1) {
+#pragma unroll
+                    for (int s = 1; s < kStageSegs; ++s)
+                        if (q >= s_off[s]) j = q - s_off[s] + s_start[s];
+                }
+                const float4 p = at4(xp, j);
+                S[3 * q] = p.x;
+                S[3 * q + 1] = p.y;
+                S[3 * q + 2] = p.z;
+            }
+            wave_lds_sync();
+            int lo = j0 - s_start[0] + s_off[0];
+            if (nseg > 1) {  // uniform
+                const int seg = __popcll(fm & upto) - 1;
+#pragma unroll
+                for (int s = 1; s < kStageSegs; ++s)
+                    if (seg == s) lo = j0 - s_start[s] + s_off[s];
+            }
+            if (__all(L <= 32))
+                m = test_row_staged<unsigned int, 3, kFast>(pi, lo, L, S, k);
+            else if (L <= 64)
+                m = test_row_staged<unsigned long long, 3, kFast>(pi, lo, L, S, k);
+            wave_lds_sync();  // the next row's staging overwrites this one's
+        } else if (L <= 64) {
+            for (int t = 0; t < L; ++t) m |= within_h<kFast>(pi, xyz_at(xp, j0 + t), k) ? 1ull << t : 0ull;
+        }
+        if (L > 64) {
+            for (int j = j0; j < j0 + L; ++j)
+                if (within_h<kFast>(pi, xyz_at(xp, j), k)) {
+                    first = first < 0 ? j : first;
+                    last = j;
+                    ++cnt;
+                }
+        } else if (m) {
+            first = first < 0 ? j0 + low_bit(m) : first;
+            last = j0 + high_bit(m);
+            cnt += __popcll(m);
+        }
+        row_m[d] = m;
+    }
+    part[layer][0][lane] = cnt;
+    part[layer][1][lane] = first;
+    part[layer][2][lane] = last;
+    __syncthreads();
+    const int c0 = part[0][0][lane], c1 = part[1][0][lane], c2 = part[2][0][lane];
+    const int c = c0 + c1 + c2;
+    bool retest = c > kNbrCap;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) retest = retest || part[l][2][lane] - part[l][1][lane] > 0xFFFF;
+    if (!act) return;
+    if (!retest) {
+        int4* __restrict__ lst = nbr_list(nb, n, i);
+        // entry p of the list: group p / 8, 16-bit place p % 8 of the int4
+        auto place = [&](int p) {
+            return reinterpret_cast<unsigned short*>(lst + (size_t)(p >> 3) * 64) + (p & 7);
+        };
+        int p = layer == 0 ? 0 : (layer == 1 ? c0 : c0 + c1);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const int j0 = row_j0[d], L = row_L[d];
+            if (L <= 64) {
+                for (unsigned long long m = row_m[d]; m; m &= m - 1ull)
+                    *place(p++) = (unsigned short)(j0 + low_bit(m) - first);
+            } else {
+                for (int j = j0; j < j0 + L; ++j)
+                    if (within_h<kFast>(pi, xyz_at(xp, j), k)) *place(p++) = (unsigned short)(j - first);
+            }
+        }
+        // the places past the count in the last group (a walk decodes them, to slot b2)
+        if (layer == 2)
+            for (int q = c; (q & 7) != 0; ++q) *place(q) = 0;
+    }
+    if (layer == 0) {
+        const int f0 = part[0][1][lane], f1 = part[1][1][lane], f2 = part[2][1][lane];
+        const int w = retest ? kNbrRetest : (c | (c0 << 16) | ((c0 + c1) << 24));
+        nbr_hdr(nb)[i] = make_int4(f0 < 0 ? i : f0, f1 < 0 ? i : f1, f2 < 0 ? i : f2, w);
+    }
+}
+
+hipError_t launch_list_build_lay(const float4* xp, const int* key2, const int* cs, int n, PbfK k,
+                                 unsigned long long* nb, const int* gate, hipStream_t s) {
+    const dim3 g(grid_for(n, 64)), b(kLayT);
+    if (k.exact)
+        launch_kernel((k_pbf_list_build_lay<false>), g, b, 0, s, xp, key2, cs, n, k, nb, gate);
+    else
+        launch_kernel((k_pbf_list_build_lay<true>), g, b, 0, s, xp, key2, cs, n, k, nb, gate);
+    return hipGetLastError();
+}
+
 template <bool kBuild, bool kFast>
 __global__ __launch_bounds__(kTileT) void k_pbf_lambda_t(const float4* __restrict__ xa,
                                                           int* __restrict__ key2,
@@ -1442,6 +1615,10 @@ hipError_t launch_pbf_lambda(const float4* xa, int* key2, const int* cs, int n, 
     if (ta.blk && build) return launch_build_blk(xp, key2, cs, n, k, xl, maxc, masks, gate, ta.blk, s);
     if (ta.blk) return launch_lambda_blk(xa, key2, cs, n, k, xl, maxc, masks, xp, gate, ta.blk, s);
     const dim3 g(grid_for(n, ta.block)), b(ta.block);
+    if (build && ta.stage && xa == xp && n > 0 && k.nph == 1 && n <= kLayMaxN) {
+        if (hipError_t e = launch_list_build_lay(xp, key2, cs, n, k, masks, gate, s)) return e;
+        build = 0;
+    }
     if (build && ta.stage && xa == xp && n > 0 && k.nph == 1) {
         if (k.exact)
             launch_kernel((k_pbf_lambda_build_ws<false, false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, masks,
@@ -2984,6 +3161,8 @@ hipError_t launch_pbf_features(int* key2, const int* cs, int n, PbfK k, unsigned
     const bool staged = ta.stage && n > 0;
     if (staged && ta.blk) {
         if (hipError_t e = launch_build_blk(xp, key2, cs, n, k, nullptr, nullptr, masks, nullptr, ta.blk, s)) return e;
+    } else if (staged && n <= kLayMaxN) {
+        if (hipError_t e = launch_list_build_lay(xp, key2, cs, n, k, masks, nullptr, s)) return e;
     } else if (staged && k.exact)
         launch_kernel((k_pbf_list_build_ws<false>), g, b, 0, s, xp, (const int*)key2, cs, n, k, masks);
     else if (staged)

@@ -111,3 +111,11 @@ def test_batch(gpu_mod):
             out.append(g.pbf_download(order=1))
     same(out[0], out[1])
     same(out[0], out[2])
+
+
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("lat", [(64, 32, 64), (64, 33, 64)])
+def test_either_side_of_the_layered_build(gpu_mod, lat, exact):
+    # 131072 particles: a wave per stencil layer; 135168: a lane per particle
+    cfg, pos, vel = scene(lat, (140, 72, 140), 0.2, 5)
+    same(plain(gpu_mod, cfg, pos, vel, 1, exact, steps=1), plain(gpu_mod, cfg, pos, vel, 0, exact, steps=1))
