@@ -401,8 +401,8 @@ def bench_fluid(args, G, scenes) -> int:
     """The reference's simulate_fluid (src/Simulate.cpp:27-115) on the GPU: the
     1,048,576-particle lattice in 256 x 128 x 256 with the reference's
     Simulation defaults (rest density 24, epsilon 10, cubic kernel, h = 4 r),
-    its sequential pressure sweep run as dependency levels.  Host clock
-    around synchronised steps (the sweep synchronises every 32 levels)."""
+    its sequential pressure sweep run as data flow.  Host clock around
+    synchronised steps (a step waits twice: for its lists and for its sweep)."""
     from oracle import oracle as O
     O.build()
     cfg = scenes.cfg2()

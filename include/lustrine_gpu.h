@@ -341,16 +341,16 @@ int lus_sand_init(LusGpu* ctx, const LusSandParams* p, int n_sand, const float* 
                   const float* vel, const int* attracted, int n_solid,
                   const float* solid_pos, const int* solid_index);
 /* One simulate_sand call.  player = Bullet player position (3 floats, may be
- * NULL when both flags are 0).  By default the call waits once for the device
- * mid-step: the neighbour lists' total length sizes their buffer before they
- * are written (the lists have no fixed capacity, as the reference's vectors).
+ * NULL when both flags are 0).  By default the call waits for the device until
+ * the step's neighbour lists are built (they have no fixed capacity, as the
+ * reference's vectors: long ones that had no room are built again with it).
  * With a fixed capacity (lus_sand_set_list_capacity) it only enqueues. */
 int lus_sand_step(LusGpu* ctx, float dt, int attract_flag, int blow_flag, const float* player);
 /* entries > 0: the neighbour lists get a fixed buffer of that many entries
  * and lus_sand_step no longer waits for the device (the reference's lists
  * grow instead, src/neighbors/Neighbors.cpp:306-361; ~33 entries per
- * particle on the 1 M sand lattice).  A step whose lists would not fit writes
- * none, skips its substeps and leaves an invalid state; the next
+ * particle on the 1 M sand lattice).  A step whose lists are longer in total
+ * projects no contact and leaves an invalid state; the next
  * lus_gpu_sync, lus_sand_download or lus_sand_neighbors reports it
  * (LUS_ESTATE) and clears the mark.  In the same way a simulate_sand_v3
  * prediction outside the grid is reported there (LUS_EINVAL).  0 (default):
@@ -500,14 +500,15 @@ int lus_fluid_init(LusGpu* ctx, const LusFluidParams* p, int total, int sand_sta
 /* One simulate_fluid call (src/Simulate.cpp:27-115): dt clamped to [0.001,
  * 0.01], prediction, neighbour lists (Neighbors.cpp:366-450), lambdas, and the
  * pressure sweep in the reference's sequential order (particle i sees the
- * particles before it corrected), run level by level on the device.  Waits for
+ * particles before it corrected), run as data flow on the device.  Waits for
  * the device.  A predicted position whose cell index lies outside the grid
  * (the reference indexes outside its cell vector there) fails with LUS_EINVAL. */
 int lus_fluid_step(LusGpu* ctx, float dt);
 /* positions, positions_star (all `total` slots), velocities (moving slots),
  * lambdas (n_lambdas); each nullable. */
 int lus_fluid_download(LusGpu* ctx, float* positions, float* positions_star, float* velocities, float* lambdas);
-/* Of the last step: dependency levels of the sweep, list entries. */
+/* Of the last step: the sweep's longest chain of dependent particles, list
+ * entries. */
 int lus_fluid_stats(LusGpu* ctx, int* levels, long* list_entries);
 
 #ifdef __cplusplus

@@ -180,7 +180,9 @@ hipError_t launch_fluid_nbr(const float4* sand_sorted, const int* sand_key, cons
 // of layer L.  A particle with more than kNbrCap neighbours, or one whose
 // neighbours lie more than 65535 slots past their layer's first, has
 // w = kNbrRetest and re-tests its candidates in every pass.  Tiled passes: 9
-// row masks per particle, masks[r * n + i].  A step uses one of the two forms.
+// row masks per particle, masks[r * n + i].  Block-staged passes (kBlkT): the
+// same groups, entries are places in the block's copy; see lus_pbf.hip.  A
+// step uses one of the forms.
 constexpr int kNbrCap = 128;  // about 4x the rest-state count (a K = 1 solve compresses 2.5x)
 constexpr int kNbrGroups = kNbrCap / 8;
 constexpr int kNbrRetest = 0xFFFF;

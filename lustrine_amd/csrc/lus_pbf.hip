@@ -19,7 +19,10 @@
 // max_i |N(i)| iterations instead of the sum over the 9 rows of the longest
 // row (about half as many on a dam break).  A particle with more than
 // kNbrCap neighbours (or with an entry beyond 16 bits) re-tests its candidates against the stored predicted
-// positions in every pass, which gives the same set in the same order.  The
+// positions in every pass, which gives the same set in the same order.  By
+// size the lists are built with a wave per stencil layer and lambda walks them
+// (kLayMaxN), or lambda is summed in the building pass, and from kBlkMinN on
+// they are block-staged: a walk reads its neighbours from LDS.  The
 // tiled passes keep the row masks instead (masks[r * n + i], bit t = slot
 // j0_r + t) and flag a particle whose stencil has a row longer than 64 slots
 // in its key (kOvf).
@@ -3175,6 +3178,9 @@ __global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ m
                                                        int cap) {
     __shared__ int wmax[kBlock / 64];
     __shared__ float wsum[kBlock / 64];
+    // no rerun: the attempt's entry stands (uniform; reducing first took the
+    // step another 12 us at 1M particles)
+    if (learned == 2 && *flag == 0) return;
     int m = INT_MIN;
     float s = 0.0f;
     for (int b = threadIdx.x; b < nblk; b += kBlock) {
@@ -3206,7 +3212,6 @@ __global__ __launch_bounds__(kBlock) void k_pbf_decide(const int* __restrict__ m
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        if (learned == 2 && *flag == 0) return;  // no rerun: the attempt's entry stands
         int b = wmax[0];
         float tot = wsum[0];
 #pragma unroll
