@@ -2073,12 +2073,18 @@ int sand_check(LusGpu* c) {
     return LUS_OK;
 }
 
-// Room for `groups` int4 in the pool of long lists
+// Room for `groups` int4 in the pool of long lists, those of the last step
+// kept (no work may be in flight).  It never shrinks while the scene lives.
 int sand_pool(SandState& S, long groups) {
-    S.pool_mem.release();
-    S.L.pool = nullptr;
-    S.L.pool_groups = 0;
-    LUS_HIP(S.pool_mem.alloc(&S.L.pool, (size_t)groups));
+    if (groups <= S.L.pool_groups) return LUS_OK;
+    Arena fresh;
+    int4* pool = nullptr;
+    LUS_HIP(fresh.alloc(&pool, (size_t)groups));
+    if (S.L.pool_groups > 0)
+        LUS_HIP(hipMemcpy(pool, S.L.pool, sizeof(int4) * (size_t)S.L.pool_groups, hipMemcpyDeviceToDevice));
+    LUS_HIP(hipDeviceSynchronize());
+    std::swap(S.pool_mem.ptrs, fresh.ptrs);  // the old one goes with `fresh`
+    S.L.pool = pool;
     S.L.pool_groups = groups;
     return LUS_OK;
 }

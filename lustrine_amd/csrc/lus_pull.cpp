@@ -10,8 +10,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <exception>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "lus_device.hpp"
@@ -189,7 +189,7 @@ hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np,
     try {
         for (; started < p.threads; ++started)
             th[started] = std::thread([&p, &err, started] { err[started] = p.run(started); });
-    } catch (const std::system_error&) {  // no thread: its chunks are taken here
+    } catch (const std::exception&) {  // no thread: its chunks are taken here
     }
     err[0] = p.run(0);
     for (int w = started; w < p.threads; ++w) err[w] = p.run(w);

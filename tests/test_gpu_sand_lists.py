@@ -153,3 +153,18 @@ def test_small_and_large_scene_forms_agree(gpu_mod, solids, spacing):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     for a, b in zip(out[0][2], out[1][2]):
         assert np.array_equal(a, b)
+
+
+def test_lists_stay_readable_when_a_capacity_is_set(gpu_mod):
+    # the last step's long lists lie in the pool; a small capacity set after it
+    # leaves them as they are
+    pos, sol = _clump_and_layer(True)
+    sp, index = _params(gpu_mod, len(pos), sol)
+    with gpu_mod.Gpu(0) as g:
+        g.sand_init(sp, pos, None, None, sol, index)
+        g.sand_step(DT, False, False, None)
+        off, idx = g.sand_neighbors()
+        for entries in (100, 10 * int(off[-1]), 0):
+            g.sand_set_list_capacity(entries)
+            a, b = g.sand_neighbors()
+            assert np.array_equal(a, off) and np.array_equal(b, idx)
