@@ -179,6 +179,11 @@ struct PbfState {
     bool use_graph = false;
     int parity = 0, graph_parity = 0;
     float graph_dt = 0.0f;
+    // nred and lists_blk as the captured steps leave them: a replay enqueues
+    // nothing that would set them, and a recorded step since the capture may
+    // have left the other form
+    int graph_nred = 0;
+    bool graph_lists_blk = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     // learned warm start and density statistics
@@ -658,8 +663,12 @@ int pbf_run(LusGpu* c, float dt, int steps) {
             LUS_HIP(hipGraphInstantiate(&P.graph_exec, P.graph, nullptr, nullptr, 0));
             P.graph_dt = dt;
             P.graph_parity = P.parity;
+            P.graph_nred = P.nred;
+            P.graph_lists_blk = P.lists_blk;
         }
         LUS_HIP(hipGraphLaunch(P.graph_exec, c->stream));
+        P.nred = P.graph_nred;
+        P.lists_blk = P.graph_lists_blk;
         left -= 2;
     }
     if (left) return pbf_enqueue(c, dt, nullptr, nullptr);
