@@ -635,19 +635,20 @@ int pbf_run(LusGpu* c, float dt, int steps) {
     }
     int left = steps;
     while (left >= 2) {
+        // a captured step that skips the key kernel relies on the step before
+        // it, and one that runs it on a cleared histogram: capture and replay
+        // only when the keys at hand are exactly what the captured steps leave
+        // behind (written for dt when the steps write keys, none otherwise).  A
+        // step with another dt, or a recorded one before learned steps, leaves
+        // other keys: an ordinary step first takes them up
+        const bool writes_keys = P.fuse_keys && !P.learned && !P.mixed && !P.tiled;
+        if (writes_keys ? !(P.keys_dt == dt) : !std::isnan(P.keys_dt)) {
+            int r = pbf_enqueue(c, dt, nullptr, nullptr);
+            if (r) return r;
+            --left;
+            continue;
+        }
         if (!P.graph_exec || P.graph_dt != dt || P.graph_parity != P.parity) {
-            // a captured step that skips the key kernel relies on the step
-            // before it: capture only when the keys at hand are exactly what
-            // the captured steps leave behind (written for dt when the steps
-            // write keys, none otherwise), so every replay sees the state the
-            // capture saw
-            const bool writes_keys = P.fuse_keys && !P.learned && !P.mixed && !P.tiled;
-            if (writes_keys != (P.keys_dt == dt)) {
-                int r = pbf_enqueue(c, dt, nullptr, nullptr);
-                if (r) return r;
-                --left;
-                continue;
-            }
             pbf_drop_graph(P);
             LUS_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             int r1 = pbf_enqueue(c, dt, nullptr, nullptr);
