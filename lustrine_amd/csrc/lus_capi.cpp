@@ -2127,6 +2127,7 @@ int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
         LUS_HIP(lus::launch_sand_permute(S.tmp, S.key, S.cs, S.x, S.xs, S.att, n, S.x2, S.A, S.att2, S.perm,
                                          S.key2, s));
         LUS_HIP(lus::launch_sand_lists(S.A, S.key2, S.cs, n, S.solid, S.ocs, k, S.L, s));
+        S.list_n = n;
         LUS_HIP(mark(2));
         if (!fixed) {
             LUS_HIP(hipMemcpyAsync(S.host_ctl, S.L.ctl, 2 * sizeof(*S.host_ctl), hipMemcpyDeviceToHost, s));
@@ -2181,7 +2182,6 @@ void sand_after(SandState& S, const lus::SandK& k) {
     std::swap(S.v, S.v2);
     std::swap(S.att, S.att2);
     if (k.variant != 2) S.prev_attract = k.attract;  // v3 keeps no previous flag
-    S.list_n = S.n;
     S.stepped = true;
 }
 
@@ -2248,6 +2248,7 @@ int lus_sand_step(LusGpu* c, float dt, int attract_flag, int blow_flag, const fl
         hit = &S.graphs.back();
     }
     LUS_HIP(hipGraphLaunch(hit->exec, c->stream));
+    S.list_n = S.n;  // the captured n: captured steps go when it changes
     sand_after(S, k);
     return LUS_OK;
 }
@@ -2447,6 +2448,7 @@ int lus_sand_sink_evict(LusGpu* c, const int* cells, int ncells, int* n_sand) {
             LUS_HIP(lus::launch_slot_moves(d_mv, m, S.x, S.v, S.att, t0, t1, t2, s));
             LUS_HIP(hipStreamSynchronize(s));
         }
+        if (end != S.n) sand_drop_graphs(S);  // the count is a kernel argument of the captured steps
         S.n = end;
     }
     if (n_sand) *n_sand = S.n;
