@@ -1153,6 +1153,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 
 hipError_t launch_sand_lists(const float4* xs, const int* key2, const int* sand_cs, int n, const float4* solid,
                              const int* solid_cs, SandK k, SandLists L, hipStream_t s) {
+    if (n <= 0) return hipSuccess;  // every grain evicted: a lane without a slot stands in for the last one
 #define LUS_LISTS(K, T) \
     launch_kernel((K), dim3(grid_for(n, T)), dim3(kBlock), 0, s, xs, key2, sand_cs, n, solid, solid_cs, k, L)
     if (n <= kSandSubMaxN) {
