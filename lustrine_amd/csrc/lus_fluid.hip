@@ -320,15 +320,18 @@ __global__ __launch_bounds__(kBlock) void k_fl_lambda(const float4* __restrict__
 // that already runs: every wait ends.  (kSweepSpins passes without progress
 // end it with an error all the same.)
 //
-// What bounds it is the longest chain of waits, 2.7 to 3.2 us a link at 32 K
-// particles (a bare store and load between two XCDs takes 0.6; the rest is the
-// last term, its sum and the divides).  One launch per level took 36 us a
-// link and more: 32 K particles, 218 to 870 links, step 8.7 to 66 -> 0.85 to 2.8 ms;
-// 1 M, 762 links, step 37 -> 18 ms.  A particle that waits for many neighbours
-// asks for the latest of them only, one that waits for at most kSweepFew asks
-// for each, with a pause between (1, 4, 10, 30 x 64 cycles at the 870 links:
-// 3.4, 2.9, 2.8, 2.8 ms), so that the waves far from the front leave the ones
-// at it alone.
+// At 32 K particles the longest chain of waits bounds it, 2.7 to 3.2 us a link
+// (a bare store and load between two XCDs takes 0.6; the rest is the last term,
+// its sum and the divides): 218 links 0.82 ms a step, 905 links 2.8 ms, where one
+// launch per level (36 us a link and more) took 8.7 and 66.  At 1 M (762 links,
+// 17.5 ms, 37 with launches) it is the window of particles in flight.  A
+// particle that waits for at most kSweepFew neighbours asks for each; one that waits
+// for more asks for the latest of each eight lanes (of each four with 16 lanes a
+// particle), so that the waves far from the front leave the ones at it alone.
+// The latest of the whole particle alone took 32 K (800 steps) 949 ms, 262 K
+// 4.28 ms and 1 M 19.0 ms; every missing one 925, 3.85, 16.9; this 887, 4.00, 17.5.
+// Between two askings it pauses (1, 4, 10, 30 x 64 cycles at the 905 links: 2.95,
+// 2.86, 2.78, 2.86 ms).
 //
 // kLanes lanes hold one particle and take its list kLanes * kPer entries at a
 // time, entry e in lane e % kLanes.  Few particles per wave shorten a link
@@ -346,10 +349,13 @@ __device__ __forceinline__ int dpp_max(int v) {
     const int o = __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xF, 0xF, false);
     return o > v ? o : v;
 }
+__device__ __forceinline__ int quad_max(int v) {  // of the lane's four
+    v = dpp_max<0xB1>(v);                        // lane ^ 1
+    return dpp_max<0x4E>(v);                     // lane ^ 2
+}
 template <int kLanes>
 __device__ __forceinline__ int sweep_max(int v) {
-    v = dpp_max<0xB1>(v);                        // lane ^ 1
-    v = dpp_max<0x4E>(v);                        // lane ^ 2
+    v = quad_max(v);
     v = dpp_max<0x141>(v);                       // half row mirrored
     v = dpp_max<0x140>(v);                       // row mirrored
 #pragma unroll
@@ -543,7 +549,8 @@ __global__ __launch_bounds__(kBlock) void k_fl_sweep(float4* __restrict__ x, con
                 u0 = u;
             }
         const bool few = __popcll(__ballot(pend != 0u) & group) <= kSweepFew;
-        const bool asks = top >= 0 && (few || sweep_max<kLanes>(top) == top);
+        const int latest = kLanes == 64 ? dpp_max<0x141>(quad_max(top)) : quad_max(top);
+        const bool asks = top >= 0 && (few || latest == top);
         SweepPos q = {};
         bool here = false;
         int spins = 0;
@@ -589,7 +596,7 @@ static void launch_sweep_lanes(float4* x, const float4* xs, float4* xs2, float4*
 // A wave per particle while the particles in flight (8,192 at 8 waves per
 // SIMD) cover most of the sweep's front, else four particles per wave
 // (measured, one / two / four per wave: 32 K at 870 links 2.8 / 3.6 / 4.4 ms,
-// 262 K 6.4 / 4.6 / 4.2 ms, 1 M 27 / 20 / 18 ms).
+// 262 K 6.4 / 4.6 / 4.0 ms, 1 M 27 / 20 / 17.5 ms).
 constexpr int kSweepWideN = 65536;
 
 static hipError_t launch_sweep(float4* x, const float4* xs, float4* xs2, float4* v, const float* lam, const int* off,
