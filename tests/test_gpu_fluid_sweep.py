@@ -1,7 +1,7 @@
-"""The data-flow form of simulate_fluid's sequential sweep at the sizes where
-it can go wrong: particle counts around a block's 32 and a wave's 8, lists
-around and past the 48 entries taken at a time (several chunks), moving slots
-that do not start at 0 with solids before and after them, and exponents other
+"""The data-flow form of simulate_fluid's sequential sweep: particle counts up
+to 4,099 and past the switch to four particles per wave (65,536), lists within
+and past the 64 entries taken at a time (several chunks), moving slots that do
+not start at 0 with solids before and after them, and exponents other
 than 4.  Same bar as test_gpu_fluid.py: positions within 1e-5 relative of the
 FP32 oracle (the one call that differs, the power in s_coor, is off by one ulp
 for about 7 in 10,000 arguments), lambdas of the step bit for bit.
