@@ -298,7 +298,7 @@ struct LusGpu {
     NetState net;
     SandState sand;
     lus::FluidState* fluid = nullptr;      // simulate_fluid state (lus_fluid.hip)
-    lus::HostPull* pull = nullptr;         // pinned memory of downloads (lus_pull.cpp)
+    lus::HostPull* pull = nullptr;         // events of downloads (lus_pull.cpp)
     std::vector<LusMlpTrainer*> trainers;  // live trainers, detached on destroy
 };
 
@@ -708,6 +708,7 @@ int lus_gpu_create(LusGpu** out, int device) {
         delete c;
         return set_error(LUS_EHIP, "hipStreamCreateWithFlags: %s", hipGetErrorString(e));
     }
+    lus::pull_open();
     *out = c;
     return LUS_OK;
 }
@@ -735,6 +736,7 @@ void lus_gpu_destroy(LusGpu* c) {
     c->fluid = nullptr;
     lus::pull_free(c->pull);
     c->pull = nullptr;
+    lus::pull_close();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1153,7 +1155,6 @@ int pbf_setup(LusGpu* c, const LusPbfParams* p, int n, const float* pos, const f
     LUS_HIP(hipMemcpy(P.maxc, mc.data(), sizeof(int) * mc.size(), hipMemcpyHostToDevice));
     // the context stream does not order against the null stream used above
     LUS_HIP(hipDeviceSynchronize());
-    lus::pull_prepare(c->pull, 28 * (size_t)n);  // lus_pbf_download
     P.ready = true;
     return LUS_OK;
 }
@@ -2046,7 +2047,6 @@ int lus_sand_init(LusGpu* c, const LusSandParams* p, int n_sand, const float* po
     LUS_HIP(m.alloc(&S.solid_ref, n_solid));
     if (n_solid) LUS_HIP(hipMemcpy(S.solid_ref, oref.data(), sizeof(int) * n_solid, hipMemcpyHostToDevice));
     LUS_HIP(hipDeviceSynchronize());
-    lus::pull_prepare(c->pull, 32 * (size_t)n);  // lus_sand_download
     S.ready = true;
     return LUS_OK;
 }

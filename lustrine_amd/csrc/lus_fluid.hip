@@ -816,8 +816,6 @@ int lus_fluid_init(LusGpu* c, const LusFluidParams* p, int total, int sand_start
         FL_HIP(hipMemcpyAsync(F->ocs, ocnt.data(), sizeof(int) * (C + 1), hipMemcpyHostToDevice, s));
         FL_HIP(hipStreamSynchronize(s));
     }
-    // lus_fluid_download
-    lus::pull_prepare(lus::ctx_pull(c), 24 * (size_t)total + 12 * (size_t)n + 4 * (size_t)k.nl);
     F->stepped = false;
     return LUS_OK;
 }

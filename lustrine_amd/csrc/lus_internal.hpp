@@ -97,11 +97,12 @@ struct HostPiece {
     void* also;
     size_t bytes;
 };
-// A context's pinned memory for downloads
+// A context's events for downloads
 struct HostPull;
-// Reserves it for a download of `total` bytes (a scene's, when it is made)
-void pull_prepare(HostPull*& hp, size_t total);
 void pull_free(HostPull* hp);
+// A context begins / ends (the pinned memory of downloads goes with the last)
+void pull_open();
+void pull_close();
 HostPull*& ctx_pull(LusGpu* c);
 // Waits for the stream's work and copies the block `dev` (np pieces, one after
 // the other) to their places; iota[r] = r for r < n_iota.

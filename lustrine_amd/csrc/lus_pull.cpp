@@ -11,8 +11,10 @@
 
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <new>
 #include <thread>
+#include <utility>
 
 #include "lus_device.hpp"
 #include "lus_internal.hpp"
@@ -22,42 +24,105 @@ namespace lus {
 // Chunks of 2 MB over four threads from 8 MB on: 48 MB take 1.4 ms with them,
 // 3.6 ms on one thread; 1 MB chunks 1.9 ms, 8 MB chunks 1.7 ms, eight threads
 // 1.45 ms.  Below, starting threads costs what they save (3 MB: 0.15 ms with
-// one or four), and 1 MB chunks overlap better.  A context holds at most
+// one or four), and 1 MB chunks overlap better.  A download holds at most
 // 16 MB of pinned memory for it.
 constexpr size_t kPullSplit = (size_t)8 << 20;
 constexpr size_t kPullChunk = (size_t)2 << 20;
 constexpr size_t kPullSmallChunk = (size_t)1 << 20;
 constexpr int kPullThreads = 4;
 
+// a context's events
 struct HostPull {
-    char* pin = nullptr;
-    size_t cap = 0;
     hipEvent_t ev[2 * kPullThreads] = {};
     int nev = 0;
 };
 
 void pull_free(HostPull* hp) {
     if (!hp) return;
-    if (hp->pin) (void)hipHostFree(hp->pin);
     for (int k = 0; k < hp->nev; ++k) (void)hipEventDestroy(hp->ev[k]);
     delete hp;
 }
 
 namespace {
 
-// pinned room for `bytes` and the events of `threads` threads
-hipError_t pull_reserve(HostPull* hp, size_t bytes, int threads) {
-    if (hp->cap < bytes) {
-        if (hp->pin) (void)hipHostFree(hp->pin);
-        hp->pin = nullptr;
-        hp->cap = 0;
-        const hipError_t e = hipHostMalloc((void**)&hp->pin, bytes, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            hp->pin = nullptr;
-            return e;
-        }
-        hp->cap = bytes;
+// The pinned memory belongs to a download only while it runs: the contexts
+// take it from these blocks in turn (allocating 16 MB takes 0.3 ms, smaller
+// ones 0.02 to 0.07).  Reserving it with each scene instead made scenes longer
+// to prepare (1M 3.4 -> 3.9 ms, 512 particles 0.24 -> 0.27), for a program that
+// downloads nothing too; a new scene's first download takes 2.7 ms at 1M and
+// 0.03 at 512 so, 3.1 and 0.04 then.  At most kPinIdle blocks are kept, and none
+// once the last context is gone.
+struct PinBlock {
+    char* p = nullptr;
+    size_t cap = 0;
+};
+constexpr int kPinIdle = 4;
+struct PinPool {
+    std::mutex m;
+    PinBlock idle[kPinIdle];
+    int contexts = 0;
+};
+// (never destroyed: at exit the runtime may be gone before it)
+PinPool& pin_pool() {
+    static PinPool* pool = new PinPool;
+    return *pool;
+}
+
+// the smallest idle block of at least `bytes`, or a new one (p null: none to be had)
+PinBlock pin_take(size_t bytes) {
+    PinPool& pool = pin_pool();
+    PinBlock got;
+    {
+        std::lock_guard<std::mutex> lock(pool.m);
+        PinBlock* best = nullptr;
+        for (PinBlock& b : pool.idle)
+            if (b.p && b.cap >= bytes && (!best || b.cap < best->cap)) best = &b;
+        if (best) std::swap(got, *best);
     }
+    if (got.p) return got;
+    if (hipHostMalloc((void**)&got.p, bytes, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        got.p = nullptr;
+        return got;
+    }
+    got.cap = bytes;
+    return got;
+}
+
+// back to the idle ones; with all places taken the smallest is freed
+void pin_give(PinBlock b) {
+    PinPool& pool = pin_pool();
+    {
+        std::lock_guard<std::mutex> lock(pool.m);
+        for (PinBlock& q : pool.idle)
+            if (q.cap < b.cap) std::swap(q, b);
+    }
+    if (b.p) (void)hipHostFree(b.p);
+}
+
+}  // namespace
+
+void pull_open() {
+    PinPool& pool = pin_pool();
+    std::lock_guard<std::mutex> lock(pool.m);
+    ++pool.contexts;
+}
+
+void pull_close() {
+    PinPool& pool = pin_pool();
+    PinBlock gone[kPinIdle];
+    {
+        std::lock_guard<std::mutex> lock(pool.m);
+        if (--pool.contexts > 0) return;
+        for (int k = 0; k < kPinIdle; ++k) std::swap(gone[k], pool.idle[k]);
+    }
+    for (const PinBlock& b : gone)
+        if (b.p) (void)hipHostFree(b.p);
+}
+
+namespace {
+
+hipError_t pull_events(HostPull* hp, int threads) {
     for (; hp->nev < 2 * threads; ++hp->nev) {
         const hipError_t e = hipEventCreateWithFlags(&hp->ev[hp->nev], hipEventDisableTiming);
         if (e != hipSuccess) return e;
@@ -68,7 +133,8 @@ hipError_t pull_reserve(HostPull* hp, size_t bytes, int threads) {
 struct Pull {
     int device;
     hipStream_t s;
-    HostPull* hp;
+    const HostPull* hp;
+    char* pin;
     const char* dev;
     const HostPiece* pc;
     int np, threads, chunks, n_iota;
@@ -78,7 +144,7 @@ struct Pull {
     size_t first(int i) const { return chunk * (size_t)i; }
     size_t length(int i) const { return first(i) + chunk <= total ? chunk : total - first(i); }
     // slot u of thread w
-    char* slot(int w, int u) const { return hp->pin + chunk * (size_t)(2 * w + u); }
+    char* slot(int w, int u) const { return pin + chunk * (size_t)(2 * w + u); }
 
     hipError_t issue(int w, int u, int i) const {
         const hipError_t e = hipMemcpyAsync(slot(w, u), dev + first(i), length(i), hipMemcpyDeviceToHost, s);
@@ -135,15 +201,6 @@ static size_t pull_plan(size_t total, size_t more, int* threads, size_t* chunk) 
     return (size_t)2 * *threads * *chunk;
 }
 
-void pull_prepare(HostPull*& hp, size_t total) {
-    if (!hp) hp = new (std::nothrow) HostPull;
-    int threads;
-    size_t chunk;
-    const size_t need = pull_plan(total, 0, &threads, &chunk);
-    // (without it the download falls back)
-    if (hp && pull_reserve(hp, need, threads) != hipSuccess) (void)hipGetLastError();
-}
-
 hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np, int* iota, int n_iota) {
     hipStream_t s = ctx_stream(c);
     HostPull*& hp = ctx_pull(c);
@@ -162,11 +219,15 @@ hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np,
     }
     const size_t need = pull_plan(p.total, sizeof(int) * (size_t)n_iota, &p.threads, &p.chunk);
     p.chunks = (int)((p.total + p.chunk - 1) / p.chunk);
-    if (!direct) {
+    PinBlock pin;
+    if (!direct && need > 0) {
         if (!hp) hp = new (std::nothrow) HostPull;
-        if (!hp || pull_reserve(hp, need, p.threads) != hipSuccess) {
+        if (!hp || pull_events(hp, p.threads) != hipSuccess) {
             (void)hipGetLastError();
             direct = true;
+        } else {
+            pin = pin_take(need);
+            direct = !pin.p;
         }
     }
     if (direct) {
@@ -183,6 +244,7 @@ hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np,
         return hipStreamSynchronize(s);
     }
     p.hp = hp;
+    p.pin = pin.p;
     hipError_t err[kPullThreads] = {};
     std::thread th[kPullThreads];
     int started = 1;
@@ -194,12 +256,12 @@ hipError_t pull_to_host(LusGpu* c, const void* dev, const HostPiece* pc, int np,
     err[0] = p.run(0);
     for (int w = started; w < p.threads; ++w) err[w] = p.run(w);
     for (int w = 1; w < started; ++w) th[w].join();
+    hipError_t bad = hipSuccess;
     for (hipError_t e : err)
-        if (e != hipSuccess) {
-            (void)hipStreamSynchronize(s);  // no copy into the slots is left in flight
-            return e;
-        }
-    return hipSuccess;
+        if (e != hipSuccess) bad = e;
+    if (bad != hipSuccess) (void)hipStreamSynchronize(s);  // no copy into the slots is left in flight
+    pin_give(pin);
+    return bad;
 }
 
 }  // namespace lus
