@@ -349,7 +349,8 @@ int lus_sand_step(LusGpu* ctx, float dt, int attract_flag, int blow_flag, const 
 /* entries > 0: the neighbour lists get a fixed buffer of that many entries
  * and lus_sand_step no longer waits for the device (the reference's lists
  * grow instead, src/neighbors/Neighbors.cpp:306-361; ~33 entries per
- * particle on the 1 M sand lattice).  A step whose lists are longer in total
+ * particle on the 1 M sand lattice; 4.5 bytes an entry beside the lists' fixed
+ * places, given back by a smaller capacity).  A step whose lists are longer in total
  * projects no contact and leaves an invalid state; the next
  * lus_gpu_sync, lus_sand_download or lus_sand_neighbors reports it
  * (LUS_ESTATE) and clears the mark.  In the same way a simulate_sand_v3

@@ -2084,14 +2084,30 @@ int sand_check(LusGpu* c) {
 }
 
 // Room for `groups` int4 in the pool of long lists, those of the last step
-// kept (no work may be in flight).  It never shrinks while the scene lives.
-int sand_pool(SandState& S, long groups) {
-    if (groups <= S.L.pool_groups) return LUS_OK;
+// kept (no work may be in flight).  fit: no more than that either.
+int sand_pool(SandState& S, long groups, bool fit) {
+    const long have = S.L.pool_groups;
+    if (groups <= have && !fit) return LUS_OK;
+    // what the last step's lists hold: the groups they asked for, as far as there was room
+    unsigned long long asked = 0;
+    if (S.stepped && have > 0) LUS_HIP(hipMemcpy(&asked, S.L.ctl + 1, sizeof(asked), hipMemcpyDeviceToHost));
+    const long keep = (long)std::min(asked, (unsigned long long)have);
+    groups = std::max(groups, keep);
+    if (groups == have) return LUS_OK;
+    if (keep == 0) {  // nothing to keep: the old memory first
+        S.pool_mem.release();
+        S.L.pool = nullptr;
+        S.L.pool_groups = 0;
+    }
     Arena fresh;
     int4* pool = nullptr;
-    LUS_HIP(fresh.alloc(&pool, (size_t)groups));
-    if (S.L.pool_groups > 0)
-        LUS_HIP(hipMemcpy(pool, S.L.pool, sizeof(int4) * (size_t)S.L.pool_groups, hipMemcpyDeviceToDevice));
+    const hipError_t e = fresh.alloc(&pool, (size_t)groups);
+    if (e != hipSuccess && groups < have && keep > 0) {
+        (void)hipGetLastError();
+        return LUS_OK;  // no room beside the larger one, which stays
+    }
+    LUS_HIP(e);
+    if (keep > 0) LUS_HIP(hipMemcpy(pool, S.L.pool, sizeof(int4) * (size_t)keep, hipMemcpyDeviceToDevice));
     LUS_HIP(hipDeviceSynchronize());
     std::swap(S.pool_mem.ptrs, fresh.ptrs);  // the old one goes with `fresh`
     S.L.pool = pool;
@@ -2153,7 +2169,7 @@ int sand_enqueue(LusGpu* c, float dt, const lus::SandK& k) {
         if (need <= (unsigned long long)S.L.pool_groups) break;
         // long lists that had no room: once more from the sort, with room
         LUS_HIP(hipStreamSynchronize(s));
-        if (int r = sand_pool(S, (long)(need + need / 4))) return r;
+        if (int r = sand_pool(S, (long)(need + need / 4), false)) return r;
         LUS_HIP(lus::launch_zero_ints(reinterpret_cast<int*>(S.L.ctl), 4, s));
     }
     LUS_HIP(mark(3));
@@ -2269,7 +2285,7 @@ int lus_sand_set_list_capacity(LusGpu* c, long entries) {
     }
     // Lists of at most `entries` in total always fit: those in the pool have
     // more than 4 groups (32 at least) entries each, rounded up to a group
-    if (int r = sand_pool(S, entries / 4 + entries / 32 + 1)) return r;
+    if (int r = sand_pool(S, entries / 4 + entries / 32 + 1, true)) return r;
     if (!S.fail) LUS_HIP(S.mem.alloc(&S.fail, 1));
     LUS_HIP(hipMemset(S.fail, 0, sizeof(int)));
     S.fixed_cap = entries;
