@@ -409,7 +409,7 @@ class Gpu:
         """staged: the list build tests wave-staged candidates in LDS; else
         per-lane gathers (same results).  2: block-staged lists at any size
         (True: at the sizes where they are faster)."""
-        _check(self._lib.lus_pbf_set_build(self._h, int(staged)), "lus_pbf_set_build")
+        _check(self._lib.lus_pbf_set_build(self._h, 2 if staged == 2 else int(bool(staged))), "lus_pbf_set_build")
 
     def pbf_set_lanes(self, lanes=0):
         """Lanes per particle in fused list walks: 0 automatic, 1 or 4."""
