@@ -1323,8 +1323,9 @@ int lus_pbf_download(LusGpu* c, int order, float* pos, float* vel, int* ids) {
     const int n = P.n;
     hipStream_t s = c->stream;
     // vec3 rows packed (and for order 1 put back in input order by id) on
-    // the device, one block for all arrays
-    if (!P.stage) LUS_HIP(P.mem.alloc(&P.stage, 7 * (size_t)n));
+    // the device, one block for all arrays; ids alone come from where they lie
+    const bool rows = pos || vel;
+    if (rows && !P.stage) LUS_HIP(P.mem.alloc(&P.stage, 7 * (size_t)n));
     lus::PackArgs pk{};
     lus::HostPiece pc[3];
     int np = 0;
@@ -1341,12 +1342,13 @@ int lus_pbf_download(LusGpu* c, int order, float* pos, float* vel, int* ids) {
         at += 3 * (size_t)n;
     }
     if (ids && order == 0) {
-        pk.i[0] = {P.id, reinterpret_cast<int*>(at), n};
+        if (rows) pk.i[0] = {P.id, reinterpret_cast<int*>(at), n};
         pc[np++] = {ids, nullptr, sizeof(int) * (size_t)n};
     }
-    if (np) LUS_HIP(lus::launch_pack(pk, n, s));
+    if (rows) LUS_HIP(lus::launch_pack(pk, n, s));
     const bool iota = ids && order == 1;
-    LUS_HIP(lus::pull_to_host(c, P.stage, pc, np, iota ? ids : nullptr, iota ? n : 0));
+    const void* block = rows ? static_cast<const void*>(P.stage) : P.id;
+    LUS_HIP(lus::pull_to_host(c, block, pc, np, iota ? ids : nullptr, iota ? n : 0));
     if (!np) LUS_HIP(hipStreamSynchronize(s));
     return LUS_OK;
 }
@@ -2337,7 +2339,8 @@ int lus_sand_download(LusGpu* c, float* pos, float* pos_star, float* vel, int* a
     // the arrays are packed on the device into one block; positions_star
     // equals positions after a step (src/Simulate.cpp:316-319) and before the
     // first one (both are the uploaded positions)
-    if (!S.stage) LUS_HIP(S.mem.alloc(&S.stage, 8 * (size_t)n));
+    const bool rows = pos || pos_star || vel;
+    if (rows && !S.stage) LUS_HIP(S.mem.alloc(&S.stage, 8 * (size_t)n));
     lus::PackArgs pk{};
     lus::HostPiece pc[4];
     int np = 0;
@@ -2353,18 +2356,22 @@ int lus_sand_download(LusGpu* c, float* pos, float* pos_star, float* vel, int* a
         at += 3 * (size_t)n;
     }
     int* q = reinterpret_cast<int*>(at);
-    if (attracted) {
+    if (attracted && rows) {
         pk.i[0] = {S.att, q, n};
         pc[np++] = {attracted, nullptr, sizeof(int) * (size_t)n};
         q += n;
     }
-    if (perm) {
+    if (perm && rows) {
         pk.i[1] = {S.perm, q, n};
         pc[np++] = {perm, nullptr, sizeof(int) * (size_t)n};
     }
-    if (np && n > 0) {
+    if (rows && n > 0) {
         LUS_HIP(lus::launch_pack(pk, n, s));
         LUS_HIP(lus::pull_to_host(c, S.stage, pc, np));
+    } else if (n > 0 && (attracted || perm)) {  // alone they come from where they lie
+        const lus::HostPiece a{attracted, nullptr, sizeof(int) * (size_t)n}, b{perm, nullptr, sizeof(int) * (size_t)n};
+        if (attracted) LUS_HIP(lus::pull_to_host(c, S.att, &a, 1));
+        if (perm) LUS_HIP(lus::pull_to_host(c, S.perm, &b, 1));
     } else {
         LUS_HIP(hipStreamSynchronize(s));
     }

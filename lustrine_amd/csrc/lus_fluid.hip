@@ -905,9 +905,11 @@ int lus_fluid_download(LusGpu* c, float* positions, float* positions_star, float
     hipStream_t s = lus::ctx_stream(c);
     FL_HIP(hipSetDevice(lus::ctx_device(c)));
     // the arrays are packed on the device into one block: positions,
-    // positions_star, the moving slots' velocities, lambdas
+    // positions_star, the moving slots' velocities, lambdas (alone they come
+    // from where they lie)
     const int total = F->total, moving = F->s1 - F->s0, nl = F->k.nl;
-    if (!F->stage) FL_HIP(fl_alloc(F, &F->stage, 6 * (size_t)total + 3 * (size_t)moving + (size_t)nl));
+    const bool rows = positions || positions_star || velocities;
+    if (rows && !F->stage) FL_HIP(fl_alloc(F, &F->stage, 6 * (size_t)total + 3 * (size_t)moving + (size_t)nl));
     lus::PackArgs pk{};
     lus::HostPiece pc[4];
     int np = 0;
@@ -928,12 +930,12 @@ int lus_fluid_download(LusGpu* c, float* positions, float* positions_star, float
         at += 3 * (size_t)moving;
     }
     if (lambdas && nl) {
-        pk.i[0] = {reinterpret_cast<const int*>(F->lam), reinterpret_cast<int*>(at), nl};
+        if (rows) pk.i[0] = {reinterpret_cast<const int*>(F->lam), reinterpret_cast<int*>(at), nl};
         pc[np++] = {lambdas, nullptr, sizeof(float) * (size_t)nl};
     }
     if (np) {
-        FL_HIP(lus::launch_pack(pk, std::max(total, nl), s));
-        FL_HIP(lus::pull_to_host(c, F->stage, pc, np));
+        if (rows) FL_HIP(lus::launch_pack(pk, std::max(total, nl), s));
+        FL_HIP(lus::pull_to_host(c, rows ? F->stage : F->lam, pc, np));
     } else {
         FL_HIP(hipStreamSynchronize(s));
     }
