@@ -1348,8 +1348,8 @@ __device__ __forceinline__ float lambda_build_ws(const float4* __restrict__ xp, 
     return Ci;
 }
 
-// the plain scene's first lambda pass (kMixed is false)
-template <bool kFast, bool kMixed>
+// the plain scene's first lambda pass
+template <bool kFast>
 __global__ __launch_bounds__(kBlock) void k_pbf_lambda_build_ws(const float4* __restrict__ xp,
                                                                  const int* __restrict__ key2,
                                                                  const int* __restrict__ cs, int n, PbfK k,
@@ -1358,8 +1358,8 @@ __global__ __launch_bounds__(kBlock) void k_pbf_lambda_build_ws(const float4* __
                                                                  unsigned long long* __restrict__ nb,
                                                                  const int* __restrict__ gate) {
     if (gate && *gate == 0) return;  // uniform: before any barrier
-    __shared__ float stage[kBlock / 64][kStageFloats<kMixed>];
-    const float Ci = lambda_build_ws<kFast, kMixed>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
+    __shared__ float stage[kBlock / 64][kStageFloats<false>];
+    const float Ci = lambda_build_ws<kFast, false>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
     block_max_store(Ci, maxc);
 }
 
@@ -1382,8 +1382,7 @@ __global__ __launch_bounds__(kBlock) void k_pbf_list_build_ws(const float4* __re
 template <bool kFast>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_mix_lambda_build_ws(
     const float4* __restrict__ xp, const int* __restrict__ key2, const int* __restrict__ cs, int n, PbfK k,
-    float4* __restrict__ xl, int* __restrict__ maxc, unsigned long long* __restrict__ nb,
-    const int* __restrict__ gate) {
+    float4* __restrict__ xl, unsigned long long* __restrict__ nb) {
     __shared__ float stage[kBlock / 64][kStageFloats<true>];
     lambda_build_ws<kFast, true>(xp, key2, cs, n, k, xl, nb, (lds_float*)stage[threadIdx.x >> 6]);
 }
@@ -1624,10 +1623,10 @@ hipError_t launch_pbf_lambda(const float4* xa, int* key2, const int* cs, int n, 
     }
     if (build && ta.stage && xa == xp && n > 0 && k.nph == 1) {
         if (k.exact)
-            launch_kernel((k_pbf_lambda_build_ws<false, false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, masks,
+            launch_kernel((k_pbf_lambda_build_ws<false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, masks,
                           gate);
         else
-            launch_kernel((k_pbf_lambda_build_ws<true, false>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, masks,
+            launch_kernel((k_pbf_lambda_build_ws<true>), g, b, 0, s, xp, key2, cs, n, k, xl, maxc, masks,
                           gate);
         return hipGetLastError();
     }
@@ -2723,11 +2722,9 @@ hipError_t launch_mix_lambda(const float4* xa, int* key2, const int* cs, int n, 
     const dim3 g(grid_for(n)), b(kBlock);
     if (build && stage && xa == xp && n > 0 && k.ph_out) {
         if (k.exact)
-            launch_kernel((k_mix_lambda_build_ws<false>), g, b, 0, s, xp, key2, cs, n, k, xl, (int*)nullptr,
-                          masks, (const int*)nullptr);
+            launch_kernel((k_mix_lambda_build_ws<false>), g, b, 0, s, xp, key2, cs, n, k, xl, masks);
         else
-            launch_kernel((k_mix_lambda_build_ws<true>), g, b, 0, s, xp, key2, cs, n, k, xl, (int*)nullptr,
-                          masks, (const int*)nullptr);
+            launch_kernel((k_mix_lambda_build_ws<true>), g, b, 0, s, xp, key2, cs, n, k, xl, masks);
         return hipGetLastError();
     }
     if (build && k.exact)
